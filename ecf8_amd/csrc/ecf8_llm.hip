@@ -99,6 +99,23 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
+// The largest value of the wave, in every lane, through DPP row shifts and
+// broadcasts (VALU latency; each __shfl_xor step is an LDS round trip).
+// A lane without a source keeps its own value.
+__device__ __forceinline__ float wave_max_dpp(float v) {
+#define ECF8_DPP_MAX(ctrl)                                                                  \
+  v = fmaxf(v, __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(                       \
+                   (int)__float_as_uint(v), (int)__float_as_uint(v), ctrl, 0xF, 0xF, false)))
+  ECF8_DPP_MAX(0x111);  // row_shr:1
+  ECF8_DPP_MAX(0x112);  // row_shr:2
+  ECF8_DPP_MAX(0x114);  // row_shr:4
+  ECF8_DPP_MAX(0x118);  // row_shr:8
+  ECF8_DPP_MAX(0x142);  // row_bcast:15
+  ECF8_DPP_MAX(0x143);  // row_bcast:31
+#undef ECF8_DPP_MAX
+  return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), 63));
+}
+
 // Quantize 16 consecutive values held by one thread; the 8 threads of a
 // 128-column group are 8 consecutive lanes.  Writes 16 e4m3fn bytes and,
 // from the group's first thread, the group scale.
@@ -1143,7 +1160,9 @@ __global__ __launch_bounds__(256) void moe_logits_kernel(const uint16_t *__restr
 
 // Top-k of one token per wave (4 tokens per 256-thread workgroup): softmax
 // over the E <= 256 logits in fp32, the top_k largest probabilities (ties
-// to the lower expert index), renormalized to sum 1.
+// to the lower expert index), renormalized to sum 1.  One wave's latency
+// bounds it: each pick is a DPP maximum and four ballots (16 tokens of 128
+// experts, top 8: 6.9 -> 4.5 us against two shuffles per butterfly step).
 __global__ __launch_bounds__(256) void moe_topk_kernel(const float *__restrict__ logits, int M,
                                                        int E, int top_k,
                                                        int *__restrict__ topk_idx,
@@ -1173,23 +1192,16 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(const float *__restrict__
   float my_w = 0.f, sel_sum = 0.f;
   int my_i = 0;
   for (int k = 0; k < top_k; ++k) {
-    float bv = -2.f;
+    // the largest probability, then the lowest expert that has it (expert
+    // lane + 64 i: the lowest i first, then the lowest lane)
+    // (-2 if none is a number)
+    const float bv = wave_max_dpp(fmaxf(fmaxf(fmaxf(fmaxf(-2.f, p[0]), p[1]), p[2]), p[3]));
     int bi = 0x7fffffff;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (p[i] > bv) {
-        bv = p[i];
-        bi = lane + 64 * i;
-      }
-    for (int o = 32; o > 0; o >>= 1) {
-      const float ov = __shfl_xor(bv, o);
-      const int oi = __shfl_xor(bi, o);
-      if (ov > bv || (ov == bv && oi < bi)) {
-        bv = ov;
-        bi = oi;
-      }
+    for (int i = 3; i >= 0; --i) {
+      const uint64_t at = __ballot(p[i] == bv);
+      if (at) bi = 64 * i + __builtin_ctzll(at);  // uniform
     }
-    // every lane now holds the same (bv, bi)
 #pragma unroll
     for (int i = 0; i < 4; ++i)
       if (lane + 64 * i == bi) p[i] = -1.f;
@@ -1211,31 +1223,75 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(const float *__restrict__
 // give each sorted position's token and routing weight, pair_pos each
 // pair's sorted position; active[0, n_active) lists the experts with pairs
 // in increasing order; select[e] (optional) = 1 if expert e has pairs.
-// Expert ids outside [0, E) are clamped into it.  Two passes over chunks of
-// 1024 pairs: integer counts per expert, then each pair's rank = pairs of
-// its expert in earlier chunks + earlier pairs of its chunk.
+// Expert ids outside [0, E) are clamped into it.
+//
+// A stable counting sort.  Wave w owns a contiguous run of 64 x chunks
+// pairs (chunks = ceil(P / 1024) <= 8); a lane's rank among the pairs of
+// its expert in its 64-pair chunk is a popcount of the wave's match mask
+// (eight ballots, one per bit of the expert), and the wave's own row of
+// counts in LDS carries the rank over its chunks.  Latency of one
+// workgroup bounds it: three barriers and 8 ballots per 64 pairs instead of
+// a serial walk over 1024 pairs per chunk and pass (MI355X: 4096 pairs
+// 168.9 -> 10.1 us, 128 pairs 8.2 -> 4.4 us).
 __global__ __launch_bounds__(1024) void moe_group_kernel(
     const int *__restrict__ topk_idx, const float *__restrict__ topk_w, int P, int top_k, int E,
     int *__restrict__ offsets, int *__restrict__ active, int *__restrict__ n_active,
     int *__restrict__ pair_tok, float *__restrict__ pair_w, int *__restrict__ pair_pos,
     int *__restrict__ select) {
-  constexpr int kChunk = 1024;
-  __shared__ int s_e[kChunk];
-  __shared__ int s_cnt[256];
-  __shared__ int s_off[257];
-  const int t = threadIdx.x;
-  auto expert_of = [&](int p) { return p < P ? min(max(topk_idx[p], 0), E - 1) : -1; };
-  if (t < 256) s_cnt[t] = 0;
-  for (int c0 = 0; c0 < P; c0 += kChunk) {
-    const int n = min(kChunk, P - c0);
-    __syncthreads();  // s_e of the previous chunk is no longer read
-    s_e[t] = expert_of(c0 + t);
-    __syncthreads();
-    if (t < E) {
-      int c = 0;
-      for (int q = 0; q < n; ++q) c += s_e[q] == t;
-      s_cnt[t] += c;
+  constexpr int kWaves = 16, kMaxChunks = 8;
+  __shared__ int s_cnt[kWaves][256];  // pairs per expert of each wave's run
+  __shared__ int s_tot[256];
+  __shared__ int s_off[256];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int chunks = (P + 1023) >> 10;
+  const int base = wave * 64 * chunks;
+  int ex[kMaxChunks], rank[kMaxChunks];
+  float w[kMaxChunks];
+#pragma unroll
+  for (int c = 0; c < kMaxChunks; ++c) {
+    const int p = base + 64 * c + lane;
+    const bool in = c < chunks && p < P;
+    ex[c] = in ? min(max(topk_idx[p], 0), E - 1) : -1;
+    w[c] = in ? topk_w[p] : 0.f;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) s_cnt[wave][lane + 64 * i] = 0;
+  // The wave's own row: LDS serves one wave in program order, so its later
+  // reads follow these writes (wave barriers keep the compiler to it).
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int c = 0; c < kMaxChunks; ++c) {
+    rank[c] = 0;
+    if (c < chunks) {  // uniform
+      const bool in = ex[c] >= 0;
+      uint64_t peers = __ballot(in);
+#pragma unroll
+      for (int bit = 0; bit < 8; ++bit) {
+        const bool one = (ex[c] >> bit) & 1;
+        const uint64_t ones = __ballot(one);
+        peers &= one ? ones : ~ones;
+      }
+      const int before = __popcll(peers & ((1ull << lane) - 1));
+      if (in) {
+        rank[c] = s_cnt[wave][ex[c]] + before;
+        __builtin_amdgcn_wave_barrier();
+        // the last pair of each expert writes the new count (all its peers
+        // have read the old one: one wave, in program order)
+        if ((peers >> lane) == 1) s_cnt[wave][ex[c]] = rank[c] + 1;
+      }
+      __builtin_amdgcn_wave_barrier();
     }
+  }
+  __syncthreads();
+  if (t < 256) {  // counts of each wave -> pairs of that expert in earlier waves
+    int run = 0;
+#pragma unroll
+    for (int v = 0; v < kWaves; ++v) {
+      const int n = s_cnt[v][t];
+      s_cnt[v][t] = run;
+      run += n;
+    }
+    s_tot[t] = run;
   }
   __syncthreads();
   if (t < 64) {
@@ -1244,8 +1300,7 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(
     int c[4], f[4], sc = 0, sf = 0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int e = 4 * t + i;
-      c[i] = e < E ? s_cnt[e] : 0;
+      c[i] = s_tot[4 * t + i];  // zero from expert E on
       f[i] = c[i] > 0;
       sc += c[i];
       sf += f[i];
@@ -1262,42 +1317,29 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int e = 4 * t + i;
+      s_off[e] = off;
       if (e < E) {
-        s_off[e] = off;
+        offsets[e] = off;
         if (f[i]) active[na] = e;
+        if (select) select[e] = f[i];
       }
       off += c[i];
       na += f[i];
     }
     if (t == 63) {
-      s_off[E] = ic;
+      offsets[E] = ic;
       *n_active = jf;
     }
   }
   __syncthreads();
-  for (int i = t; i <= E; i += kChunk) offsets[i] = s_off[i];
-  if (select && t < E) select[t] = s_cnt[t] > 0 ? 1 : 0;
-  __syncthreads();
-  if (t < 256) s_cnt[t] = 0;  // now: pairs of each expert in earlier chunks
-  for (int c0 = 0; c0 < P; c0 += kChunk) {
-    const int n = min(kChunk, P - c0);
-    __syncthreads();
-    const int e = expert_of(c0 + t);
-    s_e[t] = e;
-    __syncthreads();
-    if (t < n) {
-      int rank = s_cnt[e];
-      for (int q = 0; q < t; ++q) rank += s_e[q] == e;
-      const int q = s_off[e] + rank;
-      pair_tok[q] = (c0 + t) / top_k;
-      pair_w[q] = topk_w[c0 + t];
-      pair_pos[c0 + t] = q;
-    }
-    __syncthreads();  // every rank read s_cnt before it grows
-    if (t < E) {
-      int c = 0;
-      for (int q = 0; q < n; ++q) c += s_e[q] == t;
-      s_cnt[t] += c;
+#pragma unroll
+  for (int c = 0; c < kMaxChunks; ++c) {
+    if (ex[c] >= 0) {
+      const int p = base + 64 * c + lane;
+      const int q = s_off[ex[c]] + s_cnt[wave][ex[c]] + rank[c];
+      pair_tok[q] = p / top_k;
+      pair_w[q] = w[c];
+      pair_pos[p] = q;
     }
   }
 }

@@ -89,6 +89,48 @@ def test_group_sorts_pairs_by_expert(cuda_device, M, top_k, E):
     assert np.array_equal(r.select.cpu().numpy(), sel)
 
 
+@pytest.mark.parametrize("M,top_k,E,skew", [(1, 1, 1, False), (63, 1, 3, False), (65, 1, 256, False),
+                                             (128, 8, 256, True), (129, 8, 128, False),
+                                             (1024, 8, 256, True), (1023, 8, 255, False)])
+def test_group_run_and_chunk_edges(cuda_device, M, top_k, E, skew):
+    """Pair counts at the edges of a wave's 64-pair chunks and 1024-pair
+    rounds, up to 8192; every pair on one expert; ids outside [0, E) clamped."""
+    from ecf8_amd.llm_kernels import MoeRouting, moe_group
+
+    rng = np.random.default_rng(M + E)
+    idx = rng.integers(-2, E + 2, (M, top_k)).astype(np.int32)
+    if skew:
+        idx[:, 1:] = E - 1
+    w = rng.random((M, top_k)).astype(np.float32)
+    r = MoeRouting(M, top_k, E, cuda_device)
+    r.topk_idx.copy_(torch.from_numpy(idx))
+    r.topk_w.copy_(torch.from_numpy(w))
+    moe_group(r, M)
+    offsets, active, pos = _groups_ref(np.clip(idx, 0, E - 1), E)
+    assert int(r.n_active.item()) == len(active)
+    assert np.array_equal(r.offsets.cpu().numpy(), offsets)
+    assert np.array_equal(r.active.cpu().numpy()[:len(active)], active)
+    assert np.array_equal(r.pair_pos.cpu().numpy(), pos)
+    assert np.array_equal(r.pair_tok.cpu().numpy()[pos], np.repeat(np.arange(M), top_k))
+    assert np.array_equal(r.pair_w.cpu().numpy()[pos], w.reshape(-1))
+
+
+@pytest.mark.parametrize("E,top_k", [(1, 1), (64, 16), (65, 3), (200, 8), (256, 16)])
+def test_router_ties_go_to_the_lower_expert(cuda_device, E, top_k):
+    """Router rows drawn from three vectors, so most logits tie exactly."""
+    from ecf8_amd.llm_kernels import MoeRouting, moe_route
+
+    gen = torch.Generator().manual_seed(E)
+    x = torch.randn(5, 512, generator=gen).to(torch.bfloat16)
+    rows = (torch.randn(3, 512, generator=gen) * 0.05).to(torch.bfloat16)
+    kind = torch.randint(0, 3, (E,), generator=gen)
+    r = MoeRouting(5, top_k, E, cuda_device)
+    moe_route(x.to(cuda_device), rows[kind].contiguous().to(cuda_device), 5, r)
+    logits = r.logits.cpu()
+    want = torch.sort(logits, dim=-1, descending=True, stable=True).indices[:, :top_k]
+    assert torch.equal(r.topk_idx.cpu().long(), want)
+
+
 def _pair_linear_ref(a_rows, a_s_rows, w, ws):
     """fp64 block-scaled product of the given activation rows with one
     expert's weight (the math of the dense FP8 linear)."""
