@@ -82,6 +82,8 @@ _SIGNATURES = {
     "ecf8_moe_group": ([_vp, _vp, _i64, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp], _i32),
     "ecf8_moe_linear": ([_vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _i32, _i64, _i64, _i32, _vp,
                          _i64, _vp], _i32),
+    "ecf8_moe_linear_pairs": ([_vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _i32, _i64, _i64,
+                               _i32, _i64, _vp, _i64, _vp], _i32),
     "ecf8_moe_combine": ([_vp, _i64, _vp, _vp, _i64, _i32, _i64, _vp, _vp], _i32),
 }
 

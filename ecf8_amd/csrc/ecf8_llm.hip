@@ -1456,6 +1456,152 @@ __global__ __launch_bounds__(WAVES * 64) void moe_linear16_kernel(MoeLinear a) {
   }
 }
 
+// Workgroup barrier that waits for LDS only (a __syncthreads would also
+// wait for the prefetched global loads).
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_s_waitcnt((0x3F & 15) | (0x3 << 14) | (0x7 << 4) | (0x0 << 8));  // lgkmcnt(0)
+  gemm_barrier();
+}
+
+// The same grouped linear for many rows per expert (a prompt): workgroup
+// (strip, slot) of eight waves computes a 128-column strip of expert
+// active[slot], wave w its columns [16 w, +16), for 16 kChunks rows at a
+// time, so an expert's weights are read once per 64 (or 32) rows instead of
+// once per 16.  The rows' activations go to LDS in MFMA lane order (gathered 16-byte parts),
+// shared by the eight waves and double-buffered; a wave's weight panel goes
+// straight to its registers, one stage of PARTS groups ahead.
+//
+// The sums are moe_linear16_kernel's, bit for bit: group kg adds to partial
+// sum kg mod PARTS (that kernel's wave), the partial sums are added in
+// order.  HBM bounds it (weights read once, 403 MB for gate/up and 201 MB for
+// down of 128 experts); MI355X, 512 tokens, tile-layout weights: gate/up 347
+// -> 113 us, down 107 -> 70 us.
+template <int PARTS, int kChunks>
+__global__ __launch_bounds__(512, 8 / kChunks) void moe_rows_kernel(MoeLinear a) {
+  constexpr int kRows = 16 * kChunks, kMaxGroups = 16;
+  constexpr int kCopies = 2 * kChunks < 8 ? 8 / (2 * kChunks) : 1;  // waves per 1 KB part
+  __shared__ u32x4 s_a[2][PARTS][kChunks][2][64];
+  __shared__ __attribute__((aligned(16))) float s_s[kMaxGroups][kRows];
+  const int slot = blockIdx.y;
+  if (slot >= a.n_active[0]) return;  // uniform
+  const int e = a.active[slot];
+  const int r0 = a.offsets[e], rows = a.offsets[e + 1] - r0;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, g = lane >> 4;
+  const int seg = (int)(blockIdx.x * 128) / a.seg_n;  // seg_n is a multiple of 128
+  const int n0 = (int)(blockIdx.x * 128) - seg * a.seg_n + 16 * wave;
+  const uint8_t *w = reinterpret_cast<const uint8_t *>(a.w[(size_t)e * a.n_segs + seg]);
+  const int K = a.K, kgroups = K / kGroup;
+  const float *wsrow =
+      reinterpret_cast<const float *>(a.ws[(size_t)e * a.n_segs + seg]) +
+      (size_t)(n0 / kGroup) * kgroups;
+  const WeightLane wl(w, a.wtiled != 0, n0, r, g, K);
+  const Rsrc wr = wl.rsrc(K);
+  const int stages = (kgroups + PARTS - 1) / PARTS;
+
+  for (int rc = 0; rc < rows; rc += kRows) {
+    const int mrows = min(kRows, rows - rc);
+    const int nch = (mrows + 15) >> 4;  // 16-row chunks in use (uniform)
+    // scales, [group][row]; rows past the last take its values, unused
+    for (int i = threadIdx.x; i < kRows * kgroups; i += 512) {
+      const int row = i / kgroups, kg = i - row * kgroups;
+      const int q = r0 + rc + min(row, mrows - 1);
+      s_s[kg][row] = a.as[(size_t)(a.row_of ? a.row_of[q] : q) * kgroups + kg];
+    }
+    // wave v stages half (v / kCopies) & 1 of chunk v / kCopies / 2: groups
+    // v % kCopies, + kCopies, ... of each stage
+    const int lc = wave / kCopies >> 1, lh = wave / kCopies & 1, lu = wave % kCopies;
+    const int lq = r0 + rc + min(16 * lc + r, mrows - 1);
+    const uint8_t *arow =
+        tile_lane_base(a.aq, a.row_of ? a.row_of[lq] : lq, kgroups, g) + 1024 * lh;
+    constexpr int kA = (PARTS + kCopies - 1) / kCopies;
+    u32x4 av[kA];
+    uint4 wv[PARTS][2];
+    float wsv[PARTS];
+    // groups past the last load it again, unused
+    auto load = [&](int s, u32x4 (&av)[kA], uint4 (&wv)[PARTS][2], float (&wsv)[PARTS]) {
+#pragma unroll
+      for (int u = 0; u < kA; ++u)
+        av[u] = *reinterpret_cast<const u32x4 *>(
+            arow + (size_t)min(s * PARTS + lu + kCopies * u, kgroups - 1) * 2048);
+#pragma unroll
+      for (int u = 0; u < PARTS; ++u) {
+        const int kg = min(s * PARTS + u, kgroups - 1);
+        wl.load(wr, kg, wv[u][0], wv[u][1]);
+        wsv[u] = wsrow[kg];
+      }
+    };
+    float acc[PARTS][kChunks][4];
+#pragma unroll
+    for (int u = 0; u < PARTS; ++u)
+#pragma unroll
+      for (int c = 0; c < kChunks; ++c)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[u][c][i] = 0.f;
+    load(0, av, wv, wsv);
+    for (int s = 0; s < stages; ++s) {
+      const int buf = s & 1;
+      uint4 wc[PARTS][2];
+      float wsc[PARTS];
+#pragma unroll
+      for (int u = 0; u < kA; ++u)
+        if (lu + kCopies * u < PARTS) s_a[buf][lu + kCopies * u][lc][lh][lane] = av[u];
+#pragma unroll
+      for (int u = 0; u < PARTS; ++u) {
+        wc[u][0] = wv[u][0];
+        wc[u][1] = wv[u][1];
+        wsc[u] = wsv[u];
+      }
+      // this stage is in LDS; the other buffer was last read in stage s - 1,
+      // before every wave's arrival here
+      lds_barrier();
+      if (s + 1 < stages) load(s + 1, av, wv, wsv);
+#pragma unroll
+      for (int u = 0; u < PARTS; ++u) {
+        const int kg = s * PARTS + u;
+        if (kg >= kgroups) break;  // uniform
+#pragma unroll
+        for (int c = 0; c < kChunks; ++c) {
+          if (c < nch) {  // uniform
+            const u32x4 lo = s_a[buf][u][c][0][lane], hi = s_a[buf][u][c][1][lane];
+            const float4 sc = *reinterpret_cast<const float4 *>(&s_s[kg][16 * c + 4 * g]);
+            v4f d = {0.f, 0.f, 0.f, 0.f};
+            d = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(
+                (long)(((uint64_t)lo.y << 32) | lo.x),
+                (long)(((uint64_t)wc[u][0].y << 32) | wc[u][0].x), d, 0, 0, 0);
+            d = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(
+                (long)(((uint64_t)lo.w << 32) | lo.z),
+                (long)(((uint64_t)wc[u][0].w << 32) | wc[u][0].z), d, 0, 0, 0);
+            d = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(
+                (long)(((uint64_t)hi.y << 32) | hi.x),
+                (long)(((uint64_t)wc[u][1].y << 32) | wc[u][1].x), d, 0, 0, 0);
+            d = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(
+                (long)(((uint64_t)hi.w << 32) | hi.z),
+                (long)(((uint64_t)wc[u][1].w << 32) | wc[u][1].z), d, 0, 0, 0);
+            acc[u][c][0] = fmaf(d[0], sc.x * wsc[u], acc[u][c][0]);
+            acc[u][c][1] = fmaf(d[1], sc.y * wsc[u], acc[u][c][1]);
+            acc[u][c][2] = fmaf(d[2], sc.z * wsc[u], acc[u][c][2]);
+            acc[u][c][3] = fmaf(d[3], sc.w * wsc[u], acc[u][c][3]);
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < kChunks; ++c)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int m = 16 * c + 4 * g + i;
+        float sum = 0.f;
+#pragma unroll
+        for (int u = 0; u < PARTS; ++u) sum += acc[u][c][i];
+        if (m < mrows)
+          a.out[(size_t)(r0 + rc + m) * a.ldo + seg * a.seg_n + n0 + r] = (uint16_t)f32_bf16(sum);
+      }
+    lds_barrier();  // s_s and s_a are refilled for the next rows
+  }
+}
+
 // y[m, :] = sum_k pair_w[q] * down[q, :] over q = pair_pos[m * top_k + k],
 // k = 0 .. top_k - 1 in order, accumulated in fp32; bf16 out [M, H].  One
 // workgroup per token, 8 columns per thread.
@@ -1735,12 +1881,12 @@ extern "C" int ecf8_moe_group(const int *topk_idx, const float *topk_w, int64_t 
   return launched();
 }
 
-extern "C" int ecf8_moe_linear(const void *aq, const float *as, const int *row_of,
-                               const int *offsets, const int *active, const int *n_active,
-                               int n_experts, const void *const *weights,
-                               const float *const *weight_scales, int n_segs, int64_t seg_n,
-                               int64_t K, int weight_layout, void *out, int64_t ldo,
-                               void *stream) {
+extern "C" int ecf8_moe_linear_pairs(const void *aq, const float *as, const int *row_of,
+                                     const int *offsets, const int *active, const int *n_active,
+                                     int n_experts, const void *const *weights,
+                                     const float *const *weight_scales, int n_segs,
+                                     int64_t seg_n, int64_t K, int weight_layout, int64_t pairs,
+                                     void *out, int64_t ldo, void *stream) {
   if (!aq || !as || !offsets || !active || !n_active || !weights || !weight_scales || !out ||
       n_experts <= 0 || n_segs < 1 || n_segs > ECF8_LINEAR_MAX_SEGS || seg_n <= 0 || K <= 0 ||
       (weight_layout != ECF8_WEIGHT_ROWS && weight_layout != ECF8_WEIGHT_TILES))
@@ -1756,23 +1902,52 @@ extern "C" int ecf8_moe_linear(const void *aq, const float *as, const int *row_o
               reinterpret_cast<const uint64_t *>(weights),
               reinterpret_cast<const uint64_t *>(weight_scales), static_cast<uint16_t *>(out),
               n_segs, (int)seg_n, (int)K, (int)ldo, weight_layout == ECF8_WEIGHT_TILES};
+  const int64_t groups = K / kGroup;
+  // Four rows per expert and more: the form that reads an expert's weights
+  // once per 64 (32) rows, while its three or four partial sums fit the
+  // registers.  MI355X, 128 experts, row-major weights, us for gate/up K =
+  // 2048 and down K = 768, 16-row form against this one: 32 tokens (2 rows)
+  // 88.2 / 40.8 against 99.4 / 42.9, 48 tokens 103.9 / 46.2 against 102.3 /
+  // 45.7, 64 tokens 112.9 / 48.2 against 103.3 / 46.8, 128 tokens 145.7 /
+  // 53.7 against 105.7 / 48.6, 1024 tokens 798 / 255 against 253 / 151.
+  // 32 rows for down keep two workgroups per CU, its loads' latency being
+  // most of its two stages (64 rows: 86.0 against 92.4 us at 512 tokens, but
+  // 67.5 against 48.6 at 128); the four-part form spills at 128 VGPRs.
+  if (pairs >= 4 * (int64_t)n_experts && groups <= ECF8_MOE_FOUR_WAVE_GROUPS) {
+    const dim3 strips((unsigned)(n_segs * seg_n / 128), (unsigned)n_experts);
+    if (groups == 6)
+      moe_rows_kernel<3, 2><<<strips, 512, 0, as_stream(stream)>>>(a);
+    else
+      moe_rows_kernel<4, 4><<<strips, 512, 0, as_stream(stream)>>>(a);
+    return launched();
+  }
   const dim3 grid((unsigned)(n_segs * seg_n / 16), (unsigned)n_experts);
   // each wave's share of the K groups in one batch of loads where it fits.
   // On MI355X, Qwen3-30B-A3B experts at 16 tokens (48 layers back to back):
   // gate/up (K = 2048) 48.5 us per layer at four waves of four groups
   // against 53.4 at eight of two; down (K = 768) 23.7 us at three waves of
   // two groups against 26.9 at four (two, two, one, one)
-  const int64_t kg = K / kGroup;
   static_assert(ECF8_MOE_FOUR_WAVE_GROUPS == 16, "four waves of at most four groups");
-  if (kg == 6)
+  if (groups == 6)
     moe_linear16_kernel<3, 2><<<grid, 192, 0, as_stream(stream)>>>(a);
-  else if (kg <= 8)
+  else if (groups <= 8)
     moe_linear16_kernel<4, 2><<<grid, 256, 0, as_stream(stream)>>>(a);
-  else if (kg <= ECF8_MOE_FOUR_WAVE_GROUPS)
+  else if (groups <= ECF8_MOE_FOUR_WAVE_GROUPS)
     moe_linear16_kernel<4, 4><<<grid, 256, 0, as_stream(stream)>>>(a);
   else
     moe_linear16_kernel<8, 4><<<grid, 512, 0, as_stream(stream)>>>(a);
   return launched();
+}
+
+extern "C" int ecf8_moe_linear(const void *aq, const float *as, const int *row_of,
+                               const int *offsets, const int *active, const int *n_active,
+                               int n_experts, const void *const *weights,
+                               const float *const *weight_scales, int n_segs, int64_t seg_n,
+                               int64_t K, int weight_layout, void *out, int64_t ldo,
+                               void *stream) {
+  return ecf8_moe_linear_pairs(aq, as, row_of, offsets, active, n_active, n_experts, weights,
+                               weight_scales, n_segs, seg_n, K, weight_layout, 0, out, ldo,
+                               stream);
 }
 
 extern "C" int ecf8_moe_combine(const void *down, int64_t ldd, const int *pair_pos,

@@ -407,13 +407,12 @@ class MoeLinearPlan:
                 or tuple(a_scale.shape[1:]) != (self.K // GROUP,) or a_scale.shape[0] < rows
                 or self.out.shape[0] < P or r.E != self.E):
             raise ECF8Error("activation / output shape does not match the grouped linear")
-        check(lib().ecf8_moe_linear(aq.data_ptr(), a_scale.data_ptr(),
-                                    r.pair_tok.data_ptr() if gather else None,
-                                    r.offsets.data_ptr(), r.active.data_ptr(), r.n_active.data_ptr(),
-                                    self.E, self.w_table.data_ptr(), self.s_table.data_ptr(),
-                                    self.n_segs, self.seg_n, self.K, self.weight_layout,
-                                    self.out.data_ptr(), self.out.shape[-1], _stream(aq)),
-              "ecf8_moe_linear")
+        check(lib().ecf8_moe_linear_pairs(
+            aq.data_ptr(), a_scale.data_ptr(), r.pair_tok.data_ptr() if gather else None,
+            r.offsets.data_ptr(), r.active.data_ptr(), r.n_active.data_ptr(), self.E,
+            self.w_table.data_ptr(), self.s_table.data_ptr(), self.n_segs, self.seg_n, self.K,
+            self.weight_layout, M * r.top_k, self.out.data_ptr(), self.out.shape[-1],
+            _stream(aq)), "ecf8_moe_linear")
         return self.out
 
 

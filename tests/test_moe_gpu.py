@@ -143,6 +143,49 @@ def _pair_linear_ref(a_rows, a_s_rows, w, ws):
     return (part * scale).sum(-1)
 
 
+@pytest.mark.parametrize("K,n_segs,seg_n", [(768, 1, 256), (768, 2, 128), (2048, 2, 128),
+                                             (640, 1, 128), (128, 3, 128), (1024, 1, 384)])
+@pytest.mark.parametrize("layout", [0, 1])
+def test_grouped_linear_many_rows_is_bit_identical(cuda_device, K, n_segs, seg_n, layout):
+    """The form for many rows per expert against the 16-row form (no pair
+    count given): experts of 0, 1, 16, 17, 31, 32, 33, 63, 64, 65 and 130
+    rows, gathered and not, partial last stages of groups."""
+    from ecf8_amd._lib import lib
+    from ecf8_amd.llm_kernels import MoeLinearPlan, MoeRouting, moe_group, to_tiles
+
+    counts = [0, 1, 16, 17, 31, 32, 33, 63, 64, 65, 130]
+    E, M = len(counts), sum(counts)
+    gen = torch.Generator().manual_seed(K + seg_n)
+    idx = torch.cat([torch.full((c,), e, dtype=torch.int32) for e, c in enumerate(counts)])
+    idx = idx[torch.randperm(M, generator=gen)]
+    r = MoeRouting(M, 1, E, cuda_device)
+    r.topk_idx.copy_(idx.view(M, 1))
+    moe_group(r, M)
+    experts = []
+    for _ in range(E):
+        segs = []
+        for _ in range(n_segs):
+            w = _rand_fp8((seg_n, K), gen, cuda_device)
+            s = (torch.rand(seg_n // 128, K // 128, generator=gen) * 0.01).to(cuda_device)
+            segs.append((to_tiles(w) if layout else w, s))
+        experts.append(segs)
+    aq = to_tiles(_rand_fp8((M, K), gen, cuda_device))
+    a_s = torch.rand(M, K // 128, generator=gen).to(cuda_device)
+    assert M >= 4 * E  # the rule for the many-rows form
+    for gather in (True, False):
+        out = torch.full((M, n_segs * seg_n + 8), 7.0, dtype=torch.bfloat16, device=cuda_device)
+        plan = MoeLinearPlan(experts, out, layout)
+        got = plan(aq, a_s, r, gather=gather).clone()
+        out.fill_(7.0)
+        assert lib().ecf8_moe_linear(
+            aq.data_ptr(), a_s.data_ptr(), r.pair_tok.data_ptr() if gather else None,
+            r.offsets.data_ptr(), r.active.data_ptr(), r.n_active.data_ptr(), E,
+            plan.w_table.data_ptr(), plan.s_table.data_ptr(), n_segs, seg_n, K, layout,
+            out.data_ptr(), out.shape[1], torch.cuda.current_stream().cuda_stream) == 0
+        assert torch.equal(got.view(torch.int16), out.view(torch.int16))
+        assert bool((got[:, n_segs * seg_n:] == 7.0).all())
+
+
 @pytest.mark.parametrize("layout", [0, 1])
 @pytest.mark.parametrize("gather", [True, False])
 def test_grouped_expert_linear_matches_fp64(cuda_device, gather, layout):
