@@ -85,6 +85,10 @@ _SIGNATURES = {
     "ecf8_moe_linear_pairs": ([_vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _i32, _i64, _i64,
                                _i32, _i64, _vp, _i64, _vp], _i32),
     "ecf8_moe_combine": ([_vp, _i64, _vp, _vp, _i64, _i32, _i64, _vp, _vp], _i32),
+    # include/ecf8_attn.h: attention of many queries
+    "ecf8_packed_kv_elements": ([_i64, _i32, _i64], _i64),
+    "ecf8_prompt_attention": ([_vp, _vp, _vp, _i64, _i32, _i32, _i64, _i64, _vp, _vp, _vp, _vp],
+                              _i32),
 }
 
 EXPORTED = tuple(_SIGNATURES)

@@ -215,18 +215,14 @@ class _GreedyRunner:
         return min(marks[i].elapsed_time(marks[i + 1]) for i in range(reps)) / len(launches)
 
     def _prefill_attention(self, index: int, T: int):
-        """Causal attention of the prompt in fp32 (torch), positions 0..T-1."""
+        """Causal attention of the prompt, positions 0..T-1, in fp32 on the
+        bf16 queries and caches."""
         cfg = self.cfg
-        B, Hq, Hkv = self.B, cfg.heads, cfg.kv_heads
-        G = Hq // Hkv
-        q = self.q[: B * Hq * T * 128].view(B, Hq, T, 128).float()
-        k = self.kc[index][:, :, :T].float().repeat_interleave(G, dim=1)
-        v = self.vc[index][:, :, :T].float().repeat_interleave(G, dim=1)
-        s = torch.matmul(q, k.transpose(-1, -2).contiguous()) / math.sqrt(128)
-        mask = torch.ones(T, T, dtype=torch.bool, device=self.dev).triu(1)
-        s.masked_fill_(mask, float("-inf"))
-        o = torch.matmul(torch.softmax(s, dim=-1), v)
-        self.attn[: B * T].copy_(o.permute(0, 2, 1, 3).reshape(B * T, Hq * 128))
+        need = (self.B, cfg.kv_heads, T)
+        if getattr(self, "_kv_work", (None,))[0] != need:
+            self._kv_work = (need, K.packed_kv(*need, self.dev))
+        K.prompt_attention(self.q, self.kc[index], self.vc[index], T, self._kv_work[1], self.attn,
+                           cfg.heads)
 
     def _forward(self, prefill: bool):
         """All layers + final norm + lm_head; returns bf16 logits [B, vocab]

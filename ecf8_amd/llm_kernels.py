@@ -287,6 +287,35 @@ def decode_attention_fused(qkv, B, Hq, Hkv, q_norm, k_norm, eps, cos_t, sin_t, p
         _ptr(out_bf16), _stream(qkv)), "ecf8_decode_attention_fused")
 
 
+def packed_kv(B, Hkv, T, device):
+    """Work buffers (keys, values) of prompt_attention for T positions."""
+    n = lib().ecf8_packed_kv_elements(B, Hkv, T)
+    if n < 0:
+        raise ECF8Error("bad packed key / value size")
+    return tuple(torch.empty(n, dtype=torch.bfloat16, device=device) for _ in range(2))
+
+
+def prompt_attention(q, k_cache, v_cache, T, work, out, Hq):
+    """Causal attention of T prompt positions: the first B*Hq*T*128 elements
+    of ``q`` are [B, Hq, T, 128]; query t attends to cache positions [0, t];
+    out bf16 [>= B*T, Hq*128].  ``work``: ``packed_kv`` of this B, Hkv, T."""
+    dev = q.device
+    B, Hkv, Lmax, D = k_cache.shape
+    for t, n in ((q, "q"), (k_cache, "k_cache"), (v_cache, "v_cache"), (out, "out"),
+                 (work[0], "work"), (work[1], "work")):
+        _need(t, torch.bfloat16, n, dev)
+    if D != 128 or v_cache.shape != k_cache.shape or not 1 <= T <= Lmax:
+        raise ECF8Error("caches must be [B, Hkv, Lmax, 128] with Lmax >= T")
+    need = lib().ecf8_packed_kv_elements(B, Hkv, T)
+    if q.numel() < B * Hq * T * 128 or min(w.numel() for w in work) < need:
+        raise ECF8Error("q or work too small")
+    _rows(B * T, Hq * 128, out)
+    check(lib().ecf8_prompt_attention(q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), B, Hq,
+                                      Hkv, T, Lmax, work[0].data_ptr(), work[1].data_ptr(),
+                                      out.data_ptr(), _stream(q)), "ecf8_prompt_attention")
+    return out
+
+
 def dequant_fp8_block(weight, scale_inv, out=None):
     """bf16 [n, k] = e4m3fn weight x its 128x128 block scales."""
     dev = weight.device
