@@ -89,6 +89,11 @@ _SIGNATURES = {
     "ecf8_packed_kv_elements": ([_i64, _i32, _i64], _i64),
     "ecf8_prompt_attention": ([_vp, _vp, _vp, _i64, _i32, _i32, _i64, _i64, _vp, _vp, _vp, _vp],
                               _i32),
+    "ecf8_dit_qkv": ([_vp, _i32, _i64, _i32, _f32, _f32, _vp, _vp, _vp, _vp, _vp, _vp], _i32),
+    "ecf8_packed_attention": ([_vp, _vp, _vp, _i64, _i32, _i64, _vp, _i64, _vp], _i32),
+    "ecf8_dit_modulate": ([_vp, _i64, _i64, _i64, _vp, _i64, _vp, _i64, _f32, _vp, _vp], _i32),
+    "ecf8_dit_gated_add": ([_vp, _vp, _i64, _vp, _i64, _i64, _i64, _vp, _vp], _i32),
+    "ecf8_dit_gelu": ([_vp, _i64, _i64, _i64, _vp, _i64, _vp], _i32),
 }
 
 EXPORTED = tuple(_SIGNATURES)

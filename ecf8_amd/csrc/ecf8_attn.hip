@@ -13,6 +13,7 @@
 namespace {
 
 constexpr int kD = 128;      // head dimension
+constexpr float kLog2e = 1.4426950408889634f;
 constexpr int kBlock = 64;   // keys per step of the attention kernel
 constexpr int kQueries = 128;  // queries per workgroup: four waves of 32
 
@@ -278,14 +279,232 @@ __global__ __launch_bounds__(256) void pack_kv_kernel(const uint16_t *__restrict
   store_values(s_v, vo + (bh * (size_t)Tp + 32 * (size_t)tile) * kD);
 }
 
+// ------------------------------------------------------------ DiT operands
+
+__device__ __forceinline__ void load16(const uint16_t *p, float (&v)[16]) {
+  const u32x4 a = *reinterpret_cast<const u32x4 *>(p), b = *reinterpret_cast<const u32x4 *>(p + 8);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    v[2 * j] = bf16_f32(a[j] & 0xffffu);
+    v[2 * j + 1] = __uint_as_float(a[j] & 0xffff0000u);
+    v[8 + 2 * j] = bf16_f32(b[j] & 0xffffu);
+    v[8 + 2 * j + 1] = __uint_as_float(b[j] & 0xffff0000u);
+  }
+}
+
+// One stream's rows of the joint attention: the projection output (q heads,
+// then k heads, then v heads) and the head norms' weights.
+struct Stream {
+  const uint16_t *qkv;
+  const uint16_t *qn, *kn;
+  int64_t row, batch;  // elements between rows and between batches
+  int tokens;
+};
+
+// 32 tokens of one (batch, head): RMSNorm of the q and k heads and the
+// rotary embedding of interleaved pairs, in fp32; q scaled, rounded to bf16
+// and stored as rows, k and v packed for flash_kernel.  Tokens of `first`
+// come before those of `second`.  Eight threads a token, 16 dims each.
+// HBM bounds it: 6 bytes read and written per element where separate passes
+// moved fp32 copies of each.
+__global__ __launch_bounds__(256) void dit_qkv_kernel(Stream first, Stream second, int H, int T,
+                                                      int Tp, float eps, float scale,
+                                                      const float *__restrict__ cosv,
+                                                      const float *__restrict__ sinv,
+                                                      uint16_t *__restrict__ qo,
+                                                      uint16_t *__restrict__ ko,
+                                                      uint16_t *__restrict__ vo) {
+  __shared__ uint16_t s_v[32][kPad];
+  const int tiles = Tp / 32;
+  const int tile = blockIdx.x % tiles;
+  const int bh = blockIdx.x / tiles, b = bh / H, head = bh % H;
+  const int row = threadIdx.x >> 3, c = threadIdx.x & 7;
+  const int t = 32 * tile + row;
+  u32x4 k0 = {}, k1 = {}, v0 = {}, v1 = {};
+  if (t < T) {
+    const bool in = t < first.tokens;
+    const Stream &s = in ? first : second;
+    const uint16_t *p = s.qkv + (size_t)b * s.batch + (size_t)(in ? t : t - first.tokens) * s.row +
+                        (size_t)head * kD + 16 * c;
+    float q[16], k[16];
+    load16(p, q);
+    load16(p + (size_t)H * kD, k);
+    const u32x4 *vp = reinterpret_cast<const u32x4 *>(p + (size_t)2 * H * kD);
+    v0 = vp[0];
+    v1 = vp[1];
+    float co[8], si[8];
+#pragma unroll
+    for (int j = 0; j < 8; j += 4) {
+      const float4 cv = *reinterpret_cast<const float4 *>(cosv + (size_t)t * 64 + 8 * c + j);
+      const float4 sv = *reinterpret_cast<const float4 *>(sinv + (size_t)t * 64 + 8 * c + j);
+      co[j] = cv.x, co[j + 1] = cv.y, co[j + 2] = cv.z, co[j + 3] = cv.w;
+      si[j] = sv.x, si[j + 1] = sv.y, si[j + 2] = sv.z, si[j + 3] = sv.w;
+    }
+    auto norm_rope = [&](float (&x)[16], const uint16_t *nw, float sc) {
+      float ss = 0.f;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) ss = fmaf(x[i], x[i], ss);
+      ss += __shfl_xor(ss, 1);
+      ss += __shfl_xor(ss, 2);
+      ss += __shfl_xor(ss, 4);
+      const float rs = rsqrtf(ss / (float)kD + eps);
+      float w[16];
+      load16(nw + 16 * c, w);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float x0 = x[2 * j] * rs * w[2 * j], x1 = x[2 * j + 1] * rs * w[2 * j + 1];
+        x[2 * j] = (x0 * co[j] - x1 * si[j]) * sc;
+        x[2 * j + 1] = (x0 * si[j] + x1 * co[j]) * sc;
+      }
+    };
+    norm_rope(q, s.qn, scale);
+    norm_rope(k, s.kn, 1.f);
+    u32x4 q0, q1;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      q0[j] = pack_bf16(q[2 * j], q[2 * j + 1]);
+      q1[j] = pack_bf16(q[8 + 2 * j], q[8 + 2 * j + 1]);
+      k0[j] = pack_bf16(k[2 * j], k[2 * j + 1]);
+      k1[j] = pack_bf16(k[8 + 2 * j], k[8 + 2 * j + 1]);
+    }
+    u32x4 *qp = reinterpret_cast<u32x4 *>(qo + ((size_t)bh * T + t) * kD + 16 * c);
+    qp[0] = q0;
+    qp[1] = q1;
+  }
+  uint16_t *kb = ko + (size_t)bh * Tp * kD;
+  *reinterpret_cast<u32x4 *>(kb + packed_key(t, c, 0)) = k0;
+  *reinterpret_cast<u32x4 *>(kb + packed_key(t, c, 1)) = k1;
+  uint32_t *sv = reinterpret_cast<uint32_t *>(&s_v[row][16 * c]);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    sv[j] = v0[j];
+    sv[4 + j] = v1[j];
+  }
+  __syncthreads();
+  store_values(s_v, vo + ((size_t)bh * Tp + 32 * (size_t)tile) * kD);
+}
+
+// ------------------------------------------------- DiT elementwise passes
+//
+// Each replaces several library passes over fp32 or bf16 copies by one that
+// reads its inputs once and writes its output once (HBM-bound), with the
+// roundings of the passes it replaces.
+
+__device__ __forceinline__ void unpack8(u32x4 v, float (&f)[8]) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    f[2 * j] = bf16_f32(v[j] & 0xffffu);
+    f[2 * j + 1] = __uint_as_float(v[j] & 0xffff0000u);
+  }
+}
+
+__device__ __forceinline__ u32x4 pack8(const float (&f)[8]) {
+  return u32x4{pack_bf16(f[0], f[1]), pack_bf16(f[2], f[3]), pack_bf16(f[4], f[5]),
+               pack_bf16(f[6], f[7])};
+}
+
+// The sum over the 256 threads, in every thread, in a fixed order.
+__device__ __forceinline__ float block_sum(float v, float *part) {
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+  __syncthreads();  // part may still be read from the last sum
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
+  __syncthreads();
+  return (part[0] + part[1]) + (part[2] + part[3]);
+}
+
+// out = bf16(LayerNorm(x) * (1 + scale) + shift) per row of C <= 2048 kV,
+// mean and variance in fp32 from the row held in registers.
+template <int kV>
+__global__ __launch_bounds__(256) void modulate_kernel(const uint16_t *__restrict__ x, int rows,
+                                                       int C, const uint16_t *__restrict__ shift,
+                                                       int64_t shift_batch,
+                                                       const uint16_t *__restrict__ scale,
+                                                       int64_t scale_batch, float eps,
+                                                       uint16_t *__restrict__ out) {
+  __shared__ float part[4];
+  const size_t m = blockIdx.x;
+  const size_t b = m / (size_t)rows;
+  float v[kV][8];
+  float sum = 0.f;
+#pragma unroll
+  for (int i = 0; i < kV; ++i) {
+    const int c = 2048 * i + 8 * threadIdx.x;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[i][j] = 0.f;
+    if (c < C) unpack8(*reinterpret_cast<const u32x4 *>(x + m * C + c), v[i]);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) sum += v[i][j];
+  }
+  const float mean = block_sum(sum, part) / (float)C;
+  float sq = 0.f;
+#pragma unroll
+  for (int i = 0; i < kV; ++i) {
+    if (2048 * i + 8 * (int)threadIdx.x >= C) continue;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      v[i][j] -= mean;
+      sq = fmaf(v[i][j], v[i][j], sq);
+    }
+  }
+  const float rs = rsqrtf(block_sum(sq, part) / (float)C + eps);
+#pragma unroll
+  for (int i = 0; i < kV; ++i) {
+    const int c = 2048 * i + 8 * threadIdx.x;
+    if (c >= C) continue;
+    float sh[8], sc[8];
+    unpack8(*reinterpret_cast<const u32x4 *>(shift + b * shift_batch + c), sh);
+    unpack8(*reinterpret_cast<const u32x4 *>(scale + b * scale_batch + c), sc);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[i][j] = v[i][j] * rs * (1.f + sc[j]) + sh[j];
+    *reinterpret_cast<u32x4 *>(out + m * C + c) = pack8(v[i]);
+  }
+}
+
+// out = bf16(x + bf16(gate * y)) per row of C, gate per batch.
+__global__ __launch_bounds__(256) void gated_add_kernel(const uint16_t *__restrict__ x,
+                                                        const uint16_t *__restrict__ gate,
+                                                        int64_t gate_batch,
+                                                        const uint16_t *__restrict__ y,
+                                                        int64_t units, int rows, int C,
+                                                        uint16_t *__restrict__ out) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;  // 8 elements
+  if (i >= units) return;
+  const int64_t m = i / (C / 8);
+  const int c = 8 * (int)(i - m * (C / 8));
+  float xf[8], gf[8], yf[8];
+  unpack8(*reinterpret_cast<const u32x4 *>(x + 8 * i), xf);
+  unpack8(*reinterpret_cast<const u32x4 *>(y + 8 * i), yf);
+  unpack8(*reinterpret_cast<const u32x4 *>(gate + (m / rows) * gate_batch + c), gf);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) xf[j] += bf16_f32(pack_bf16(gf[j] * yf[j], 0.f) & 0xffffu);
+  *reinterpret_cast<u32x4 *>(out + 8 * i) = pack8(xf);
+}
+
+// out[m, :C] = bf16(gelu_tanh(x[m, :C])), both with a row stride: 0.5 x (1 +
+// tanh(u)) = x / (1 + exp(-2 u)), u = sqrt(2 / pi) (x + 0.044715 x^3).
+__global__ __launch_bounds__(256) void gelu_kernel(const uint16_t *__restrict__ x, int64_t x_row,
+                                                   int64_t units, int C,
+                                                   uint16_t *__restrict__ out, int64_t out_row) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= units) return;
+  const int64_t m = i / (C / 8);
+  const int c = 8 * (int)(i - m * (C / 8));
+  float v[8];
+  unpack8(*reinterpret_cast<const u32x4 *>(x + m * x_row + c), v);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float u = 0.7978845608028654f * (v[j] + 0.044715f * v[j] * v[j] * v[j]);
+    v[j] = v[j] * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-2.f * kLog2e * u));
+  }
+  *reinterpret_cast<u32x4 *>(out + m * out_row + c) = pack8(v);
+}
+
 inline hipStream_t as_stream(void *s) { return reinterpret_cast<hipStream_t>(s); }
 inline bool aligned(const void *p, uintptr_t a) {
   return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0;
 }
 inline int launched() { return hipGetLastError() == hipSuccess ? ECF8_OK : ECF8_ERR_HIP; }
 inline int64_t padded(int64_t T) { return (T + kBlock - 1) / kBlock * kBlock; }
-
-constexpr float kLog2e = 1.4426950408889634f;
 
 }  // namespace
 
@@ -316,5 +535,112 @@ extern "C" int ecf8_prompt_attention(const void *q, const void *k_cache, const v
                (int64_t)Hq * kD, (int)T, (int)Tp, Hq, Hq / Hkv, (int)tiles, (int)(B * Hq),
                kLog2e / sqrtf((float)kD)};
   flash_kernel<true, true><<<(unsigned)(B * Hq * tiles), 256, 0, as_stream(stream)>>>(a);
+  return launched();
+}
+
+extern "C" int ecf8_dit_qkv(const ecf8_dit_stream *streams, int n_streams, int64_t B, int H,
+                            float eps, float scale, const float *cos_t, const float *sin_t,
+                            void *q, void *k_packed, void *v_packed, void *stream) {
+  if (!streams || n_streams < 1 || n_streams > 2 || B <= 0 || H <= 0 || !cos_t || !sin_t || !q ||
+      !k_packed || !v_packed)
+    return ECF8_ERR_INVALID_ARG;
+  Stream s[2] = {};
+  int64_t T = 0;
+  for (int i = 0; i < n_streams; ++i) {
+    const ecf8_dit_stream &g = streams[i];
+    if (!g.qkv || !g.q_norm || !g.k_norm || g.tokens <= 0) return ECF8_ERR_INVALID_ARG;
+    if (g.row_stride < 3 * (int64_t)H * kD || g.row_stride % 8 || g.batch_stride % 8 ||
+        (B > 1 && g.batch_stride < g.row_stride))
+      return ECF8_ERR_UNSUPPORTED;
+    if (!aligned(g.qkv, 16) || !aligned(g.q_norm, 16) || !aligned(g.k_norm, 16))
+      return ECF8_ERR_MISALIGNED;
+    if (g.tokens > (1 << 24)) return ECF8_ERR_UNSUPPORTED;
+    s[i] = Stream{static_cast<const uint16_t *>(g.qkv), static_cast<const uint16_t *>(g.q_norm),
+                  static_cast<const uint16_t *>(g.k_norm), g.row_stride, g.batch_stride,
+                  (int)g.tokens};
+    T += g.tokens;
+  }
+  const int64_t Tp = padded(T);
+  if (T > (1 << 24) || B > (1 << 24) || B * H * (Tp / 32) > INT32_MAX) return ECF8_ERR_UNSUPPORTED;
+  if (!aligned(cos_t, 16) || !aligned(sin_t, 16) || !aligned(q, 16) || !aligned(k_packed, 16) ||
+      !aligned(v_packed, 16))
+    return ECF8_ERR_MISALIGNED;
+  dit_qkv_kernel<<<(unsigned)(B * H * (Tp / 32)), 256, 0, as_stream(stream)>>>(
+      s[0], s[1], H, (int)T, (int)Tp, eps, scale, cos_t, sin_t, static_cast<uint16_t *>(q),
+      static_cast<uint16_t *>(k_packed), static_cast<uint16_t *>(v_packed));
+  return launched();
+}
+
+extern "C" int ecf8_packed_attention(const void *q, const void *k_packed, const void *v_packed,
+                                     int64_t B, int H, int64_t T, void *out, int64_t out_stride,
+                                     void *stream) {
+  if (!q || !k_packed || !v_packed || !out || B <= 0 || H <= 0 || T <= 0)
+    return ECF8_ERR_INVALID_ARG;
+  const int64_t tiles = (T + kQueries - 1) / kQueries;
+  if (T > (1 << 24) || B > (1 << 24) || B * H * tiles > INT32_MAX || out_stride % 4)
+    return ECF8_ERR_UNSUPPORTED;
+  if (out_stride < (int64_t)H * kD) return ECF8_ERR_CAPACITY;
+  if (!aligned(q, 16) || !aligned(k_packed, 16) || !aligned(v_packed, 16) || !aligned(out, 8))
+    return ECF8_ERR_MISALIGNED;
+  const Attn a{static_cast<const uint16_t *>(q), static_cast<const uint16_t *>(k_packed),
+               static_cast<const uint16_t *>(v_packed), static_cast<uint16_t *>(out), out_stride,
+               (int)T, (int)padded(T), H, 1, (int)tiles, (int)(B * H), kLog2e};
+  flash_kernel<false, false><<<(unsigned)(B * H * tiles), 256, 0, as_stream(stream)>>>(a);
+  return launched();
+}
+
+extern "C" int ecf8_dit_modulate(const void *x, int64_t B, int64_t rows, int64_t C,
+                                 const void *shift, int64_t shift_batch, const void *scale,
+                                 int64_t scale_batch, float eps, void *out, void *stream) {
+  if (!x || !shift || !scale || !out || B <= 0 || rows <= 0 || C <= 0) return ECF8_ERR_INVALID_ARG;
+  if (C % 8 || C > 8192 || shift_batch % 8 || scale_batch % 8 || rows > (1 << 24) ||
+      B * rows > INT32_MAX)
+    return ECF8_ERR_UNSUPPORTED;
+  if (!aligned(x, 16) || !aligned(shift, 16) || !aligned(scale, 16) || !aligned(out, 16))
+    return ECF8_ERR_MISALIGNED;
+  const auto *xp = static_cast<const uint16_t *>(x), *sh = static_cast<const uint16_t *>(shift),
+             *sc = static_cast<const uint16_t *>(scale);
+  auto *op = static_cast<uint16_t *>(out);
+  const unsigned grid = (unsigned)(B * rows);
+#define ECF8_MODULATE(V)                                                                        \
+  modulate_kernel<V><<<grid, 256, 0, as_stream(stream)>>>(xp, (int)rows, (int)C, sh, shift_batch, \
+                                                          sc, scale_batch, eps, op)
+  if (C <= 2048)
+    ECF8_MODULATE(1);
+  else if (C <= 4096)
+    ECF8_MODULATE(2);
+  else
+    ECF8_MODULATE(4);
+#undef ECF8_MODULATE
+  return launched();
+}
+
+extern "C" int ecf8_dit_gated_add(const void *x, const void *gate, int64_t gate_batch,
+                                  const void *y, int64_t B, int64_t rows, int64_t C, void *out,
+                                  void *stream) {
+  if (!x || !gate || !y || !out || B <= 0 || rows <= 0 || C <= 0) return ECF8_ERR_INVALID_ARG;
+  const int64_t units = B * rows * (C / 8);
+  if (C % 8 || C > (1 << 24) || gate_batch % 8 || rows > (1 << 24) || B > (1 << 24) ||
+      (units + 255) / 256 > INT32_MAX)
+    return ECF8_ERR_UNSUPPORTED;
+  if (!aligned(x, 16) || !aligned(gate, 16) || !aligned(y, 16) || !aligned(out, 16))
+    return ECF8_ERR_MISALIGNED;
+  gated_add_kernel<<<(unsigned)((units + 255) / 256), 256, 0, as_stream(stream)>>>(
+      static_cast<const uint16_t *>(x), static_cast<const uint16_t *>(gate), gate_batch,
+      static_cast<const uint16_t *>(y), units, (int)rows, (int)C, static_cast<uint16_t *>(out));
+  return launched();
+}
+
+extern "C" int ecf8_dit_gelu(const void *x, int64_t x_row, int64_t rows, int64_t C, void *out,
+                             int64_t out_row, void *stream) {
+  if (!x || !out || rows <= 0 || C <= 0 || x_row < C || out_row < C) return ECF8_ERR_INVALID_ARG;
+  const int64_t units = rows * (C / 8);
+  if (C % 8 || C > (1 << 24) || x_row % 8 || out_row % 8 || rows > INT32_MAX ||
+      (units + 255) / 256 > INT32_MAX)
+    return ECF8_ERR_UNSUPPORTED;
+  if (!aligned(x, 16) || !aligned(out, 16)) return ECF8_ERR_MISALIGNED;
+  gelu_kernel<<<(unsigned)((units + 255) / 256), 256, 0, as_stream(stream)>>>(
+      static_cast<const uint16_t *>(x), x_row, units, (int)C, static_cast<uint16_t *>(out),
+      out_row);
   return launched();
 }

@@ -19,9 +19,12 @@ conditioning.  Random init.
 Compute: the FP8 Linears run at thousands of rows, where the work is
 matrix-bound, so each one dequantizes its e4m3fn weight with its 128x128
 block scales to bf16 (ecf8_dequant_fp8_block) and calls the library bf16
-GEMM; attention runs on bf16 operands with fp32 accumulation (chunked over
-queries), the precision of the reference's bf16 pipeline.  The same
-consumer runs for the compressed and the uncompressed model.
+GEMM; attention runs on bf16 operands with fp32 scores, softmax and sums
+(ecf8_amd.dit_kernels, with the head norms, the rotary embedding and the
+elementwise passes around it), the precision of the reference's bf16
+pipeline or better.  The same consumer runs for the compressed and the
+uncompressed model.  What those kernels do not take (autograd, other
+devices and head dimensions) runs the same computation in torch.
 """
 
 from __future__ import annotations
@@ -34,6 +37,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from . import dit_kernels as DK
 from . import llm_kernels as K
 from .llm import FP8Linear
 
@@ -104,8 +108,16 @@ def _bf16_linear(i, o):
 
 
 def _modulate(x, shift, scale):
+    out = DK.modulate(x, shift, scale)
+    if out is not None:
+        return out
     x = F.layer_norm(x.float(), (x.shape[-1],), eps=1e-6)
     return (x * (1 + scale.float()[:, None]) + shift.float()[:, None]).to(torch.bfloat16)
+
+
+def _gated_add(x, gate, y):
+    out = DK.gated_add(x, gate, y)
+    return x + gate[:, None] * y if out is None else out
 
 
 def _rope(x, cos, sin):
@@ -176,18 +188,22 @@ class DoubleBlock(nn.Module):
         at = self.attn
         sa, ca, ga, sma, cma, gma = self.norm1_a(emb)
         sb, cb, gb, smb, cmb, gmb = self.norm1_b(emb)
-        qa, ka, va = _heads(at.a_to_qkv(_modulate(img, sa, ca)), at.heads * 3).chunk(3, dim=1)
-        qb, kb, vb = _heads(at.b_to_qkv(_modulate(txt, sb, cb)), at.heads * 3).chunk(3, dim=1)
-        q = torch.cat([at.norm_q_b(qb), at.norm_q_a(qa)], dim=2)
-        k = torch.cat([at.norm_k_b(kb), at.norm_k_a(ka)], dim=2)
-        v = torch.cat([vb.float(), va.float()], dim=2)
-        o = _attention(_rope(q, cos, sin), _rope(k, cos, sin), v)
-        o = o.transpose(1, 2).reshape(img.shape[0], -1, img.shape[-1]).to(torch.bfloat16)
+        qkv_a, qkv_b = at.a_to_qkv(_modulate(img, sa, ca)), at.b_to_qkv(_modulate(txt, sb, cb))
+        o = DK.joint_attention([(qkv_b, at.norm_q_b, at.norm_k_b),
+                                (qkv_a, at.norm_q_a, at.norm_k_a)], at.heads, cos, sin)
+        if o is None:
+            qa, ka, va = _heads(qkv_a, at.heads * 3).chunk(3, dim=1)
+            qb, kb, vb = _heads(qkv_b, at.heads * 3).chunk(3, dim=1)
+            q = torch.cat([at.norm_q_b(qb), at.norm_q_a(qa)], dim=2)
+            k = torch.cat([at.norm_k_b(kb), at.norm_k_a(ka)], dim=2)
+            v = torch.cat([vb.float(), va.float()], dim=2)
+            o = _attention(_rope(q, cos, sin), _rope(k, cos, sin), v)
+            o = o.transpose(1, 2).reshape(img.shape[0], -1, img.shape[-1]).to(torch.bfloat16)
         n_txt = txt.shape[1]
-        img = img + ga[:, None] * at.a_to_out(o[:, n_txt:])
-        txt = txt + gb[:, None] * at.b_to_out(o[:, :n_txt])
-        img = img + gma[:, None] * self.ff_a(_modulate(img, sma, cma))
-        txt = txt + gmb[:, None] * self.ff_b(_modulate(txt, smb, cmb))
+        img = _gated_add(img, ga, at.a_to_out(o[:, n_txt:]))
+        txt = _gated_add(txt, gb, at.b_to_out(o[:, :n_txt]))
+        img = _gated_add(img, gma, self.ff_a(_modulate(img, sma, cma)))
+        txt = _gated_add(txt, gmb, self.ff_b(_modulate(txt, smb, cmb)))
         return img, txt
 
 
@@ -211,12 +227,15 @@ class SingleBlock(nn.Module):
         shift, scale, gate = self.norm.linear(F.silu(emb)).chunk(3, dim=-1)
         y = self.to_qkv_mlp(_modulate(x, shift, scale))
         qkv, mlp = y[..., : 3 * self.hidden], y[..., 3 * self.hidden:]
-        q, k, v = _heads(qkv, self.heads * 3).chunk(3, dim=1)
-        o = _attention(_rope(self.norm_q_a(q), cos, sin), _rope(self.norm_k_a(k), cos, sin),
-                       v.float())
-        o = o.transpose(1, 2).reshape(x.shape[0], -1, self.hidden).to(torch.bfloat16)
-        out = self.proj_out(torch.cat([o, F.gelu(mlp, approximate="tanh")], dim=-1))
-        return x + gate[:, None] * out
+        o = DK.joint_attention([(qkv, self.norm_q_a, self.norm_k_a)], self.heads, cos, sin,
+                               tail=mlp)
+        if o is None:
+            q, k, v = _heads(qkv, self.heads * 3).chunk(3, dim=1)
+            o = _attention(_rope(self.norm_q_a(q), cos, sin), _rope(self.norm_k_a(k), cos, sin),
+                           v.float())
+            o = o.transpose(1, 2).reshape(x.shape[0], -1, self.hidden).to(torch.bfloat16)
+            o = torch.cat([o, F.gelu(mlp, approximate="tanh")], dim=-1)
+        return _gated_add(x, gate, self.proj_out(o))
 
 
 def _timestep_embedding(t: torch.Tensor, dim: int = 256) -> torch.Tensor:

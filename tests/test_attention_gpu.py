@@ -67,3 +67,147 @@ def test_prompt_attention_refuses_what_does_not_fit(cuda_device):
         a = {**dict(q=q, kc=kc, T=8, work=work, out=out, Hq=4), **bad}
         with pytest.raises(ECF8Error):
             prompt_attention(a["q"], a["kc"], a["kc"], a["T"], a["work"], a["out"], a["Hq"])
+
+
+def _dit_reference(streams, heads, cos, sin, tail):
+    """Float64 restatement of dit_kernels.joint_attention."""
+    qs, ks, vs = [], [], []
+    for t, nq, nk in streams:
+        q, k, v = t.double().unflatten(2, (3, heads, 128)).permute(2, 0, 3, 1, 4)
+
+        def norm(x, w):
+            return x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + 1e-6) * w.weight.double()
+
+        qs.append(norm(q, nq))
+        ks.append(norm(k, nk))
+        vs.append(v)
+
+    def rope(x):
+        x0, x1 = x[..., 0::2], x[..., 1::2]
+        c, s = cos.double(), sin.double()
+        return torch.stack([x0 * c - x1 * s, x0 * s + x1 * c], -1).flatten(-2)
+
+    q, k, v = rope(torch.cat(qs, 2)), rope(torch.cat(ks, 2)), torch.cat(vs, 2)
+    o = torch.softmax(q @ k.transpose(-1, -2).contiguous() / math.sqrt(128), -1) @ v
+    o = o.transpose(1, 2).flatten(2)
+    if tail is not None:
+        x = tail.double()
+        g = 0.5 * x * (1 + torch.tanh(math.sqrt(2 / math.pi) * (x + 0.044715 * x ** 3)))
+        o = torch.cat([o, g], -1)
+    return o
+
+
+@pytest.mark.parametrize("B,tokens,heads,tail", [
+    (1, (1,), 1, 0), (1, (31, 32), 8, 0), (2, (5, 59), 2, 0), (1, (64,), 3, 8), (1, (65,), 8, 520),
+    (2, (127,), 2, 264), (1, (1, 127), 1, 0), (1, (128, 1), 16, 0), (3, (200,), 4, 1024)])
+def test_dit_joint_attention_matches_fp64(cuda_device, B, tokens, heads, tail):
+    """One stream (a strided slice of a wider projection, with a GELU tail)
+    and two, at the edges of the 32-token, 64-key and 128-query tiles.
+    Against fp64, relative L2: q, k and the probabilities are rounded to
+    bf16 (2^-8 largest, 2^-9.8 rms), the output again: 4 * 2^-9.8."""
+    from ecf8_amd import dit_kernels as DK
+    from ecf8_amd.dit import _Norm
+
+    gen = torch.Generator(device=cuda_device).manual_seed(sum(tokens) * 10 + heads)
+
+    def rand(*shape):
+        return torch.randn(shape, generator=gen, device=cuda_device).to(torch.bfloat16)
+
+    C, streams, last = heads * 128, [], None
+    for n in tokens:
+        y = rand(B, n, 3 * C + tail)
+        norms = [_Norm(128).to(cuda_device) for _ in range(2)]
+        for m in norms:
+            m.weight.data.copy_(1 + 0.2 * rand(128).float())
+        streams.append((y[..., : 3 * C], *norms))
+        last = y[..., 3 * C:] if tail else None
+    T = sum(tokens)
+    angle = torch.rand(1, 1, T, 64, generator=gen, device=cuda_device) * 6.28
+    cos, sin = torch.cos(angle), torch.sin(angle)
+    got = DK.joint_attention(streams, heads, cos, sin, tail=last)
+    assert got.shape == (B, T, C + tail) and got.dtype == torch.bfloat16
+    want = _dit_reference(streams, heads, cos, sin, last)
+    for part in (slice(0, C), slice(C, C + tail)):
+        if want[..., part].numel():
+            err = (got[..., part].double() - want[..., part]).norm() / want[..., part].norm()
+            assert float(err) <= 4 * 2.0 ** -9.8, float(err)
+
+
+@pytest.mark.parametrize("B,T,C", [(1, 1, 8), (2, 3, 2048), (1, 5, 2056), (2, 2, 4096), (1, 3, 8192)])
+def test_dit_elementwise_matches_torch(cuda_device, B, T, C):
+    """LayerNorm modulation (fp32, one bf16 rounding: at most one ulp from
+    torch's) and gated add (the same two roundings: bit-identical)."""
+    import torch.nn.functional as F
+
+    from ecf8_amd import dit_kernels as DK
+
+    gen = torch.Generator(device=cuda_device).manual_seed(C)
+
+    def rand(*shape):
+        return torch.randn(shape, generator=gen, device=cuda_device).to(torch.bfloat16)
+
+    x, y, emb = rand(B, T, C) + 0.5, rand(B, T, C), rand(B, 6 * C)
+    shift, scale, gate = emb.chunk(6, dim=-1)[1:4]
+    want = F.layer_norm(x.float(), (C,), eps=1e-6) * (1 + scale.float()[:, None])
+    want = (want + shift.float()[:, None])
+    got = DK.modulate(x, shift, scale)
+    assert bool(((got.float() - want).abs() <= want.abs() * 2.0 ** -8 * 1.01 + 1e-5).all())
+    assert torch.equal(DK.gated_add(x, gate, y), x + gate[:, None] * y)
+
+
+@pytest.mark.parametrize("B", [1, 2])
+@pytest.mark.parametrize("kind", ["single", "double"])
+def test_dit_blocks_agree_with_the_torch_path(cuda_device, monkeypatch, kind, B):
+    """A block's forward through the kernels against the same forward in
+    torch: bf16 roundings at the same places, scores kept in fp32 instead of
+    bf16 (2 % of the block's update), and the update added to x and rounded
+    to bf16 up to twice, each rounding 2^-9.8 of x rms on either side: 2 *
+    sqrt(2) * 2^-9.8 < 2^-8 of the output's norm.  Also what the kernels leave
+    to torch: autograd, transposed inputs, fp16 autocast, hooks on a norm."""
+    from ecf8_amd import dit_kernels as DK
+    from ecf8_amd.dit import FluxConfig, random_pipeline
+
+    cfg = FluxConfig(hidden=256, heads=2, mlp=512, double=1, single=1, txt_dim=128, pooled_dim=128)
+    pipe, _ = random_pipeline(cfg, cuda_device, seed=5)
+    gen = torch.Generator(device=cuda_device).manual_seed(B)
+
+    def rand(*shape):
+        return torch.randn(shape, generator=gen, device=cuda_device).to(torch.bfloat16)
+
+    img, txt, emb = rand(B, 35, 256), rand(B, 7, 256), rand(B, 256)
+    cos, sin = pipe.dit.rope_tables(7, 5, 7, cuda_device)
+    blk, args = ((pipe.dit.blocks[0], (img, txt, emb)) if kind == "double"
+                 else (pipe.dit.single_blocks[0], (torch.cat([txt, img], 1), emb)))
+    calls = []
+    monkeypatch.setattr(DK, "_launch", lambda *a, _f=DK._launch: (calls.append(a[1]), _f(*a))[1])
+
+    def run(*a):
+        calls.clear()
+        out = blk(*a, cos, sin)
+        return out if isinstance(out, tuple) else (out,)
+
+    with torch.no_grad():
+        fused = run(*args)
+        assert "ecf8_packed_attention" in calls and "ecf8_dit_modulate" in calls
+        with monkeypatch.context() as mp:
+            mp.setattr(DK, "_untracked", lambda: False)
+            plain = run(*args)
+        assert not calls
+        for a, b, x in zip(fused, plain, args):
+            diff, update = (a.double() - b.double()).norm(), (b.double() - x.double()).norm()
+            assert float(diff) <= 0.02 * float(update) + 2.0 ** -8 * float(b.double().norm())
+        turned = [t.transpose(1, 2).contiguous().transpose(1, 2) if t.dim() == 3 else t for t in args]
+        for a, b in zip(run(*turned), plain):
+            assert float((a.double() - b.double()).norm() / b.double().norm()) <= 0.02
+        with torch.autocast("cuda", dtype=torch.float16):
+            run(*args)
+        assert not calls
+        norm = blk.attn.norm_k_a if kind == "double" else blk.norm_k_a
+        seen = []
+        handle = norm.register_forward_hook(lambda *_: seen.append(1))
+        run(*args)
+        handle.remove()
+        assert seen and "ecf8_packed_attention" not in calls
+    leaf = args[0].clone().requires_grad_()
+    run(leaf, *args[1:])[0].float().sum().backward()
+    assert "ecf8_packed_attention" not in calls and bool(torch.isfinite(leaf.grad).all())
