@@ -231,6 +231,7 @@ struct WeightLane {
 // contiguous run of tiles, column block by column block: the weight block
 // a tile column reads stays in that XCD's L2 across its row blocks.
 typedef int v8i __attribute__((ext_vector_type(8)));
+typedef int v4i __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ void lds_load16(const uint8_t *g, void *lds) {
   __builtin_amdgcn_global_load_lds(g, (__attribute__((address_space(3))) void *)lds, 16, 0, 0);
@@ -436,6 +437,140 @@ __global__ __launch_bounds__(kGemmWaves * 64) void fp8_gemm_kernel(
         for (int j = 0; j < 4; ++j) o[16 * j] = (uint16_t)f32_bf16(acc[i][j][q]);
       }
     }
+}
+
+// ------------------------------------------ middle form (16 < M, few tiles)
+//
+// The tile GEMM above has one workgroup per 256 x 128 outputs: a few dozen
+// at the row counts of a served batch or a short prompt, most CUs idle.
+// Here a workgroup of eight waves computes 16 kCh rows x 16 P columns and
+// splits K over its waves (wave w: the w-th run of groups); a wave reads its
+// operands straight into registers in MFMA order, one group ahead, and the
+// waves' sums meet in LDS and are added in wave order.  P trades the
+// number of workgroups against re-reading the activations per column strip
+// (from L2).  HBM or L2 bounds it; MI355X, 64 rows: N = K = 4096 34.8 -> 8.9
+// us, N = 4096, K = 12288 94 -> 20 us.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+template <int P, int kCh>
+__global__ __launch_bounds__(512) void fp8_rows_kernel(const uint8_t *__restrict__ aq,
+                                                       const float *__restrict__ as, int M, int K,
+                                                       LinearSegs segs, uint16_t *__restrict__ out,
+                                                       int ldo) {
+  constexpr int kWaves = 8, kVals = 4 * kCh;
+  __shared__ float red[kWaves][kVals][64];
+  __shared__ __attribute__((aligned(16))) float s_sc[kWaves][2][64];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, g = lane >> 4;
+  const int kgroups = K / kGroup;
+  const int m0 = blockIdx.y * 16 * kCh;
+
+  int n0 = blockIdx.x * 16 * P;
+  const uint8_t *w = segs.w[0];
+  const float *ws = segs.ws[0];
+  int col = segs.col[0], seg_start = 0, wt = segs.tiled[0];
+#pragma unroll
+  for (int s = 1; s < ECF8_LINEAR_MAX_SEGS; ++s) {
+    if (s < segs.count && n0 >= segs.n_end[s - 1]) {
+      w = segs.w[s];
+      ws = segs.ws[s];
+      col = segs.col[s];
+      wt = segs.tiled[s];
+      seg_start = segs.n_end[s - 1];
+    }
+  }
+  n0 -= seg_start;  // 16 P divides 128, so the strip lies in one segment and scale row
+  const float *wsrow = ws + (size_t)(n0 / kGroup) * kgroups;
+  const WeightLane wl(w, wt != 0, n0, r, g, K);
+  // the strip's 16 P rows x K bytes; panel p starts 16 K bytes after p - 1
+  const Rsrc wr = make_rsrc(wl.base, 16u * P * (uint32_t)K);
+  const int last_rb = (M + 15) / 16 - 1;  // rows past M read the last 16-row block
+  const uint8_t *ab[kCh];
+#pragma unroll
+  for (int c = 0; c < kCh; ++c)
+    ab[c] = aq + (size_t)min(m0 / 16 + c, last_rb) * kgroups * 2048 + 16 * lane;
+  const float *asr = as + (size_t)min(m0 + min(lane, 16 * kCh - 1), M - 1) * kgroups;
+
+  const int run = (kgroups + kWaves - 1) / kWaves;
+  const int k0 = wave * run, k1 = min(k0 + run, kgroups);
+
+  struct Stage {
+    u32x4 wv[P][2], av[kCh][2];
+    float sa, sw;
+  };
+  auto load = [&](int kg, Stage &s) {
+    const int k = min(kg, kgroups - 1);  // past the run: loaded, unused
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      const uint32_t at = (uint32_t)k * (uint32_t)wl.step + 16u * (uint32_t)p * (uint32_t)K;
+      s.wv[p][0] = __builtin_amdgcn_raw_buffer_load_b128(wr, wl.lane, at, 0);
+      s.wv[p][1] = __builtin_amdgcn_raw_buffer_load_b128(wr, wl.lane, at + (uint32_t)wl.half, 0);
+    }
+#pragma unroll
+    for (int c = 0; c < kCh; ++c) {
+      s.av[c][0] = *reinterpret_cast<const u32x4 *>(ab[c] + (size_t)k * 2048);
+      s.av[c][1] = *reinterpret_cast<const u32x4 *>(ab[c] + (size_t)k * 2048 + 1024);
+    }
+    s.sa = asr[k];
+    s.sw = wsrow[k];
+  };
+  v4f acc[P][kCh];
+#pragma unroll
+  for (int p = 0; p < P; ++p)
+#pragma unroll
+    for (int c = 0; c < kCh; ++c) acc[p][c] = v4f{0.f, 0.f, 0.f, 0.f};
+  auto step = [&](const Stage &s, int buf) {
+    // the rows' scales, lane = row, to the lanes that hold those rows' sums
+    // (the wave's own LDS: program order, no barrier)
+    s_sc[wave][buf][lane] = s.sa * s.sw;
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int c = 0; c < kCh; ++c) {
+      const f32x4 sc = *reinterpret_cast<const f32x4 *>(&s_sc[wave][buf][16 * c + 4 * g]);
+      const v8i a = __builtin_shufflevector(__builtin_bit_cast(v4i, s.av[c][0]),
+                                            __builtin_bit_cast(v4i, s.av[c][1]), 0, 1, 2, 3, 4, 5,
+                                            6, 7);
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+        const v8i b = __builtin_shufflevector(__builtin_bit_cast(v4i, s.wv[p][0]),
+                                              __builtin_bit_cast(v4i, s.wv[p][1]), 0, 1, 2, 3, 4,
+                                              5, 6, 7);
+        const v4f z = {0.f, 0.f, 0.f, 0.f};
+        const v4f d = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, z, 0, 0, 0, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[p][c][i] = fmaf(d[i], sc[i], acc[p][c][i]);
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+  };
+  if (k0 < k1) {
+    Stage s0, s1;
+    load(k0, s0);
+    for (int kg = k0; kg < k1; kg += 2) {
+      load(kg + 1, s1);
+      step(s0, 0);
+      load(kg + 2, s0);
+      if (kg + 1 < k1) step(s1, 1);  // uniform
+    }
+  }
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    if (p) __syncthreads();  // red is rewritten
+#pragma unroll
+    for (int c = 0; c < kCh; ++c)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) red[wave][4 * c + i][lane] = acc[p][c][i];
+    __syncthreads();
+    for (int t = threadIdx.x; t < 64 * kVals; t += 512) {
+      const int ci = t >> 6, l = t & 63;
+      float sum = 0.f;
+#pragma unroll
+      for (int v = 0; v < kWaves; ++v) sum += red[v][ci][l];
+      const int m = m0 + 16 * (ci >> 2) + 4 * (l >> 4) + (ci & 3);
+      if (m < M) out[(size_t)m * ldo + col + n0 + 16 * p + (l & 15)] = (uint16_t)f32_bf16(sum);
+    }
+  }
 }
 
 // Small-M form (M <= 16, the decode step): one 16-row MFMA tile per
@@ -1691,6 +1826,44 @@ extern "C" int ecf8_fp8_linear(const void *aq, const float *as, int64_t M, int64
       fp8_linear16_kernel<8><<<n_tiles, 512, 0, as_stream(stream)>>>(a, as, (int)M, (int)K, s, o,
                                                                      (int)ldo);
   } else {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+      return ECF8_ERR_HIP;
+    // The middle form while its 64 x 64 blocks are at most two per CU: the
+    // tile GEMM then has at most one workgroup on a quarter of the CUs.
+    // MI355X, us, middle form against tile GEMM (four weight copies rotated):
+    // N = K = 4096: M = 64 8.9 / 34.8, M = 256 13.4 / 35.6, M = 512 (512
+    // blocks) 24.3 / 36.2, M = 768 35.0 / 36.7, M = 1024 45.7 / 37.2; N =
+    // 24576: M = 64 (384 blocks) 35.5 / 39.0, M = 96 (768) 56.8 / 41.4.
+    const int64_t blocks = (M + 63) / 64 * (n_total / 64);
+    if (blocks <= 2 * (int64_t)cus) {
+      // The narrowest strips that need no second round of workgroups; for a
+      // single block of rows, where the weights come from HBM once, three
+      // workgroups per CU hide each other's loads (N = 24576, M = 64: two
+      // panels 35.5, four 38.7 us; N = 6144, M = 64: one 13.0, two 10.3,
+      // four 13.8).  32 rows a block where that covers M: M = 32, N = 4096
+      // 8.3 us.
+      const bool narrow = M <= 32;
+      const int64_t row_blocks = narrow ? 1 : (M + 63) / 64;
+      const int64_t one = row_blocks * (n_total / 16);
+      const int panels = one <= cus ? 1 : one / 2 <= (row_blocks == 1 ? 3 : 1) * cus ? 2 : 4;
+      const dim3 grid((unsigned)(n_total / (16 * panels)), (unsigned)row_blocks);
+#define ECF8_ROWS(P, CH)                                                                    \
+  fp8_rows_kernel<P, CH><<<grid, 512, 0, as_stream(stream)>>>(a, as, (int)M, (int)K, s, o, \
+                                                              (int)ldo)
+      if (narrow) {
+        if (panels == 1) ECF8_ROWS(1, 2);
+        else if (panels == 2) ECF8_ROWS(2, 2);
+        else ECF8_ROWS(4, 2);
+      } else {
+        if (panels == 1) ECF8_ROWS(1, 4);
+        else if (panels == 2) ECF8_ROWS(2, 4);
+        else ECF8_ROWS(4, 4);
+      }
+#undef ECF8_ROWS
+      return launched();
+    }
     const int n_mb = (int)((M + kGemmBM - 1) / kGemmBM);
     const int64_t n_tiles = (n_total / kGemmBN) * n_mb;
     if (n_tiles > INT32_MAX) return ECF8_ERR_UNSUPPORTED;

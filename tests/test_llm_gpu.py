@@ -197,6 +197,38 @@ def test_fp8_linear_eight_wave_shape_matches_fp64(cuda_device, M):
     assert bool(((got - ref).abs() <= tol).all())
 
 
+@pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("M,shapes,Kd", [
+    (17, (128,), 128), (31, (128, 256, 128), 384), (32, (4096,), 1024), (32, (4096, 128), 1152),
+    (32, (12288, 384), 256), (33, (128,), 2176), (48, (4096, 256), 1024), (64, (128,), 12288),
+    (64, (12416,), 256), (65, (2048, 128), 1024), (127, (2048, 128, 128), 640), (129, (2048,), 896),
+    (700, (512, 128), 384), (2048, (1024,), 256), (2113, (1024,), 256), (2113, (128, 1024), 512)])
+def test_fp8_linear_many_rows_either_form(cuda_device, M, shapes, Kd, layout):
+    """Both forms above 16 rows, at the edges of their row blocks (32, 64,
+    256) and strips (16, 32 and 64 columns in one, two and four panels),
+    with fewer K groups than waves and uneven runs; the last two shapes are
+    past the 512 blocks of 64 x 64 that the middle form takes on 256 CUs."""
+    from ecf8_amd.llm_kernels import LinearPlan
+
+    gen = torch.Generator().manual_seed(M * 7 + Kd)
+    aq = _rand_fp8((M, Kd), gen, cuda_device)
+    a_s = (torch.rand(M, Kd // 128, generator=gen) * 1e-2 + 1e-4).to(cuda_device)
+    segs = [(_rand_fp8((n, Kd), gen, cuda_device),
+             (torch.rand(n // 128, Kd // 128, generator=gen) * 1e-3 + 1e-5).to(cuda_device))
+            for n in shapes]
+    N = sum(shapes)
+    out = torch.full((M + 1, N + 64), 7.0, dtype=torch.bfloat16, device=cuda_device)
+    LinearPlan([(to_tiles(w), ws, 1) if layout else (w, ws) for w, ws in segs], out)(
+        to_tiles(aq), a_s, M)
+    a = aq.double().view(M, Kd // 128, 128) * a_s.double()[:, :, None]
+    ref = torch.cat([a.view(M, Kd) @ (w.double().view(-1, 128, Kd // 128, 128)
+                                      * ws.double()[:, None, :, None]).view(-1, Kd).t()
+                     for w, ws in segs], 1)
+    tol = 2 ** -7 * ref.abs() + 1e-4 * ref.abs().max()  # bf16 output, as above
+    assert bool(((out[:M, :N].double() - ref).abs() <= tol).all())
+    assert bool((out[:, N:] == 7.0).all()) and bool((out[M:] == 7.0).all())
+
+
 def test_fp8_linear_persistent_path_matches_fp64(cuda_device):
     """More 16-column tiles than one workgroup per CU at K = 4096 (the
     gate/up shape) takes the persistent kernel that keeps the activations
