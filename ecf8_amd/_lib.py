@@ -94,6 +94,12 @@ _SIGNATURES = {
     "ecf8_dit_modulate": ([_vp, _i64, _i64, _i64, _vp, _i64, _vp, _i64, _f32, _vp, _vp], _i32),
     "ecf8_dit_gated_add": ([_vp, _vp, _i64, _vp, _i64, _i64, _i64, _vp, _vp], _i32),
     "ecf8_dit_gelu": ([_vp, _i64, _i64, _i64, _vp, _i64, _vp], _i32),
+    # include/ecf8_head.h: the ends of a decode step
+    "ecf8_bf16_linear16": ([_vp, _i64, _i64, _i64, _vp, _i64, _vp, _vp, _i64, _vp], _i32),
+    "ecf8_greedy_work_bytes": ([_i64], _i64),
+    "ecf8_greedy_emit": ([_vp, _i64, _i64, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _i32, _vp],
+                         _i32),
+    "ecf8_embed_rows": ([_vp, _i64, _vp, _i64, _i64, _vp, _vp], _i32),
 }
 
 EXPORTED = tuple(_SIGNATURES)

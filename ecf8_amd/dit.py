@@ -39,6 +39,8 @@ import torch.nn.functional as F
 
 from . import dit_kernels as DK
 from . import llm_kernels as K
+from .guards import bare
+from .head_kernels import small_linear
 from .llm import FP8Linear
 
 DOUBLE_REGEX = r"dit\.blocks\.\d+"
@@ -90,7 +92,7 @@ class _Lin(FP8Linear):
         w = self.__dict__.get("_w_bf16")
         if w is None:
             w = K.dequant_fp8_block(self.weight, self.weight_scale_inv)
-        return F.linear(x, w, self.bias)
+        return small_linear(x, w, self.bias)
 
 
 class _Norm(nn.Module):
@@ -129,6 +131,14 @@ def _rope(x, cos, sin):
     return out
 
 
+def _joint_attention(streams, heads, cos, sin, tail=None):
+    """dit_kernels.joint_attention, or None where it does not take the call
+    or a head norm is not a plain _Norm."""
+    if not all(bare(n, _Norm) for _, *pair in streams for n in pair):
+        return None
+    return DK.joint_attention(streams, heads, cos, sin, tail)
+
+
 def _attention(q, k, v, chunk: int = 1152):
     """Softmax attention of q, k, v [B, H, T, D] (fp32 in, fp32 out), chunked
     over queries, in the precision the reference's bf16 pipeline attends
@@ -156,7 +166,9 @@ class _AdaNorm(nn.Module):
         self.n = n
 
     def forward(self, emb):
-        return self.linear(F.silu(emb)).chunk(self.n, dim=-1)
+        x, lin = F.silu(emb), self.linear
+        y = small_linear(x, lin.weight, lin.bias) if bare(lin, nn.Linear) else lin(x)
+        return y.chunk(self.n, dim=-1)
 
 
 class _JointAttention(nn.Module):
@@ -189,8 +201,8 @@ class DoubleBlock(nn.Module):
         sa, ca, ga, sma, cma, gma = self.norm1_a(emb)
         sb, cb, gb, smb, cmb, gmb = self.norm1_b(emb)
         qkv_a, qkv_b = at.a_to_qkv(_modulate(img, sa, ca)), at.b_to_qkv(_modulate(txt, sb, cb))
-        o = DK.joint_attention([(qkv_b, at.norm_q_b, at.norm_k_b),
-                                (qkv_a, at.norm_q_a, at.norm_k_a)], at.heads, cos, sin)
+        o = _joint_attention([(qkv_b, at.norm_q_b, at.norm_k_b),
+                              (qkv_a, at.norm_q_a, at.norm_k_a)], at.heads, cos, sin)
         if o is None:
             qa, ka, va = _heads(qkv_a, at.heads * 3).chunk(3, dim=1)
             qb, kb, vb = _heads(qkv_b, at.heads * 3).chunk(3, dim=1)
@@ -227,8 +239,7 @@ class SingleBlock(nn.Module):
         shift, scale, gate = self.norm.linear(F.silu(emb)).chunk(3, dim=-1)
         y = self.to_qkv_mlp(_modulate(x, shift, scale))
         qkv, mlp = y[..., : 3 * self.hidden], y[..., 3 * self.hidden:]
-        o = DK.joint_attention([(qkv, self.norm_q_a, self.norm_k_a)], self.heads, cos, sin,
-                               tail=mlp)
+        o = _joint_attention([(qkv, self.norm_q_a, self.norm_k_a)], self.heads, cos, sin, tail=mlp)
         if o is None:
             q, k, v = _heads(qkv, self.heads * 3).chunk(3, dim=1)
             o = _attention(_rope(self.norm_q_a(q), cos, sin), _rope(self.norm_k_a(k), cos, sin),

@@ -14,36 +14,19 @@ import ctypes
 import math
 
 import torch
-from torch.autograd import forward_ad
 
 from ._lib import check, lib
+from .guards import takes as _takes
+from .guards import untracked as _untracked
 from .llm_kernels import packed_kv
 
 HEAD_DIM = 128
-_PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 
 class _Stream(ctypes.Structure):
     _fields_ = [("qkv", ctypes.c_void_p), ("q_norm", ctypes.c_void_p), ("k_norm", ctypes.c_void_p),
                 ("tokens", ctypes.c_int64), ("row_stride", ctypes.c_int64),
                 ("batch_stride", ctypes.c_int64)]
-
-
-def _untracked() -> bool:
-    """No tracer, dispatch mode, dual level or autocast region is active."""
-    return not (torch._C._len_torch_dispatch_stack() or forward_ad._current_level >= 0
-                or torch.is_autocast_enabled("cuda") or torch.jit.is_tracing()
-                or torch.compiler.is_compiling())
-
-
-def _takes(tensors, dtype=torch.bfloat16) -> bool:
-    """Plain, non-empty, 16-byte aligned CUDA tensors of one dtype on one
-    device that autograd does not follow."""
-    dev, grad = tensors[0].device, torch.is_grad_enabled()
-    return all(type(t) in _PLAIN and t.is_cuda and t.device == dev and t.dtype == dtype
-               and t.numel() > 0 and not (grad and t.requires_grad)
-               and not torch._C._functorch.is_functorch_wrapped_tensor(t)
-               and t.data_ptr() % 16 == 0 for t in tensors)
 
 
 def _vector(t, B, C) -> bool:
@@ -96,7 +79,7 @@ def joint_attention(streams, heads, cos, sin, tail=None):
     ``tail`` [B, T, m]: GELU (tanh) of it follows the heads in the result's
     columns."""
     norms = [n for _, *pair in streams for n in pair]
-    if any(n._forward_hooks or n._forward_pre_hooks for n in norms) or not _untracked():
+    if not _untracked():
         return None
     every = [s[0] for s in streams] + [n.weight for n in norms]
     if not _takes(every if tail is None else every + [tail]) or not _takes((cos, sin),

@@ -30,6 +30,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import llm_kernels as K
+from . import head_kernels as HK
 from . import tiled
 from ._lib import ECF8Error
 
@@ -234,7 +235,7 @@ class _GreedyRunner:
             x = layer(self, i, x, prefill)
         K.rmsnorm(self.res, self.model.model.norm.weight, cfg.eps, B * T, x=x, out_bf16=self.h)
         last = self.h[: B * T].view(B, T, cfg.hidden)[:, T - 1]
-        return F.linear(last, self.model.lm_head.weight)
+        return HK.small_linear(last, self.model.lm_head.weight)
 
     def prefill(self, prompt: torch.Tensor) -> torch.Tensor:
         """prompt int64 [B, T] -> logits of the last position; sets the
@@ -251,18 +252,29 @@ class _GreedyRunner:
         self.pos.fill_(T)
         return logits
 
-    def _emit(self, logits):
-        tok = logits.argmax(dim=-1)
-        self.tokens.index_copy_(1, self.step, tok.unsqueeze(1))
-        self.next_tok.copy_(tok)
-        self.step.add_(1)
+    def _emit(self, logits, advance: int = 0):
+        """The greedy token of each row -> next_tok and this step's column of
+        tokens; step += 1, pos += advance."""
+        if logits.dtype != torch.bfloat16 or self.B > 65535:  # a head in another dtype
+            tok = logits.argmax(dim=-1)
+            self.tokens.index_copy_(1, self.step, tok.unsqueeze(1))
+            self.next_tok.copy_(tok)
+            self.step.add_(1)
+            self.pos.add_(advance)
+            return
+        if not hasattr(self, "_greedy_work"):
+            self._greedy_work = HK.greedy_work(self.B, self.dev)
+        HK.greedy_emit(logits, self._greedy_work, self.tokens, self.next_tok, self.step, self.pos,
+                       advance)
 
     def _decode_body(self):
-        emb = F.embedding(self.next_tok, self.model.model.embed_tokens.weight)
-        self.res[: self.B].copy_(emb)
+        table = self.model.model.embed_tokens.weight
+        if table.dtype == torch.bfloat16 and self.B <= 65535:
+            HK.embed_rows(self.next_tok, table, self.res)
+        else:
+            self.res[: self.B].copy_(F.embedding(self.next_tok, table))
         logits = self._forward(False)
-        self._emit(logits)
-        self.pos.add_(1)
+        self._emit(logits, advance=1)
         return logits
 
     def decode_step(self) -> torch.Tensor:
