@@ -250,13 +250,6 @@ __device__ __forceinline__ void gemm_barrier() {
   asm volatile("" ::: "memory");
 }
 
-// Workgroup barrier that waits for LDS only (a __syncthreads would also
-// wait for the prefetched global loads).
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_s_waitcnt((0x3F & 15) | (0x3 << 14) | (0x7 << 4) | (0x0 << 8));  // lgkmcnt(0)
-  gemm_barrier();
-}
-
 // 16 bytes of LDS at byte offset `off` + the immediate O of a stage, read
 // by inline asm: the compiler cannot see that it reads LDS, so it does not
 // wait for the loads still filling the other stages (the caller waits for
@@ -926,40 +919,25 @@ __global__ __launch_bounds__(256) void act_quant_kernel(const uint16_t *__restri
 // One wave, one head row of 128 bf16 values (lane l holds dims 2l, 2l+1):
 // RMSNorm over the head (bf16 weights nw), then the rotary embedding at
 // position p (rotate-half convention, cos/sin tables [Lmax, 64]); returns
-// the lane's two results as packed bf16.  The loads are apart from the
-// arithmetic, so a kernel can issue them ahead of longer ones.
-struct RopeIn {
-  uint32_t w2;   // the norm's weights
-  float2 c, s;   // the rotary tables at p
-};
-
-__device__ __forceinline__ RopeIn rope_load(const uint16_t *__restrict__ nw,
-                                            const float *__restrict__ cosv,
-                                            const float *__restrict__ sinv, int p, int lane) {
-  const int j = (2 * lane) & 63;
-  return RopeIn{*reinterpret_cast<const uint32_t *>(nw + 2 * lane),
-                make_float2(cosv[p * 64 + j], cosv[p * 64 + j + 1]),
-                make_float2(sinv[p * 64 + j], sinv[p * 64 + j + 1])};
-}
-
-__device__ __forceinline__ uint32_t norm_rope(uint32_t x2, const RopeIn &in, float eps, int lane) {
-  float x0 = bf16_f32(x2 & 0xffffu), x1 = bf16_f32(x2 >> 16);
-  const float ss = wave_sum(x0 * x0 + x1 * x1);
-  const float rs = rsqrtf(ss / (float)kHeadDim + eps);
-  x0 = x0 * rs * bf16_f32(in.w2 & 0xffffu);
-  x1 = x1 * rs * bf16_f32(in.w2 >> 16);
-  const float y0 = __shfl_xor(x0, 32), y1 = __shfl_xor(x1, 32);  // dims d +- 64
-  const float sg = lane < 32 ? -1.f : 1.f;
-  x0 = x0 * in.c.x + sg * y0 * in.s.x;
-  x1 = x1 * in.c.y + sg * y1 * in.s.y;
-  return f32_bf16(x0) | (f32_bf16(x1) << 16);
-}
-
+// the lane's two results as packed bf16.
 __device__ __forceinline__ uint32_t norm_rope_pair(uint32_t x2, const uint16_t *__restrict__ nw,
                                                    float eps, const float *__restrict__ cosv,
                                                    const float *__restrict__ sinv, int p,
                                                    int lane) {
-  return norm_rope(x2, rope_load(nw, cosv, sinv, p, lane), eps, lane);
+  float x0 = bf16_f32(x2 & 0xffffu), x1 = bf16_f32(x2 >> 16);
+  const float ss = wave_sum(x0 * x0 + x1 * x1);
+  const float rs = rsqrtf(ss / (float)kHeadDim + eps);
+  const uint32_t w2 = *reinterpret_cast<const uint32_t *>(nw + 2 * lane);
+  x0 = x0 * rs * bf16_f32(w2 & 0xffffu);
+  x1 = x1 * rs * bf16_f32(w2 >> 16);
+  const float y0 = __shfl_xor(x0, 32), y1 = __shfl_xor(x1, 32);  // dims d +- 64
+  const int j = (2 * lane) & 63;
+  const float c0 = cosv[p * 64 + j], c1 = cosv[p * 64 + j + 1];
+  const float s0 = sinv[p * 64 + j], s1 = sinv[p * 64 + j + 1];
+  const float sg = lane < 32 ? -1.f : 1.f;
+  x0 = x0 * c0 + sg * y0 * s0;
+  x1 = x1 * c1 + sg * y1 * s1;
+  return f32_bf16(x0) | (f32_bf16(x1) << 16);
 }
 
 // One wave per (token, head) of the fused qkv projection output
@@ -998,6 +976,38 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(
 
 // ------------------------------------------------------ decode attention
 
+// Merge the splits [0, used) of one (b, head) (partials m, l [B*Hq, S] and
+// acc [B*Hq, S, 128]) and write the head's 128 outputs: quantized as one
+// o-projection group, and optionally as bf16.  One wave, two dims per lane.
+__device__ __forceinline__ void combine_head(const float *__restrict__ wm,
+                                             const float *__restrict__ wl,
+                                             const float *__restrict__ wacc, size_t bh, int S,
+                                             int used, int lane, int Hq,
+                                             uint8_t *__restrict__ oq, float *__restrict__ os,
+                                             uint16_t *__restrict__ ob) {
+  float mx = -INFINITY;
+  for (int s = 0; s < used; ++s) mx = fmaxf(mx, wm[bh * S + s]);
+  float l = 0.f, a0 = 0.f, a1 = 0.f;
+  for (int s = 0; s < used; ++s) {
+    const float f = expf(wm[bh * S + s] - mx);
+    l = fmaf(f, wl[bh * S + s], l);
+    const float *ap = wacc + (bh * S + s) * kHeadDim + 2 * lane;
+    a0 = fmaf(f, ap[0], a0);
+    a1 = fmaf(f, ap[1], a1);
+  }
+  a0 /= l;
+  a1 /= l;
+  if (ob) reinterpret_cast<uint32_t *>(ob)[bh * 64 + lane] = f32_bf16(a0) | (f32_bf16(a1) << 16);
+  float amax = wave_max(fmaxf(fabsf(a0), fabsf(a1)));
+  const float sc = amax > 0.f ? amax / kFp8Max : 1.f;
+  const uint32_t q2 = f32_e4m3(a0 / sc) | (f32_e4m3(a1 / sc) << 8);
+  // row b = bh / Hq, group = head: bytes 2 lane, 2 lane + 1 of the group
+  const int b = (int)(bh / (size_t)Hq), head = (int)(bh % (size_t)Hq);
+  *reinterpret_cast<uint16_t *>(oq + tile_chunk_off(b, head, Hq, lane >> 3) + 2 * (lane & 7)) =
+      (uint16_t)q2;
+  if (lane == 0) os[bh] = sc;
+}
+
 // What the fused form of the split kernel needs besides the caches.
 struct AttnFused {
   const uint16_t *qkv;  // [B, (Hq + 2 Hkv) * 128], one new token per sequence
@@ -1009,13 +1019,9 @@ struct AttnFused {
 // Split-sequence attention for one new token per sequence: workgroup
 // (b * Hkv + kh, split) handles positions [split*256, +256) of the L =
 // pos[0] + 1 cached ones for the G = Hq / Hkv query heads sharing kv head
-// kh, each of its eight waves 32 of them with a softmax of its own.  Scores
-// come from v_mfma_f32_16x16x32_bf16 (keys times heads, fp32), whose
-// operand loads read 64 contiguous bytes of each key row; PV runs in fp32
-// FMAs, 8 dims per lane.  A wave issues its 8 KB of keys and 8 KB of
-// values together, before q is prepared, so one round trip covers both.  The waves' partials meet
-// in LDS, and the workgroup's go to work: m, l [B*Hq, S] (m in units of the
-// unscaled scores) and acc [B*Hq, S, 128].
+// kh.  Scores: one lane per position; softmax partials per head; PV: one
+// thread per (head, dim pair).  Partials go to work: m, l [B*Hq, S] and
+// acc [B*Hq, S, 128].
 //
 // kFused: q comes from the projection output through the per-head norm and
 // rotary embedding (norm_rope_pair), and the split holding position pos[0]
@@ -1024,295 +1030,179 @@ struct AttnFused {
 // last workgroup to finish would need device-scope fences, which on this
 // multi-XCD part write back and invalidate the whole L2: the merge stays a
 // kernel of its own.)
-//
-// HBM-bound for long contexts, the latency of one workgroup for short ones;
-// MI355X, 16 sequences, with the merge (four waves of 64 positions, keys one
-// row per lane, before): G = 4, 8192 positions 142.9 -> 107.9 us (5.0 TB/s),
-// 640 19.7 -> 15.6; G = 8, 8192 100.5 -> 66.7.
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-constexpr float kScoreExp2 = 0.08838834764831845f * 1.4426950408889634f;  // log2(e) / sqrt(128)
-
-constexpr int kAttnWaves = 8;  // of 32 positions each
-
-// Rows (16 lanes) 0..3 of x and y -> rows x0 + x2, x1 + x3, y0 + y2, y1 + y3.
-__device__ __forceinline__ float add_swap32(float x, float y) {
-  const auto v = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false,
-                                                  false);
-  return __uint_as_float(v[0]) + __uint_as_float(v[1]);
-}
-// -> rows x0 + x1, y0 + y1, x2 + x3, y2 + y3.
-__device__ __forceinline__ float add_swap16(float x, float y) {
-  const auto v = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false,
-                                                  false);
-  return __uint_as_float(v[0]) + __uint_as_float(v[1]);
-}
-
 template <int G, bool kFused>
-__global__ __launch_bounds__(512) void attn_split_kernel(const uint16_t *__restrict__ q,
-                                                            uint16_t *__restrict__ kc,
-                                                            uint16_t *__restrict__ vc,
-                                                            const int *__restrict__ pos, int Hkv,
-                                                            int Lmax, int S, float *__restrict__ wm,
-                                                            float *__restrict__ wl,
-                                                            float *__restrict__ wacc,
-                                                            AttnFused fu) {
-  // the heads' q rows, then (fused) the new token's k and v rows: bf16 pairs
-  __shared__ __attribute__((aligned(16))) uint32_t qs[G + 2][kHeadDim / 2];
-  __shared__ __attribute__((aligned(16))) float pw[kAttnWaves][G][32];
-  __shared__ float part[kAttnWaves][G][kHeadDim];  // PV partials of each wave
-  __shared__ float s_m[kAttnWaves][G], s_l[kAttnWaves][G];
+__global__ __launch_bounds__(256) void attn_split_kernel(const uint16_t *__restrict__ q,
+                                                         uint16_t *__restrict__ kc,
+                                                         uint16_t *__restrict__ vc,
+                                                         const int *__restrict__ pos, int Hkv,
+                                                         int Lmax, int S, float *__restrict__ wm,
+                                                         float *__restrict__ wl,
+                                                         float *__restrict__ wacc, AttnFused fu) {
+  __shared__ float qs[G][kHeadDim];
+  __shared__ float pw[G][kAttnChunk];
+  __shared__ float part[4 * G * kHeadDim];  // PV partials [wave][head][dim]
+  __shared__ float red[G][4];
   const int bk = blockIdx.x, split = blockIdx.y;
   const int b = bk / Hkv, kh = bk % Hkv;
   const int Hq = Hkv * G;
-  const int t = threadIdx.x, lane = t & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int p = pos[0];
   int L = p + 1;
   L = L < 1 ? 1 : (L > Lmax ? Lmax : L);
   const int c0 = split * kAttnChunk;
   const size_t head0 = (size_t)b * Hq + kh * G;
-  if (c0 >= L) return;  // the merge reads the splits in use only
-  const int n = min(kAttnChunk, L - c0);
-  // fused: the new token's position in this chunk, whose cache row is
-  // written here and taken from LDS; past every position otherwise
-  const int fresh = kFused && p >= c0 && p < c0 + kAttnChunk && p < Lmax ? p - c0 : kAttnChunk;
-
-  const int r = lane & 15, g = lane >> 4;
-  const int w0 = 32 * wave;  // the wave's first position in the chunk
-  // The wave's head of q and the new token's k or v (the waves past the
-  // heads, or the first two): loaded first, since loads return in order and
-  // the keys take longest.
-  constexpr int kNew = G < 8 ? 4 : 0;  // wave kNew: k, wave kNew + 1: v
-  RopeIn qin, nin;
-  uint32_t qx = 0, nx = 0;
-  if constexpr (kFused) {
-    const uint16_t *row = fu.qkv + (size_t)b * (Hq + 2 * Hkv) * kHeadDim + 2 * lane;
-    qin = rope_load(fu.qn, fu.cosv, fu.sinv, min(max(p, 0), Lmax - 1), lane);
-    nin = qin;
-    nin.w2 = *reinterpret_cast<const uint32_t *>(fu.kn + 2 * lane);
-    if (wave < G) qx = *reinterpret_cast<const uint32_t *>(row + (size_t)(kh * G + wave) * kHeadDim);
-    if (wave == kNew || wave == kNew + 1)
-      nx = *reinterpret_cast<const uint32_t *>(row +
-                                               (size_t)(Hq + (wave - kNew) * Hkv + kh) * kHeadDim);
-  }
-  // keys: position 16 tt + r, dims 32 kk + 8 g (lane's A operand); values:
-  // positions 8 g + st, dims 8 r; positions past n read row n - 1.  In
-  // flight while q is prepared.
-  v8bf kf[2][4];
-  u32x4 vv[8];
-  if (w0 < n) {
-    const uint16_t *kbase = kc + (((size_t)b * Hkv + kh) * Lmax + c0) * kHeadDim + 8 * g;
-    const uint16_t *vbase = vc + (((size_t)b * Hkv + kh) * Lmax + c0) * kHeadDim + 8 * r;
-#pragma unroll
-    for (int tt = 0; tt < 2; ++tt) {
-      const uint16_t *kr = kbase + (size_t)min(w0 + 16 * tt + r, n - 1) * kHeadDim;
-#pragma unroll
-      for (int kk = 0; kk < 4; ++kk) kf[tt][kk] = *reinterpret_cast<const v8bf *>(kr + 32 * kk);
+  if (c0 >= L) {
+    if (t < G) {
+      wm[(head0 + t) * S + split] = -INFINITY;
+      wl[(head0 + t) * S + split] = 0.f;
     }
-#pragma unroll
-    for (int st = 0; st < 8; ++st)
-      vv[st] = *reinterpret_cast<const u32x4 *>(
-          vbase + (size_t)min(w0 + 8 * g + st, n - 1) * kHeadDim);
+    return;
   }
+  const int n = min(kAttnChunk, L - c0);
+  const float scale = rsqrtf((float)kHeadDim);
   if constexpr (kFused) {
-    if (wave < G) qs[wave][lane] = norm_rope(qx, qin, fu.eps, lane);
-    if (fresh < kAttnChunk && (wave == kNew || wave == kNew + 1)) {
-      const uint32_t y2 = wave == kNew ? norm_rope(nx, nin, fu.eps, lane) : nx;
-      uint16_t *cache = wave == kNew ? kc : vc;
+    const uint16_t *row = fu.qkv + (size_t)b * (Hq + 2 * Hkv) * kHeadDim;
+    const int pc = min(max(p, 0), Lmax - 1);  // rotary row (p is in range for a valid call)
+    for (int h = wave; h < G; h += 4) {
+      const uint32_t x2 =
+          *reinterpret_cast<const uint32_t *>(row + (kh * G + h) * kHeadDim + 2 * lane);
+      const uint32_t y2 = norm_rope_pair(x2, fu.qn, fu.eps, fu.cosv, fu.sinv, pc, lane);
+      qs[h][2 * lane] = bf16_f32(y2 & 0xffffu) * scale;
+      qs[h][2 * lane + 1] = bf16_f32(y2 >> 16) * scale;
+    }
+    if (p >= c0 && p < c0 + kAttnChunk && p < Lmax && wave < 2) {
+      // the new token's k (wave 0) and v (wave 1) go to the caches first
+      const int hh = Hq + wave * Hkv + kh;
+      const uint32_t x2 = *reinterpret_cast<const uint32_t *>(row + hh * kHeadDim + 2 * lane);
+      const uint32_t y2 = wave == 0 ? norm_rope_pair(x2, fu.kn, fu.eps, fu.cosv, fu.sinv, p, lane)
+                                    : x2;
+      uint16_t *cache = wave == 0 ? kc : vc;
       *reinterpret_cast<uint32_t *>(cache + (((size_t)b * Hkv + kh) * Lmax + p) * kHeadDim +
                                     2 * lane) = y2;
-      qs[G + wave - kNew][lane] = y2;
     }
+    __threadfence_block();  // the row is read back below by other waves
   } else {
-    for (int i = t; i < G * (kHeadDim / 2); i += 512)
-      qs[i / 64][i % 64] =
-          reinterpret_cast<const uint32_t *>(q + head0 * kHeadDim)[i];
+    for (int i = t; i < G * kHeadDim; i += 256) {
+      qs[i / kHeadDim][i % kHeadDim] =
+          bf16_f32(q[(head0 + i / kHeadDim) * kHeadDim + i % kHeadDim]) * scale;
+    }
   }
-  lds_barrier();
+  __syncthreads();
 
-  if (w0 < n) {
-    if (kFused && fresh < w0 + 32) {  // uniform
-      // the fresh row, also for the positions past it (their loads found
-      // the row as it was before)
+  const int j = 64 * wave + lane;  // position within the chunk
+  float s[G];
 #pragma unroll
-      for (int tt = 0; tt < 2; ++tt)
+  for (int h = 0; h < G; ++h) s[h] = 0.f;
+  const bool valid = j < n;
+  if (valid) {
+    // the whole 256-byte key row in flight at once
+    const uint4 *kr = reinterpret_cast<const uint4 *>(kc + (((size_t)b * Hkv + kh) * Lmax + c0 + j) * kHeadDim);
+    uint4 kv[kHeadDim / 8];
 #pragma unroll
-        for (int kk = 0; kk < 4; ++kk)
-          if (w0 + 16 * tt + r >= fresh)
-            kf[tt][kk] = *reinterpret_cast<const v8bf *>(&qs[G][16 * kk + 4 * g]);
+    for (int c = 0; c < kHeadDim / 8; ++c) kv[c] = kr[c];
 #pragma unroll
-      for (int st = 0; st < 8; ++st)
-        if (w0 + 8 * g + st >= fresh)
-          vv[st] = *reinterpret_cast<const u32x4 *>(&qs[G + 1][4 * r]);
-    }
-    v4f s[2];
+    for (int c = 0; c < kHeadDim / 8; ++c) {
+      const uint32_t wds[4] = {kv[c].x, kv[c].y, kv[c].z, kv[c].w};
 #pragma unroll
-    for (int tt = 0; tt < 2; ++tt) s[tt] = v4f{0.f, 0.f, 0.f, 0.f};
+      for (int e = 0; e < 4; ++e) {
+        const float k0 = bf16_f32(wds[e] & 0xffffu), k1 = bf16_f32(wds[e] >> 16);
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-      // heads past G repeat head r mod G; their columns are not used
-      const v8bf qf = *reinterpret_cast<const v8bf *>(&qs[r % G][16 * kk + 4 * g]);
-#pragma unroll
-      for (int tt = 0; tt < 2; ++tt)
-        s[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[tt][kk], qf, s[tt], 0, 0, 0);
-    }
-    // lane: head r, positions 16 tt + 4 g + i of the wave's 32
-    float mx = -INFINITY;
-#pragma unroll
-    for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if (w0 + 16 * tt + 4 * g + i >= n) s[tt][i] = -INFINITY;
-        mx = fmaxf(mx, s[tt][i]);
-      }
-    mx = fmaxf(mx, __shfl_xor(mx, 16));
-    mx = fmaxf(mx, __shfl_xor(mx, 32));
-    float sum = 0.f;
-#pragma unroll
-    for (int tt = 0; tt < 2; ++tt) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        s[tt][i] = __builtin_amdgcn_exp2f((s[tt][i] - mx) * kScoreExp2);
-        sum += s[tt][i];
-      }
-      if (r < G) *reinterpret_cast<v4f *>(&pw[wave][r][16 * tt + 4 * g]) = s[tt];
-    }
-    sum += __shfl_xor(sum, 16);
-    sum += __shfl_xor(sum, 32);
-    if (lane < G) {
-      s_m[wave][lane] = mx;
-      s_l[wave][lane] = sum;
-    }
-    // the wave's own rows of pw: LDS serves one wave in program order
-    __builtin_amdgcn_wave_barrier();
-    float acc[G][8];
-#pragma unroll
-    for (int h = 0; h < G; ++h)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) acc[h][e] = 0.f;
-#pragma unroll
-    for (int s4 = 0; s4 < 2; ++s4) {
-      v4f pv[G];
-#pragma unroll
-      for (int h = 0; h < G; ++h)
-        pv[h] = *reinterpret_cast<const v4f *>(&pw[wave][h][8 * g + 4 * s4]);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const u32x4 wds = vv[4 * s4 + j];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float v0 = bf16_f32(wds[e] & 0xffffu), v1 = __uint_as_float(wds[e] & 0xffff0000u);
-#pragma unroll
-          for (int h = 0; h < G; ++h) {
-            acc[h][2 * e] = fmaf(pv[h][j], v0, acc[h][2 * e]);
-            acc[h][2 * e + 1] = fmaf(pv[h][j], v1, acc[h][2 * e + 1]);
-          }
+        for (int h = 0; h < G; ++h) {
+          s[h] = fmaf(qs[h][8 * c + 2 * e], k0, s[h]);
+          s[h] = fmaf(qs[h][8 * c + 2 * e + 1], k1, s[h]);
         }
       }
     }
-    // the four lane rows' sums: four accumulators at a time, after which
-    // lane row g holds the total of the g-th
+  }
+  float mh[G];
+#pragma unroll
+  for (int h = 0; h < G; ++h) {
+    const float mw = wave_max(valid ? s[h] : -INFINITY);
+    if (lane == 0) red[h][wave] = mw;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int h = 0; h < G; ++h) mh[h] = fmaxf(fmaxf(red[h][0], red[h][1]), fmaxf(red[h][2], red[h][3]));
+  __syncthreads();
+#pragma unroll
+  for (int h = 0; h < G; ++h) {
+    const float e = valid ? expf(s[h] - mh[h]) : 0.f;
+    pw[h][j] = e;
+    const float sw = wave_sum(e);
+    if (lane == 0) red[h][wave] = sw;
+  }
+  __syncthreads();
+  if (t < G) {
+    wm[(head0 + t) * S + split] = mh[t];
+    wl[(head0 + t) * S + split] = (red[t][0] + red[t][1]) + (red[t][2] + red[t][3]);
+  }
+  // PV: wave w takes positions [64w, 64w + 64) of the chunk, four rows per
+  // step (lane / 16), eight dims per lane (16-byte loads), all 16 row loads
+  // in flight; positions past n read row n - 1 with weight 0.
+  const int dg = lane & 15, rr = lane >> 4;
+  const uint16_t *vbase = vc + (((size_t)b * Hkv + kh) * Lmax + c0) * kHeadDim + 8 * dg;
+  uint4 vv[16];
+#pragma unroll
+  for (int st = 0; st < 16; ++st) {
+    const int jj = min(64 * wave + 4 * st + rr, n - 1);
+    vv[st] = *reinterpret_cast<const uint4 *>(vbase + (size_t)jj * kHeadDim);
+  }
+  float acc[G][8];
+#pragma unroll
+  for (int h = 0; h < G; ++h)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[h][e] = 0.f;
+#pragma unroll
+  for (int st = 0; st < 16; ++st) {
+    const int jp = 64 * wave + 4 * st + rr;
+    const uint32_t wds[4] = {vv[st].x, vv[st].y, vv[st].z, vv[st].w};
+#pragma unroll
+    for (int h = 0; h < G; ++h) {
+      const float p = pw[h][jp];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        acc[h][2 * e] = fmaf(p, bf16_f32(wds[e] & 0xffffu), acc[h][2 * e]);
+        acc[h][2 * e + 1] = fmaf(p, bf16_f32(wds[e] >> 16), acc[h][2 * e + 1]);
+      }
+    }
+  }
+#pragma unroll
+  for (int h = 0; h < G; ++h)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      float v = acc[h][e];
+      v += __shfl_xor(v, 16);
+      v += __shfl_xor(v, 32);
+      acc[h][e] = v;
+    }
+  if (rr == 0) {
 #pragma unroll
     for (int h = 0; h < G; ++h)
 #pragma unroll
-      for (int e = 0; e < 8; e += 4)
-        part[wave][h][8 * r + e + g] =
-            add_swap16(add_swap32(acc[h][e], acc[h][e + 2]),
-                       add_swap32(acc[h][e + 1], acc[h][e + 3]));
-  } else if (lane < G) {
-    s_m[wave][lane] = -INFINITY;
-    s_l[wave][lane] = 0.f;
+      for (int e = 0; e < 8; ++e) part[(wave * G + h) * kHeadDim + 8 * dg + e] = acc[h][e];
   }
   __syncthreads();
-  const int waves = (n + 31) >> 5;  // waves with positions
-  for (int v = t; v < G * kHeadDim; v += 512) {
+  for (int v = t; v < G * kHeadDim; v += 256) {
     const int h = v / kHeadDim, d = v % kHeadDim;
-    float mx = -INFINITY;
-#pragma unroll
-    for (int w = 0; w < kAttnWaves; ++w) mx = fmaxf(mx, s_m[w][h]);
-    float sum = 0.f, l = 0.f;
-#pragma unroll
-    for (int w = 0; w < kAttnWaves; ++w) {
-      if (w < waves) {
-        const float f = __builtin_amdgcn_exp2f((s_m[w][h] - mx) * kScoreExp2);
-        l = fmaf(f, s_l[w][h], l);
-        sum = fmaf(f, part[w][h][d], sum);
-      }
-    }
+    const float sum = (part[(0 * G + h) * kHeadDim + d] + part[(1 * G + h) * kHeadDim + d]) +
+                      (part[(2 * G + h) * kHeadDim + d] + part[(3 * G + h) * kHeadDim + d]);
     wacc[((head0 + h) * S + split) * kHeadDim + d] = sum;
-    if (d == 0) {
-      wm[(head0 + h) * S + split] = mx;
-      wl[(head0 + h) * S + split] = l;
-    }
   }
 }
 
-// Merge the splits of one (b, head) -- partials m, l [B*Hq, S] and acc
-// [B*Hq, S, 128] -- and write its 128 outputs: quantized as one o-projection
-// group, and optionally as bf16.  Four waves take every fourth split each
-// (two dims per lane, eight splits' loads in flight) and add up in wave
-// order.  Latency-bound: one wave walking 33 splits one by one took 15.9 us
-// for 16 x 32 heads, this 5.7.
-__global__ __launch_bounds__(256) void attn_combine_kernel(const float *__restrict__ wm,
-                                                           const float *__restrict__ wl,
-                                                           const float *__restrict__ wacc,
-                                                           const int *__restrict__ pos, int Lmax,
-                                                           int S, int Hq, uint8_t *__restrict__ oq,
-                                                           float *__restrict__ os,
-                                                           uint16_t *__restrict__ ob) {
-  __shared__ float s_part[4][3][64];
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+// Merge the splits of one (b, head) and quantize the head's 128 outputs
+// (one activation group of the o projection); optionally also write bf16.
+__global__ __launch_bounds__(64) void attn_combine_kernel(const float *__restrict__ wm,
+                                                          const float *__restrict__ wl,
+                                                          const float *__restrict__ wacc,
+                                                          const int *__restrict__ pos, int Lmax,
+                                                          int S, int Hq, uint8_t *__restrict__ oq,
+                                                          float *__restrict__ os,
+                                                          uint16_t *__restrict__ ob) {
   int L = pos[0] + 1;
   L = L < 1 ? 1 : (L > Lmax ? Lmax : L);
   const int used = (L + kAttnChunk - 1) / kAttnChunk;
-  const size_t bh = blockIdx.x;
-  const float *pm = wm + bh * S, *pl = wl + bh * S;
-  const float2 *pa = reinterpret_cast<const float2 *>(wacc + bh * S * kHeadDim) + lane;
-  float mx = -INFINITY;
-  for (int s = lane; s < used; s += 64) mx = fmaxf(mx, pm[s]);
-  mx = wave_max_dpp(mx);
-  float l = 0.f, a0 = 0.f, a1 = 0.f;
-  constexpr int kU = 8;
-  for (int s0 = wave; s0 < used; s0 += 4 * kU) {
-    float2 a[kU];
-    float f[kU], ls[kU];
-#pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      const int s = min(s0 + 4 * u, used - 1);
-      a[u] = pa[(size_t)s * 64];
-      f[u] = pm[s];
-      ls[u] = pl[s];
-    }
-#pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      if (s0 + 4 * u < used) {  // uniform
-        const float e = __builtin_amdgcn_exp2f((f[u] - mx) * kScoreExp2);
-        l = fmaf(e, ls[u], l);
-        a0 = fmaf(e, a[u].x, a0);
-        a1 = fmaf(e, a[u].y, a1);
-      }
-    }
-  }
-  s_part[wave][0][lane] = l;
-  s_part[wave][1][lane] = a0;
-  s_part[wave][2][lane] = a1;
-  __syncthreads();
-  if (wave) return;
-  l = (s_part[0][0][lane] + s_part[1][0][lane]) + (s_part[2][0][lane] + s_part[3][0][lane]);
-  a0 = (s_part[0][1][lane] + s_part[1][1][lane]) + (s_part[2][1][lane] + s_part[3][1][lane]);
-  a1 = (s_part[0][2][lane] + s_part[1][2][lane]) + (s_part[2][2][lane] + s_part[3][2][lane]);
-  a0 /= l;
-  a1 /= l;
-  if (ob) reinterpret_cast<uint32_t *>(ob)[bh * 64 + lane] = f32_bf16(a0) | (f32_bf16(a1) << 16);
-  const float amax = wave_max_dpp(fmaxf(fabsf(a0), fabsf(a1)));
-  const float sc = amax > 0.f ? amax / kFp8Max : 1.f;
-  const uint32_t q2 = f32_e4m3(a0 / sc) | (f32_e4m3(a1 / sc) << 8);
-  // row b = bh / Hq, group = head: bytes 2 lane, 2 lane + 1 of the group
-  const int b = (int)(bh / (size_t)Hq), head = (int)(bh % (size_t)Hq);
-  *reinterpret_cast<uint16_t *>(oq + tile_chunk_off(b, head, Hq, lane >> 3) + 2 * (lane & 7)) =
-      (uint16_t)q2;
-  if (lane == 0) os[bh] = sc;
+  combine_head(wm, wl, wacc, blockIdx.x, S, used, threadIdx.x, Hq, oq, os, ob);
 }
 
 // ---------------------------------------------------- FP8 block dequantize
@@ -1701,6 +1591,13 @@ __global__ __launch_bounds__(WAVES * 64) void moe_linear16_kernel(MoeLinear a) {
   }
 }
 
+// Workgroup barrier that waits for LDS only (a __syncthreads would also
+// wait for the prefetched global loads).
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_s_waitcnt((0x3F & 15) | (0x3 << 14) | (0x7 << 4) | (0x0 << 8));  // lgkmcnt(0)
+  gemm_barrier();
+}
+
 // The same grouped linear for many rows per expert (a prompt): workgroup
 // (strip, slot) of eight waves computes a 128-column strip of expert
 // active[slot], wave w its columns [16 w, +16), for 16 kChunks rows at a
@@ -2078,12 +1975,12 @@ extern "C" int ecf8_decode_attention(const void *q, const void *k_cache, const v
   auto *vp = static_cast<uint16_t *>(const_cast<void *>(v_cache));
   const AttnFused none{};
   if (Hq == 4 * Hkv)
-    attn_split_kernel<4, false><<<grid, 64 * kAttnWaves, 0, as_stream(stream)>>>(
+    attn_split_kernel<4, false><<<grid, 256, 0, as_stream(stream)>>>(
         qp, kp, vp, pos, Hkv, (int)Lmax, (int)S, wm, wl, wacc, none);
   else
-    attn_split_kernel<8, false><<<grid, 64 * kAttnWaves, 0, as_stream(stream)>>>(
+    attn_split_kernel<8, false><<<grid, 256, 0, as_stream(stream)>>>(
         qp, kp, vp, pos, Hkv, (int)Lmax, (int)S, wm, wl, wacc, none);
-  attn_combine_kernel<<<(unsigned)(B * Hq), 256, 0, as_stream(stream)>>>(
+  attn_combine_kernel<<<(unsigned)(B * Hq), 64, 0, as_stream(stream)>>>(
       wm, wl, wacc, pos, (int)Lmax, (int)S, Hq, static_cast<uint8_t *>(out_q), out_scale,
       static_cast<uint16_t *>(out_bf16));
   return launched();
@@ -2113,12 +2010,12 @@ extern "C" int ecf8_decode_attention_fused(const void *qkv, int64_t B, int Hq, i
   auto *kp = static_cast<uint16_t *>(k_cache);
   auto *vp = static_cast<uint16_t *>(v_cache);
   if (Hq == 4 * Hkv)
-    attn_split_kernel<4, true><<<grid, 64 * kAttnWaves, 0, as_stream(stream)>>>(
+    attn_split_kernel<4, true><<<grid, 256, 0, as_stream(stream)>>>(
         nullptr, kp, vp, pos, Hkv, (int)Lmax, (int)S, wm, wl, wacc, fu);
   else
-    attn_split_kernel<8, true><<<grid, 64 * kAttnWaves, 0, as_stream(stream)>>>(
+    attn_split_kernel<8, true><<<grid, 256, 0, as_stream(stream)>>>(
         nullptr, kp, vp, pos, Hkv, (int)Lmax, (int)S, wm, wl, wacc, fu);
-  attn_combine_kernel<<<(unsigned)(B * Hq), 256, 0, as_stream(stream)>>>(
+  attn_combine_kernel<<<(unsigned)(B * Hq), 64, 0, as_stream(stream)>>>(
       wm, wl, wacc, pos, (int)Lmax, (int)S, Hq, static_cast<uint8_t *>(out_q), out_scale,
       static_cast<uint16_t *>(out_bf16));
   return launched();
