@@ -31,6 +31,7 @@ constexpr int kAttnChunk = 256;      // positions per attention workgroup
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 // Tile layout of FP8 operands (activations always, weights optionally; see
 // ecf8_llm.h): per 16 rows and 128-column group one 2 KB block in the
@@ -248,6 +249,13 @@ __device__ __forceinline__ void gemm_barrier() {
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
+}
+
+// Workgroup barrier that waits for LDS only (a __syncthreads would also
+// wait for the prefetched global loads).
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_s_waitcnt((0x3F & 15) | (0x3 << 14) | (0x7 << 4) | (0x0 << 8));  // lgkmcnt(0)
+  gemm_barrier();
 }
 
 // 16 bytes of LDS at byte offset `off` + the immediate O of a stage, read
@@ -919,25 +927,40 @@ __global__ __launch_bounds__(256) void act_quant_kernel(const uint16_t *__restri
 // One wave, one head row of 128 bf16 values (lane l holds dims 2l, 2l+1):
 // RMSNorm over the head (bf16 weights nw), then the rotary embedding at
 // position p (rotate-half convention, cos/sin tables [Lmax, 64]); returns
-// the lane's two results as packed bf16.
+// the lane's two results as packed bf16.  The loads are apart from the
+// arithmetic, so a kernel can issue them ahead of longer ones.
+struct RopeIn {
+  uint32_t w2;   // the norm's weights
+  float2 c, s;   // the rotary tables at p
+};
+
+__device__ __forceinline__ RopeIn rope_load(const uint16_t *__restrict__ nw,
+                                            const float *__restrict__ cosv,
+                                            const float *__restrict__ sinv, int p, int lane) {
+  const int j = (2 * lane) & 63;
+  return RopeIn{*reinterpret_cast<const uint32_t *>(nw + 2 * lane),
+                make_float2(cosv[p * 64 + j], cosv[p * 64 + j + 1]),
+                make_float2(sinv[p * 64 + j], sinv[p * 64 + j + 1])};
+}
+
+__device__ __forceinline__ uint32_t norm_rope(uint32_t x2, const RopeIn &in, float eps, int lane) {
+  float x0 = bf16_f32(x2 & 0xffffu), x1 = bf16_f32(x2 >> 16);
+  const float ss = wave_sum(x0 * x0 + x1 * x1);
+  const float rs = rsqrtf(ss / (float)kHeadDim + eps);
+  x0 = x0 * rs * bf16_f32(in.w2 & 0xffffu);
+  x1 = x1 * rs * bf16_f32(in.w2 >> 16);
+  const float y0 = __shfl_xor(x0, 32), y1 = __shfl_xor(x1, 32);  // dims d +- 64
+  const float sg = lane < 32 ? -1.f : 1.f;
+  x0 = x0 * in.c.x + sg * y0 * in.s.x;
+  x1 = x1 * in.c.y + sg * y1 * in.s.y;
+  return f32_bf16(x0) | (f32_bf16(x1) << 16);
+}
+
 __device__ __forceinline__ uint32_t norm_rope_pair(uint32_t x2, const uint16_t *__restrict__ nw,
                                                    float eps, const float *__restrict__ cosv,
                                                    const float *__restrict__ sinv, int p,
                                                    int lane) {
-  float x0 = bf16_f32(x2 & 0xffffu), x1 = bf16_f32(x2 >> 16);
-  const float ss = wave_sum(x0 * x0 + x1 * x1);
-  const float rs = rsqrtf(ss / (float)kHeadDim + eps);
-  const uint32_t w2 = *reinterpret_cast<const uint32_t *>(nw + 2 * lane);
-  x0 = x0 * rs * bf16_f32(w2 & 0xffffu);
-  x1 = x1 * rs * bf16_f32(w2 >> 16);
-  const float y0 = __shfl_xor(x0, 32), y1 = __shfl_xor(x1, 32);  // dims d +- 64
-  const int j = (2 * lane) & 63;
-  const float c0 = cosv[p * 64 + j], c1 = cosv[p * 64 + j + 1];
-  const float s0 = sinv[p * 64 + j], s1 = sinv[p * 64 + j + 1];
-  const float sg = lane < 32 ? -1.f : 1.f;
-  x0 = x0 * c0 + sg * y0 * s0;
-  x1 = x1 * c1 + sg * y1 * s1;
-  return f32_bf16(x0) | (f32_bf16(x1) << 16);
+  return norm_rope(x2, rope_load(nw, cosv, sinv, p, lane), eps, lane);
 }
 
 // One wave per (token, head) of the fused qkv projection output
@@ -976,38 +999,6 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(
 
 // ------------------------------------------------------ decode attention
 
-// Merge the splits [0, used) of one (b, head) (partials m, l [B*Hq, S] and
-// acc [B*Hq, S, 128]) and write the head's 128 outputs: quantized as one
-// o-projection group, and optionally as bf16.  One wave, two dims per lane.
-__device__ __forceinline__ void combine_head(const float *__restrict__ wm,
-                                             const float *__restrict__ wl,
-                                             const float *__restrict__ wacc, size_t bh, int S,
-                                             int used, int lane, int Hq,
-                                             uint8_t *__restrict__ oq, float *__restrict__ os,
-                                             uint16_t *__restrict__ ob) {
-  float mx = -INFINITY;
-  for (int s = 0; s < used; ++s) mx = fmaxf(mx, wm[bh * S + s]);
-  float l = 0.f, a0 = 0.f, a1 = 0.f;
-  for (int s = 0; s < used; ++s) {
-    const float f = expf(wm[bh * S + s] - mx);
-    l = fmaf(f, wl[bh * S + s], l);
-    const float *ap = wacc + (bh * S + s) * kHeadDim + 2 * lane;
-    a0 = fmaf(f, ap[0], a0);
-    a1 = fmaf(f, ap[1], a1);
-  }
-  a0 /= l;
-  a1 /= l;
-  if (ob) reinterpret_cast<uint32_t *>(ob)[bh * 64 + lane] = f32_bf16(a0) | (f32_bf16(a1) << 16);
-  float amax = wave_max(fmaxf(fabsf(a0), fabsf(a1)));
-  const float sc = amax > 0.f ? amax / kFp8Max : 1.f;
-  const uint32_t q2 = f32_e4m3(a0 / sc) | (f32_e4m3(a1 / sc) << 8);
-  // row b = bh / Hq, group = head: bytes 2 lane, 2 lane + 1 of the group
-  const int b = (int)(bh / (size_t)Hq), head = (int)(bh % (size_t)Hq);
-  *reinterpret_cast<uint16_t *>(oq + tile_chunk_off(b, head, Hq, lane >> 3) + 2 * (lane & 7)) =
-      (uint16_t)q2;
-  if (lane == 0) os[bh] = sc;
-}
-
 // What the fused form of the split kernel needs besides the caches.
 struct AttnFused {
   const uint16_t *qkv;  // [B, (Hq + 2 Hkv) * 128], one new token per sequence
@@ -1016,182 +1007,272 @@ struct AttnFused {
   const float *cosv, *sinv;
 };
 
+// Sum over the wave in the association of wave_sum (lane 0's: halves, then
+// 16, 8, 4, 2, 1 lanes apart), in every lane, without LDS shuffles: after
+// each step the values repeat with half the period, so a row rotation
+// brings the same partner as an exclusive-or.
+__device__ __forceinline__ float wave_sum_dpp(float v) {
+  auto swap = [](uint32_t a, bool half) {
+    const auto u = half ? __builtin_amdgcn_permlane32_swap(a, a, false, false)
+                        : __builtin_amdgcn_permlane16_swap(a, a, false, false);
+    return __uint_as_float(u[0]) + __uint_as_float(u[1]);
+  };
+  v = swap(__float_as_uint(v), true);
+  v = swap(__float_as_uint(v), false);
+#define ECF8_DPP_ADD(ctrl)                                                                 \
+  v += __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), ctrl, \
+                                                             0xF, 0xF, true))
+  ECF8_DPP_ADD(0x128);  // row_ror:8
+  ECF8_DPP_ADD(0x124);  // row_ror:4
+  ECF8_DPP_ADD(0x4E);   // quad_perm 2, 3, 0, 1
+  ECF8_DPP_ADD(0xB1);   // quad_perm 1, 0, 3, 2
+#undef ECF8_DPP_ADD
+  return v;
+}
+
+// Rows (16 lanes) 0..3 of x and y -> rows x0 + x1, y0 + y1, x2 + x3, y2 + y3.
+__device__ __forceinline__ float add_swap16(float x, float y) {
+  const auto v = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false,
+                                                  false);
+  return __uint_as_float(v[0]) + __uint_as_float(v[1]);
+}
+// -> rows x0 + x2, x1 + x3, y0 + y2, y1 + y3.
+__device__ __forceinline__ float add_swap32(float x, float y) {
+  const auto v = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false,
+                                                  false);
+  return __uint_as_float(v[0]) + __uint_as_float(v[1]);
+}
+
 // Split-sequence attention for one new token per sequence: workgroup
 // (b * Hkv + kh, split) handles positions [split*256, +256) of the L =
 // pos[0] + 1 cached ones for the G = Hq / Hkv query heads sharing kv head
-// kh.  Scores: one lane per position; softmax partials per head; PV: one
-// thread per (head, dim pair).  Partials go to work: m, l [B*Hq, S] and
-// acc [B*Hq, S, 128].
+// kh.  Scores: one lane per position, an FMA chain over the dims; softmax
+// partials per head; PV: one thread per (head, dim) and position mod 4.
+// Partials go to work: m, l [B*Hq, S] and acc [B*Hq, S, 128].
+//
+// Eight waves: wave v takes positions 64 (v mod 4).. and half of the heads
+// for the scores, half of the dims for PV.  Keys and values are both loaded
+// before q is prepared (one round trip); keys go to LDS in coalesced loads,
+// 16-byte units exclusive-ored with their row so a lane reads its row
+// without conflicts; a wave's sums use permlane swaps and DPP.
 //
 // kFused: q comes from the projection output through the per-head norm and
-// rotary embedding (norm_rope_pair), and the split holding position pos[0]
-// first writes the new token's k and v to the caches -- the work of
-// qk_norm_rope_kernel, in the same arithmetic.  (Merging the splits in the
-// last workgroup to finish would need device-scope fences, which on this
+// rotary embedding (norm_rope), and the split holding position pos[0] writes
+// the new token's k and v to the caches -- the work of qk_norm_rope_kernel,
+// in the same arithmetic -- and takes them from LDS.  (Merging the splits in
+// the last workgroup to finish would need device-scope fences, which on this
 // multi-XCD part write back and invalidate the whole L2: the merge stays a
 // kernel of its own.)
+//
+// HBM-bound for long contexts, the latency of one workgroup for short ones;
+// MI355X, 16 sequences, with the merge, us before (each lane loading its own
+// key row, values after the softmax, LDS shuffles) and now: 8192 positions
+// 142.9 -> 118.4 (8 query heads per KV head 100.5 -> 79.4), 640 19.7 -> 18.8.
+// (Scores from MFMAs took 108 and 67, but sum in another order: the FP8
+// codes of a decode step then differ from those of the kernel it replaces.)
+constexpr int kAttnWaves = 8;
+
 template <int G, bool kFused>
-__global__ __launch_bounds__(256) void attn_split_kernel(const uint16_t *__restrict__ q,
-                                                         uint16_t *__restrict__ kc,
-                                                         uint16_t *__restrict__ vc,
-                                                         const int *__restrict__ pos, int Hkv,
-                                                         int Lmax, int S, float *__restrict__ wm,
-                                                         float *__restrict__ wl,
-                                                         float *__restrict__ wacc, AttnFused fu) {
-  __shared__ float qs[G][kHeadDim];
-  __shared__ float pw[G][kAttnChunk];
-  __shared__ float part[4 * G * kHeadDim];  // PV partials [wave][head][dim]
-  __shared__ float red[G][4];
+__global__ __launch_bounds__(64 * kAttnWaves) void attn_split_kernel(
+    const uint16_t *__restrict__ q, uint16_t *__restrict__ kc, uint16_t *__restrict__ vc,
+    const int *__restrict__ pos, int Hkv, int Lmax, int S, float *__restrict__ wm,
+    float *__restrict__ wl, float *__restrict__ wacc, AttnFused fu) {
+  constexpr int kUnits = kHeadDim / 8;  // 16-byte units of a row
+  __shared__ u32x4 s_k[kAttnChunk * kUnits];
+  __shared__ __attribute__((aligned(16))) float qs[G][kHeadDim];
+  // probability of position 64 w + j: [h][w][16 (j mod 4) + j / 4]
+  __shared__ __attribute__((aligned(16))) float pw[G][4][64];
+  __shared__ uint32_t s_new[kHeadDim / 2];  // the new token's v
+  __shared__ float red[2][G][4];
+  // PV partials [position group][head][dim], over the keys once they are read
+  float(*part)[G][kHeadDim] = reinterpret_cast<float(*)[G][kHeadDim]>(s_k);
   const int bk = blockIdx.x, split = blockIdx.y;
   const int b = bk / Hkv, kh = bk % Hkv;
   const int Hq = Hkv * G;
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int p = pos[0];
   int L = p + 1;
   L = L < 1 ? 1 : (L > Lmax ? Lmax : L);
   const int c0 = split * kAttnChunk;
   const size_t head0 = (size_t)b * Hq + kh * G;
-  if (c0 >= L) {
-    if (t < G) {
-      wm[(head0 + t) * S + split] = -INFINITY;
-      wl[(head0 + t) * S + split] = 0.f;
-    }
-    return;
-  }
+  if (c0 >= L) return;  // the merge reads the splits in use only
   const int n = min(kAttnChunk, L - c0);
+  // fused: the new token's position in this chunk; past every position
+  // otherwise
+  const int fresh = kFused && p >= c0 && p < c0 + kAttnChunk && p < Lmax ? p - c0 : kAttnChunk;
   const float scale = rsqrtf((float)kHeadDim);
+
+  // The wave's head of q and the new token's k or v (the waves past the
+  // heads, or the first two): loaded first, since loads return in order and
+  // the keys take longest.
+  constexpr int kNew = G < 8 ? 4 : 0;  // wave kNew: k, wave kNew + 1: v
+  RopeIn qin, nin;
+  uint32_t qx = 0, nx = 0;
   if constexpr (kFused) {
-    const uint16_t *row = fu.qkv + (size_t)b * (Hq + 2 * Hkv) * kHeadDim;
-    const int pc = min(max(p, 0), Lmax - 1);  // rotary row (p is in range for a valid call)
-    for (int h = wave; h < G; h += 4) {
-      const uint32_t x2 =
-          *reinterpret_cast<const uint32_t *>(row + (kh * G + h) * kHeadDim + 2 * lane);
-      const uint32_t y2 = norm_rope_pair(x2, fu.qn, fu.eps, fu.cosv, fu.sinv, pc, lane);
-      qs[h][2 * lane] = bf16_f32(y2 & 0xffffu) * scale;
-      qs[h][2 * lane + 1] = bf16_f32(y2 >> 16) * scale;
+    const uint16_t *row = fu.qkv + (size_t)b * (Hq + 2 * Hkv) * kHeadDim + 2 * lane;
+    // rotary row (p is in range for a valid call)
+    qin = rope_load(fu.qn, fu.cosv, fu.sinv, min(max(p, 0), Lmax - 1), lane);
+    nin = qin;
+    nin.w2 = *reinterpret_cast<const uint32_t *>(fu.kn + 2 * lane);
+    if (wave < G) qx = *reinterpret_cast<const uint32_t *>(row + (size_t)(kh * G + wave) * kHeadDim);
+    if (wave == kNew || wave == kNew + 1)
+      nx = *reinterpret_cast<const uint32_t *>(row +
+                                               (size_t)(Hq + (wave - kNew) * Hkv + kh) * kHeadDim);
+  }
+  const size_t row0 = ((size_t)b * Hkv + kh) * Lmax + c0;
+  const int pg = wave & 3, half = wave >> 2;
+  const int dg = lane & 15, rr = lane >> 4;
+  u32x4 kr[kAttnChunk * kUnits / 512];
+#pragma unroll
+  for (int i = 0; i < kAttnChunk * kUnits / 512; ++i) {
+    const int row = (t + 512 * i) / kUnits, c = t % kUnits;
+    if (row < n)
+      kr[i] = *reinterpret_cast<const u32x4 *>(kc + (row0 + row) * kHeadDim + 8 * c);
+  }
+  // values: positions 64 pg + 4 st + rr, dims 64 half + 4 dg..; positions
+  // past n read row n - 1 with weight 0
+  u32x2 vv[16];
+#pragma unroll
+  for (int st = 0; st < 16; ++st)
+    vv[st] = *reinterpret_cast<const u32x2 *>(
+        vc + (row0 + min(64 * pg + 4 * st + rr, n - 1)) * kHeadDim + 64 * half + 4 * dg);
+
+  if constexpr (kFused) {
+    if (wave < G) {
+      const uint32_t y2 = norm_rope(qx, qin, fu.eps, lane);
+      qs[wave][2 * lane] = bf16_f32(y2 & 0xffffu) * scale;
+      qs[wave][2 * lane + 1] = bf16_f32(y2 >> 16) * scale;
     }
-    if (p >= c0 && p < c0 + kAttnChunk && p < Lmax && wave < 2) {
-      // the new token's k (wave 0) and v (wave 1) go to the caches first
-      const int hh = Hq + wave * Hkv + kh;
-      const uint32_t x2 = *reinterpret_cast<const uint32_t *>(row + hh * kHeadDim + 2 * lane);
-      const uint32_t y2 = wave == 0 ? norm_rope_pair(x2, fu.kn, fu.eps, fu.cosv, fu.sinv, p, lane)
-                                    : x2;
-      uint16_t *cache = wave == 0 ? kc : vc;
-      *reinterpret_cast<uint32_t *>(cache + (((size_t)b * Hkv + kh) * Lmax + p) * kHeadDim +
-                                    2 * lane) = y2;
+    if (fresh < kAttnChunk && (wave == kNew || wave == kNew + 1)) {
+      const uint32_t y2 = wave == kNew ? norm_rope(nx, nin, fu.eps, lane) : nx;
+      uint16_t *cache = wave == kNew ? kc : vc;
+      *reinterpret_cast<uint32_t *>(cache + (row0 + fresh) * kHeadDim + 2 * lane) = y2;
+      if (wave == kNew)
+        reinterpret_cast<uint32_t *>(
+            &s_k[fresh * kUnits + ((lane >> 2) ^ (fresh & (kUnits - 1)))])[lane & 3] = y2;
+      else
+        s_new[lane] = y2;
     }
-    __threadfence_block();  // the row is read back below by other waves
   } else {
-    for (int i = t; i < G * kHeadDim; i += 256) {
+    for (int i = t; i < G * kHeadDim; i += 512)
       qs[i / kHeadDim][i % kHeadDim] =
           bf16_f32(q[(head0 + i / kHeadDim) * kHeadDim + i % kHeadDim]) * scale;
-    }
   }
-  __syncthreads();
-
-  const int j = 64 * wave + lane;  // position within the chunk
-  float s[G];
 #pragma unroll
-  for (int h = 0; h < G; ++h) s[h] = 0.f;
+  for (int i = 0; i < kAttnChunk * kUnits / 512; ++i) {
+    const int row = (t + 512 * i) / kUnits, c = t % kUnits;
+    if (row < n && row != fresh) s_k[row * kUnits + (c ^ (row & (kUnits - 1)))] = kr[i];
+  }
+  lds_barrier();
+  if (kFused && fresh < 64 * pg + 64) {  // uniform
+    // the fresh row, also for the positions past it (their loads found the
+    // row as it was before)
+    const u32x2 nv = *reinterpret_cast<const u32x2 *>(&s_new[32 * half + 2 * dg]);
+#pragma unroll
+    for (int st = 0; st < 16; ++st)
+      if (64 * pg + 4 * st + rr >= fresh) vv[st] = nv;
+  }
+
+  constexpr int kH = G / 2;  // heads of this wave's scores: half * kH..
+  const int j = 64 * pg + lane;  // position within the chunk
+  float s[kH];
+#pragma unroll
+  for (int h = 0; h < kH; ++h) s[h] = 0.f;
   const bool valid = j < n;
   if (valid) {
-    // the whole 256-byte key row in flight at once
-    const uint4 *kr = reinterpret_cast<const uint4 *>(kc + (((size_t)b * Hkv + kh) * Lmax + c0 + j) * kHeadDim);
-    uint4 kv[kHeadDim / 8];
 #pragma unroll
-    for (int c = 0; c < kHeadDim / 8; ++c) kv[c] = kr[c];
-#pragma unroll
-    for (int c = 0; c < kHeadDim / 8; ++c) {
-      const uint32_t wds[4] = {kv[c].x, kv[c].y, kv[c].z, kv[c].w};
+    for (int c = 0; c < kUnits; ++c) {
+      const u32x4 kv = s_k[j * kUnits + (c ^ (j & (kUnits - 1)))];
+      float kf[8];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float k0 = bf16_f32(wds[e] & 0xffffu), k1 = bf16_f32(wds[e] >> 16);
+        kf[2 * e] = bf16_f32(kv[e] & 0xffffu);
+        kf[2 * e + 1] = __uint_as_float(kv[e] & 0xffff0000u);
+      }
 #pragma unroll
-        for (int h = 0; h < G; ++h) {
-          s[h] = fmaf(qs[h][8 * c + 2 * e], k0, s[h]);
-          s[h] = fmaf(qs[h][8 * c + 2 * e + 1], k1, s[h]);
-        }
+      for (int h = 0; h < kH; ++h) {
+        const float4 q0 = *reinterpret_cast<const float4 *>(&qs[half * kH + h][8 * c]);
+        const float4 q1 = *reinterpret_cast<const float4 *>(&qs[half * kH + h][8 * c + 4]);
+        s[h] = fmaf(q0.x, kf[0], s[h]);
+        s[h] = fmaf(q0.y, kf[1], s[h]);
+        s[h] = fmaf(q0.z, kf[2], s[h]);
+        s[h] = fmaf(q0.w, kf[3], s[h]);
+        s[h] = fmaf(q1.x, kf[4], s[h]);
+        s[h] = fmaf(q1.y, kf[5], s[h]);
+        s[h] = fmaf(q1.z, kf[6], s[h]);
+        s[h] = fmaf(q1.w, kf[7], s[h]);
       }
     }
   }
-  float mh[G];
 #pragma unroll
-  for (int h = 0; h < G; ++h) {
-    const float mw = wave_max(valid ? s[h] : -INFINITY);
-    if (lane == 0) red[h][wave] = mw;
+  for (int h = 0; h < kH; ++h) {
+    const float mw = wave_max_dpp(valid ? s[h] : -INFINITY);
+    if (lane == 0) red[0][half * kH + h][pg] = mw;
   }
-  __syncthreads();
+  lds_barrier();
 #pragma unroll
-  for (int h = 0; h < G; ++h) mh[h] = fmaxf(fmaxf(red[h][0], red[h][1]), fmaxf(red[h][2], red[h][3]));
-  __syncthreads();
-#pragma unroll
-  for (int h = 0; h < G; ++h) {
-    const float e = valid ? expf(s[h] - mh[h]) : 0.f;
-    pw[h][j] = e;
-    const float sw = wave_sum(e);
-    if (lane == 0) red[h][wave] = sw;
+  for (int h = 0; h < kH; ++h) {
+    const float *rm = red[0][half * kH + h];
+    const float mh = fmaxf(fmaxf(rm[0], rm[1]), fmaxf(rm[2], rm[3]));
+    const float e = valid ? expf(s[h] - mh) : 0.f;
+    pw[half * kH + h][pg][16 * (lane & 3) + (lane >> 2)] = e;
+    const float sw = wave_sum_dpp(e);
+    if (lane == 0) red[1][half * kH + h][pg] = sw;
   }
-  __syncthreads();
+  lds_barrier();
   if (t < G) {
-    wm[(head0 + t) * S + split] = mh[t];
-    wl[(head0 + t) * S + split] = (red[t][0] + red[t][1]) + (red[t][2] + red[t][3]);
+    wm[(head0 + t) * S + split] =
+        fmaxf(fmaxf(red[0][t][0], red[0][t][1]), fmaxf(red[0][t][2], red[0][t][3]));
+    wl[(head0 + t) * S + split] =
+        (red[1][t][0] + red[1][t][1]) + (red[1][t][2] + red[1][t][3]);
   }
-  // PV: wave w takes positions [64w, 64w + 64) of the chunk, four rows per
-  // step (lane / 16), eight dims per lane (16-byte loads), all 16 row loads
-  // in flight; positions past n read row n - 1 with weight 0.
-  const int dg = lane & 15, rr = lane >> 4;
-  const uint16_t *vbase = vc + (((size_t)b * Hkv + kh) * Lmax + c0) * kHeadDim + 8 * dg;
-  uint4 vv[16];
-#pragma unroll
-  for (int st = 0; st < 16; ++st) {
-    const int jj = min(64 * wave + 4 * st + rr, n - 1);
-    vv[st] = *reinterpret_cast<const uint4 *>(vbase + (size_t)jj * kHeadDim);
-  }
-  float acc[G][8];
+  float acc[G][4];
 #pragma unroll
   for (int h = 0; h < G; ++h)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) acc[h][e] = 0.f;
+    for (int e = 0; e < 4; ++e) acc[h][e] = 0.f;
 #pragma unroll
-  for (int st = 0; st < 16; ++st) {
-    const int jp = 64 * wave + 4 * st + rr;
-    const uint32_t wds[4] = {vv[st].x, vv[st].y, vv[st].z, vv[st].w};
-#pragma unroll
-    for (int h = 0; h < G; ++h) {
-      const float p = pw[h][jp];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        acc[h][2 * e] = fmaf(p, bf16_f32(wds[e] & 0xffffu), acc[h][2 * e]);
-        acc[h][2 * e + 1] = fmaf(p, bf16_f32(wds[e] >> 16), acc[h][2 * e + 1]);
-      }
-    }
-  }
-#pragma unroll
-  for (int h = 0; h < G; ++h)
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      float v = acc[h][e];
-      v += __shfl_xor(v, 16);
-      v += __shfl_xor(v, 32);
-      acc[h][e] = v;
-    }
-  if (rr == 0) {
+  for (int s4 = 0; s4 < 4; ++s4) {
+    float4 pv[G];
 #pragma unroll
     for (int h = 0; h < G; ++h)
+      pv[h] = *reinterpret_cast<const float4 *>(&pw[h][pg][16 * rr + 4 * s4]);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) part[(wave * G + h) * kHeadDim + 8 * dg + e] = acc[h][e];
+    for (int i = 0; i < 4; ++i) {
+      const u32x2 wds = vv[4 * s4 + i];
+      const float v0 = bf16_f32(wds[0] & 0xffffu), v1 = __uint_as_float(wds[0] & 0xffff0000u);
+      const float v2 = bf16_f32(wds[1] & 0xffffu), v3 = __uint_as_float(wds[1] & 0xffff0000u);
+#pragma unroll
+      for (int h = 0; h < G; ++h) {
+        const float pr = i == 0 ? pv[h].x : i == 1 ? pv[h].y : i == 2 ? pv[h].z : pv[h].w;
+        acc[h][0] = fmaf(pr, v0, acc[h][0]);
+        acc[h][1] = fmaf(pr, v1, acc[h][1]);
+        acc[h][2] = fmaf(pr, v2, acc[h][2]);
+        acc[h][3] = fmaf(pr, v3, acc[h][3]);
+      }
+    }
   }
-  __syncthreads();
-  for (int v = t; v < G * kHeadDim; v += 256) {
+  // every wave is past its keys (two barriers ago): part overlays them.  The
+  // four lane rows' sums, (0 + 1) + (2 + 3), four accumulators at a time:
+  // lane row g holds dim 4 dg + g's.
+#pragma unroll
+  for (int h = 0; h < G; ++h)
+    part[pg][h][64 * half + 4 * dg + rr] =
+        add_swap32(add_swap16(acc[h][0], acc[h][1]), add_swap16(acc[h][2], acc[h][3]));
+  lds_barrier();
+  for (int v = t; v < G * kHeadDim; v += 512) {
     const int h = v / kHeadDim, d = v % kHeadDim;
-    const float sum = (part[(0 * G + h) * kHeadDim + d] + part[(1 * G + h) * kHeadDim + d]) +
-                      (part[(2 * G + h) * kHeadDim + d] + part[(3 * G + h) * kHeadDim + d]);
-    wacc[((head0 + h) * S + split) * kHeadDim + d] = sum;
+    wacc[((head0 + h) * S + split) * kHeadDim + d] =
+        (part[0][h][d] + part[1][h][d]) + (part[2][h][d] + part[3][h][d]);
   }
 }
 
-// Merge the splits of one (b, head) and quantize the head's 128 outputs
-// (one activation group of the o projection); optionally also write bf16.
+// Merge the splits [0, used) of one (b, head) -- partials m, l [B*Hq, S] and
+// acc [B*Hq, S, 128] -- in order, and write its 128 outputs: quantized as
+// one o-projection group, and optionally as bf16.  One wave, two dims per
+// lane.  Latency-bound, so eight splits' loads are in flight at a time (16 x
+// 32 heads of 33 splits: 15.9 us one by one, 7.8 now).
 __global__ __launch_bounds__(64) void attn_combine_kernel(const float *__restrict__ wm,
                                                           const float *__restrict__ wl,
                                                           const float *__restrict__ wacc,
@@ -1199,10 +1280,56 @@ __global__ __launch_bounds__(64) void attn_combine_kernel(const float *__restric
                                                           int S, int Hq, uint8_t *__restrict__ oq,
                                                           float *__restrict__ os,
                                                           uint16_t *__restrict__ ob) {
+  const int lane = threadIdx.x;
   int L = pos[0] + 1;
   L = L < 1 ? 1 : (L > Lmax ? Lmax : L);
   const int used = (L + kAttnChunk - 1) / kAttnChunk;
-  combine_head(wm, wl, wacc, blockIdx.x, S, used, threadIdx.x, Hq, oq, os, ob);
+  const size_t bh = blockIdx.x;
+  const float *pm = wm + bh * S, *pl = wl + bh * S;
+  const float2 *pa = reinterpret_cast<const float2 *>(wacc + bh * S * kHeadDim) + lane;
+  constexpr int kU = 8;
+  float2 a[kU];
+  auto load = [&](int s0) {
+#pragma unroll
+    for (int u = 0; u < kU; ++u) a[u] = pa[(size_t)min(s0 + u, used - 1) * 64];
+  };
+  load(0);
+  float mx = -INFINITY;
+  for (int s = lane; s < used; s += 64) mx = fmaxf(mx, pm[s]);
+  mx = wave_max_dpp(mx);
+  float l = 0.f, a0 = 0.f, a1 = 0.f;
+  for (int s0 = 0; s0 < used; s0 += kU) {
+    float2 c[kU];
+    float f[kU], ls[kU];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const int s = min(s0 + u, used - 1);
+      c[u] = a[u];
+      f[u] = pm[s];
+      ls[u] = pl[s];
+    }
+    if (s0 + kU < used) load(s0 + kU);
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      if (s0 + u < used) {  // uniform
+        const float e = expf(f[u] - mx);
+        l = fmaf(e, ls[u], l);
+        a0 = fmaf(e, c[u].x, a0);
+        a1 = fmaf(e, c[u].y, a1);
+      }
+    }
+  }
+  a0 /= l;
+  a1 /= l;
+  if (ob) reinterpret_cast<uint32_t *>(ob)[bh * 64 + lane] = f32_bf16(a0) | (f32_bf16(a1) << 16);
+  const float amax = wave_max_dpp(fmaxf(fabsf(a0), fabsf(a1)));
+  const float sc = amax > 0.f ? amax / kFp8Max : 1.f;
+  const uint32_t q2 = f32_e4m3(a0 / sc) | (f32_e4m3(a1 / sc) << 8);
+  // row b = bh / Hq, group = head: bytes 2 lane, 2 lane + 1 of the group
+  const int b = (int)(bh / (size_t)Hq), head = (int)(bh % (size_t)Hq);
+  *reinterpret_cast<uint16_t *>(oq + tile_chunk_off(b, head, Hq, lane >> 3) + 2 * (lane & 7)) =
+      (uint16_t)q2;
+  if (lane == 0) os[bh] = sc;
 }
 
 // ---------------------------------------------------- FP8 block dequantize
@@ -1591,13 +1718,6 @@ __global__ __launch_bounds__(WAVES * 64) void moe_linear16_kernel(MoeLinear a) {
   }
 }
 
-// Workgroup barrier that waits for LDS only (a __syncthreads would also
-// wait for the prefetched global loads).
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_s_waitcnt((0x3F & 15) | (0x3 << 14) | (0x7 << 4) | (0x0 << 8));  // lgkmcnt(0)
-  gemm_barrier();
-}
-
 // The same grouped linear for many rows per expert (a prompt): workgroup
 // (strip, slot) of eight waves computes a 128-column strip of expert
 // active[slot], wave w its columns [16 w, +16), for 16 kChunks rows at a
@@ -1975,10 +2095,10 @@ extern "C" int ecf8_decode_attention(const void *q, const void *k_cache, const v
   auto *vp = static_cast<uint16_t *>(const_cast<void *>(v_cache));
   const AttnFused none{};
   if (Hq == 4 * Hkv)
-    attn_split_kernel<4, false><<<grid, 256, 0, as_stream(stream)>>>(
+    attn_split_kernel<4, false><<<grid, 64 * kAttnWaves, 0, as_stream(stream)>>>(
         qp, kp, vp, pos, Hkv, (int)Lmax, (int)S, wm, wl, wacc, none);
   else
-    attn_split_kernel<8, false><<<grid, 256, 0, as_stream(stream)>>>(
+    attn_split_kernel<8, false><<<grid, 64 * kAttnWaves, 0, as_stream(stream)>>>(
         qp, kp, vp, pos, Hkv, (int)Lmax, (int)S, wm, wl, wacc, none);
   attn_combine_kernel<<<(unsigned)(B * Hq), 64, 0, as_stream(stream)>>>(
       wm, wl, wacc, pos, (int)Lmax, (int)S, Hq, static_cast<uint8_t *>(out_q), out_scale,
@@ -2010,10 +2130,10 @@ extern "C" int ecf8_decode_attention_fused(const void *qkv, int64_t B, int Hq, i
   auto *kp = static_cast<uint16_t *>(k_cache);
   auto *vp = static_cast<uint16_t *>(v_cache);
   if (Hq == 4 * Hkv)
-    attn_split_kernel<4, true><<<grid, 256, 0, as_stream(stream)>>>(
+    attn_split_kernel<4, true><<<grid, 64 * kAttnWaves, 0, as_stream(stream)>>>(
         nullptr, kp, vp, pos, Hkv, (int)Lmax, (int)S, wm, wl, wacc, fu);
   else
-    attn_split_kernel<8, true><<<grid, 256, 0, as_stream(stream)>>>(
+    attn_split_kernel<8, true><<<grid, 64 * kAttnWaves, 0, as_stream(stream)>>>(
         nullptr, kp, vp, pos, Hkv, (int)Lmax, (int)S, wm, wl, wacc, fu);
   attn_combine_kernel<<<(unsigned)(B * Hq), 64, 0, as_stream(stream)>>>(
       wm, wl, wacc, pos, (int)Lmax, (int)S, Hq, static_cast<uint8_t *>(out_q), out_scale,

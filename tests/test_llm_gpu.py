@@ -411,6 +411,62 @@ def test_decode_attention_matches_fp32(cuda_device, pos0, G):
     _assert_fp8_close(from_tiles(oq, B, Hq * 128), os_, ref, rel=2 ** -4 + 5e-3)
 
 
+@pytest.mark.parametrize("G", [4, 8])
+@pytest.mark.parametrize("p", [0, 1, 30, 31, 32, 33, 63, 64, 223, 254, 255, 256, 287, 288, 700])
+def test_fused_decode_attention_at_the_edges_of_its_splits(cuda_device, p, G):
+    """Positions at the edges of a wave's 64 and a workgroup's 256; the
+    caches from the new position on hold NaN, which must not reach a result.
+    Against fp64 on bf16-rounded q and k (2^-8 relative for the bf16 output
+    plus 2^-16 of the largest value)."""
+    from ecf8_amd.llm_kernels import attention_work, decode_attention_fused
+
+    B, Hkv, Lmax = 3, 2, 701
+    Hq, dev = G * Hkv, cuda_device
+    gen = torch.Generator(device=dev).manual_seed(p * 10 + G)
+
+    def rand(*shape):
+        return torch.randn(shape, generator=gen, device=dev).to(torch.bfloat16)
+
+    qkv, kc, vc = rand(B, (Hq + 2 * Hkv) * 128), rand(B, Hkv, Lmax, 128), rand(B, Hkv, Lmax, 128)
+    kc[:, :, p:] = float("nan")
+    vc[:, :, p:] = float("nan")
+    qn, kn = (1 + 0.1 * rand(128).float()).bfloat16(), (1 + 0.1 * rand(128).float()).bfloat16()
+    cos, sin = (t.to(dev) for t in _rope_tables(Lmax))
+    pos = torch.tensor([p], dtype=torch.int32, device=dev)
+    out_q = torch.zeros(16, Hq * 128, dtype=torch.uint8, device=dev).view(torch.float8_e4m3fn)
+    out_s, out_b = torch.zeros(B, Hq, device=dev), torch.zeros(B, Hq * 128, dtype=torch.bfloat16,
+                                                               device=dev)
+    old_k, old_v = kc.clone(), vc.clone()
+    decode_attention_fused(qkv, B, Hq, Hkv, qn, kn, 1e-6, cos, sin, pos, kc, vc,
+                           attention_work(B, Hq, Lmax, dev), out_q, out_s, out_b)
+    x = qkv.double().view(B, Hq + 2 * Hkv, 128)
+
+    def rope(t, w):
+        t = t * torch.rsqrt(t.pow(2).mean(-1, keepdim=True) + 1e-6) * w.double()
+        a, b = t[..., :64], t[..., 64:]
+        c, s = cos[p].double(), sin[p].double()
+        return torch.cat([a * c - b * s, b * c + a * s], -1)
+
+    assert torch.equal(vc[:, :, p], qkv.view(B, -1, 128)[:, Hq + Hkv:])
+    k_new = rope(x[:, Hq:Hq + Hkv], kn)
+    assert torch.allclose(kc[:, :, p].double(), k_new, rtol=2 ** -7, atol=1e-6)
+    keep = torch.arange(Lmax, device=dev) != p
+    for new, old in ((kc, old_k), (vc, old_v)):  # nothing else is written
+        assert torch.equal(new[:, :, keep].view(torch.int16), old[:, :, keep].view(torch.int16))
+    q = rope(x[:, :Hq], qn).bfloat16().double()
+    k = kc[:, :, :p + 1].double().repeat_interleave(G, 1)
+    v = vc[:, :, :p + 1].double().repeat_interleave(G, 1)
+    w = torch.softmax((q[:, :, None] * k).sum(-1) / 128 ** 0.5, -1)
+    want = (w[..., None] * v).sum(2)
+    # q and k are rounded to bf16 from fp32 here and from fp64 above: a
+    # flipped last bit of q moves a score by up to 2^-8 of |q_i k_i|
+    err = (out_b.double().view(B, Hq, 128) - want).abs()
+    assert float(err.max()) <= 2.0 ** -6 * float(v.abs().max())
+    assert float(err.norm() / want.norm()) <= 2.0 ** -8
+    deq = from_tiles(out_q, B, Hq * 128).double().view(B, Hq, 128) * out_s.double()[..., None]
+    assert float((deq - want).norm() / want.norm()) <= 2.0 ** -4
+
+
 def test_wrappers_reject_bad_arguments_before_launch(cuda_device):
     """Missing outputs, short norm weights, scale buffers with too few rows
     and an empty position tensor are refused on the host; nothing is
