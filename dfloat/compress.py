@@ -19,9 +19,9 @@ import torch
 from .utils import (
     encode_exponents_for_cuda,
     flatten_block_of_weights,
-    get_exponents_and_other_4bits_fp8_e4m3,
     get_luts_from_huffman_table,
     get_nbit_codec,
+    split_fp8_counted,
 )
 
 PACKAGE_FORMAT_VERSION = "0.2.0"  # dfloat_config["version"] (scripts/compress.py:67)
@@ -32,10 +32,9 @@ def compress_flat(flat_weights: torch.Tensor, bytes_per_thread: int = 8,
     """Compress one flattened e4m3fn block (scripts/compress.py:197-247):
     split, count exponents in ascending order, length-limited codebook,
     LUTs, bitstream.  Returns the tensors plus ``entropy`` and ``table``."""
-    exps, packed = get_exponents_and_other_4bits_fp8_e4m3(flat_weights)
+    exps, packed, counts = split_fp8_counted(flat_weights)
     # a 16-bin count is O(n); the reference's ascending-symbol counter order
     # (scripts/compress.py:205, 213-215) is kept by listing present symbols
-    counts = torch.bincount(exps.reshape(-1), minlength=16)
     present = counts > 0
     freqs = counts[present]
     p = freqs.double() / freqs.sum()

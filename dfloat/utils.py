@@ -161,22 +161,46 @@ def encode_exponents_for_cuda(exponents_4bits, codec, bytes_per_thread: int = 8,
         exps = np.ascontiguousarray(exponents_4bits, dtype=np.uint8)
     bits, vals, eof_bits, eof_val = _code_arrays(codec)
     L = lib()
-    n = exps.size
+    n, threads = exps.size, host_threads()
     nb, ng, no = ctypes.c_int64(), ctypes.c_int64(), ctypes.c_int64()
     vp = lambda a: a.ctypes.data_as(ctypes.c_void_p)  # noqa: E731
-    check(L.ecf8_encoded_sizes(vp(exps), n, vp(bits), bytes_per_thread, threads_per_block,
-                               ctypes.byref(nb), ctypes.byref(ng), ctypes.byref(no)),
-          "ecf8_encoded_sizes")
-    encoded = np.zeros(max(nb.value, 1), np.uint8)
-    gaps = np.zeros(max(ng.value, 1), np.uint8)
-    op = np.zeros(no.value, np.uint64)
-    check(L.ecf8_encode_exponents(vp(exps), n, vp(bits), vp(vals), eof_bits, eof_val,
-                                  bytes_per_thread, threads_per_block, vp(encoded), nb.value,
-                                  vp(gaps), ng.value, vp(op), no.value),
-          "ecf8_encode_exponents")
-    return (torch.from_numpy(encoded[: nb.value].copy()),
-            torch.from_numpy(gaps[: ng.value].copy()),
+    check(L.ecf8_encoded_sizes_threads(vp(exps), n, vp(bits), bytes_per_thread, threads_per_block,
+                                       threads, ctypes.byref(nb), ctypes.byref(ng),
+                                       ctypes.byref(no)), "ecf8_encoded_sizes")
+    encoded = np.empty(max(nb.value, 1), np.uint8)
+    gaps = np.empty(max(ng.value, 1), np.uint8)
+    op = np.empty(no.value, np.uint64)
+    check(L.ecf8_encode_exponents_threads(vp(exps), n, vp(bits), vp(vals), eof_bits, eof_val,
+                                          bytes_per_thread, threads_per_block, threads,
+                                          vp(encoded), nb.value, vp(gaps), ng.value, vp(op),
+                                          no.value), "ecf8_encode_exponents")
+    return (torch.from_numpy(encoded)[: nb.value], torch.from_numpy(gaps)[: ng.value],
             torch.from_numpy(op))
+
+
+def host_threads() -> int:
+    """Threads of the host codec: torch's own count, at most 16."""
+    return max(1, min(torch.get_num_threads(), 16))
+
+
+def split_fp8_counted(data: torch.Tensor):
+    """(exponents, packed nibbles, exponent counts [16]) of a flat e4m3fn
+    tensor: get_exponents_and_other_4bits_fp8_e4m3 and a count; plain host
+    tensors in one native pass."""
+    if (data.device.type == "cpu" and type(data) in (torch.Tensor, torch.nn.Parameter)
+            and data.ndim == 1 and data.dtype == torch.float8_e4m3fn and data.is_contiguous()
+            and data.numel() % 2 == 0 and data.numel() > 0):
+        from ecf8_amd._lib import check, lib
+
+        n = data.numel()
+        exps = torch.empty(n, dtype=torch.uint8)
+        packed = torch.empty(n // 2, dtype=torch.uint8)
+        counts = torch.empty(16, dtype=torch.int64)
+        check(lib().ecf8_split_fp8(data.data_ptr(), n, exps.data_ptr(), packed.data_ptr(),
+                                   counts.data_ptr(), host_threads()), "ecf8_split_fp8")
+        return exps, packed, counts
+    exps, packed = get_exponents_and_other_4bits_fp8_e4m3(data)
+    return exps, packed, torch.bincount(exps.reshape(-1), minlength=16)
 
 
 # ------------------------------------------------------------ block lookup

@@ -57,6 +57,10 @@ _SIGNATURES = {
     ),
     "ecf8_stream_probe": ([_i32, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _vp, _vp], _i32),
     # include/ecf8_tile.h: the tiled execution layout
+    "ecf8_encoded_sizes_threads": ([_vp, _i64, _vp, _i32, _i32, _i32, _vp, _vp, _vp], _i32),
+    "ecf8_encode_exponents_threads": ([_vp, _i64, _vp, _vp, _i32, _u32, _i32, _i32, _i32, _vp,
+                                       _i64, _vp, _i64, _vp, _i64], _i32),
+    "ecf8_split_fp8": ([_vp, _i64, _vp, _vp, _vp, _i32], _i32),
     "ecf8_code_from_luts": ([_vp, _i32, _vp, _vp], _i32),
     "ecf8_tile_sizes": ([_vp, _i64, _i64, _vp, _vp, _vp], _i32),
     "ecf8_tile_encode": ([_vp, _i64, _i64, _vp, _vp, _vp, _i64, _vp, _vp, _vp, _i32], _i32),

@@ -302,6 +302,29 @@ int ecf8_encode_exponents(const uint8_t *exponents, int64_t n, const uint8_t *co
                           uint64_t *output_positions, int64_t output_positions_capacity);
 
 /*
+ * ecf8_encoded_sizes and ecf8_encode_exponents on up to n_threads threads
+ * (64 at most, 65,536 exponents or more each), the same bytes and statuses.
+ */
+int ecf8_encoded_sizes_threads(const uint8_t *exponents, int64_t n, const uint8_t *code_bits,
+                               int bytes_per_thread, int threads_per_block, int n_threads,
+                               int64_t *n_bytes, int64_t *gaps_bytes,
+                               int64_t *n_output_positions);
+int ecf8_encode_exponents_threads(const uint8_t *exponents, int64_t n, const uint8_t *code_bits,
+                                  const uint32_t *code_vals, int eof_bits, uint32_t eof_value,
+                                  int bytes_per_thread, int threads_per_block, int n_threads,
+                                  uint8_t *encoded, int64_t encoded_capacity, uint8_t *gaps,
+                                  int64_t gaps_capacity, uint64_t *output_positions,
+                                  int64_t output_positions_capacity);
+
+/*
+ * e4m3fn weights (n even) -> 4-bit exponents u8[n], sign | mantissa nibbles
+ * u8[n/2] (even element high) and the count of each exponent i64[16], in one
+ * pass on up to n_threads threads.  Host memory.
+ */
+int ecf8_split_fp8(const uint8_t *weights, int64_t n, uint8_t *exponents, uint8_t *packed,
+                   int64_t *counts, int n_threads);
+
+/*
  * Format validator for one compressed block (host memory).  No reference
  * counterpart (the reference validates nothing before launch); it checks the
  * invariants the decode rule relies on: LUT stack shape and pointers

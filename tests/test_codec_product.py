@@ -191,3 +191,79 @@ def test_product_length_limiter_equals_the_oracle_on_a_large_alphabet():
     assert {str(k): v for k, v in table.items()} == {str(k): v for k, v in ref_table.items()}
     assert dict(used) == dict(ref_used)
     assert codec.get_code_table() is table
+
+
+def _huffman_codes(rng, kind):
+    """(exponent distribution, code lengths, code values) of a prefix code."""
+    from dfloat.huffman import get_nbit_codec
+
+    p = {"flat": np.ones(16), "steep": 0.5 ** np.arange(16), "two": np.array([.9, .1] + [0] * 14),
+         "fib": np.array([1, 1, 2, 3, 5, 8, 13, 21, 34, 55, 89, 144, 233, 377, 610, 987.])}[kind]
+    p = p / p.sum()
+    counter = {i: max(1, int(1e6 * v)) for i, v in enumerate(p) if v > 0}
+    codec = get_nbit_codec(counter, max_n_bits=16)[0]
+    bits, vals = np.zeros(16, np.uint8), np.zeros(16, np.uint32)
+    for s, (b, v) in codec._table.items():
+        if isinstance(s, (int, np.integer)):
+            bits[s], vals[s] = b, v
+    return p, bits, vals, *codec._table[codec._eof]
+
+
+@pytest.mark.parametrize("kind", ["flat", "steep", "two", "fib"])
+@pytest.mark.parametrize("bpt,tpb", [(8, 512), (8, 128), (2, 2), (3, 6), (64, 4096)])
+def test_threaded_encoder_writes_the_same_bytes(kind, bpt, tpb):
+    """Runs that start inside bytes, chunks and format-blocks, against the
+    one-thread encoder, byte for byte with guard bytes past every output."""
+    import ctypes
+
+    from ecf8_amd._lib import lib
+
+    L, rng = lib(), np.random.default_rng(bpt * 100 + tpb)
+    p, bits, vals, eof_bits, eof_val = _huffman_codes(rng, kind)
+    vp = lambda a: a.ctypes.data_as(ctypes.c_void_p)  # noqa: E731
+    for n in (0, 1, 2, 65536 * 2 - 1, 65536 * 2, 65536 * 3 + 17, 65536 * 7 + 1):
+        exps = rng.choice(16, n, p=p).astype(np.uint8)
+        ref = [ctypes.c_int64() for _ in range(3)]
+        assert L.ecf8_encoded_sizes(vp(exps), n, vp(bits), bpt, tpb, *map(ctypes.byref, ref)) == 0
+        want = [np.zeros(ref[0].value, np.uint8), np.zeros(ref[1].value, np.uint8),
+                np.zeros(ref[2].value, np.uint64)]
+        assert L.ecf8_encode_exponents(vp(exps), n, vp(bits), vp(vals), eof_bits, eof_val, bpt, tpb,
+                                       vp(want[0]), want[0].size, vp(want[1]), want[1].size,
+                                       vp(want[2]), want[2].size) == 0
+        for threads in (1, 2, 3, 7, 200):
+            got = [ctypes.c_int64() for _ in range(3)]
+            assert L.ecf8_encoded_sizes_threads(vp(exps), n, vp(bits), bpt, tpb, threads,
+                                                *map(ctypes.byref, got)) == 0
+            assert [g.value for g in got] == [r.value for r in ref]
+            out = [np.full(w.size + 2, 0xA5, w.dtype) for w in want]
+            assert L.ecf8_encode_exponents_threads(
+                vp(exps), n, vp(bits), vp(vals), eof_bits, eof_val, bpt, tpb, threads, vp(out[0]),
+                want[0].size, vp(out[1]), want[1].size, vp(out[2]), want[2].size) == 0
+            for o, w in zip(out, want):
+                assert np.array_equal(o[: w.size], w) and (o[w.size:] == 0xA5).all()
+            if n > 65536 * 2 and threads > 1:  # refusals
+                short = L.ecf8_encode_exponents_threads(
+                    vp(exps), n, vp(bits), vp(vals), eof_bits, eof_val, bpt, tpb, threads,
+                    vp(out[0]), want[0].size - 1, vp(out[1]), want[1].size, vp(out[2]),
+                    want[2].size)
+                assert short == 6
+                bad = exps.copy()
+                bad[n - 3] = 16
+                assert L.ecf8_encode_exponents_threads(
+                    vp(bad), n, vp(bits), vp(vals), eof_bits, eof_val, bpt, tpb, threads,
+                    vp(out[0]), want[0].size, vp(out[1]), want[1].size, vp(out[2]),
+                    want[2].size) == 4
+
+
+@pytest.mark.parametrize("n", [2, 254, 131072, 131074, 400002])
+def test_split_counts_and_nibbles(n):
+    from dfloat.utils import get_exponents_and_other_4bits_fp8_e4m3, split_fp8_counted
+
+    b = torch.from_numpy(np.random.default_rng(n).integers(0, 256, n, dtype=np.uint8))
+    w = b.view(torch.float8_e4m3fn)
+    exps, packed, counts = split_fp8_counted(w)
+    want_e, want_p = get_exponents_and_other_4bits_fp8_e4m3(w)
+    assert torch.equal(exps, want_e) and torch.equal(packed, want_p)
+    assert torch.equal(counts, torch.bincount(want_e, minlength=16))
+    again = split_fp8_counted(b.repeat_interleave(2)[::2].view(torch.float8_e4m3fn))  # strided
+    assert torch.equal(again[0], want_e) and torch.equal(again[1], want_p)
