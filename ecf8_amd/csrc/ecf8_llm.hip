@@ -213,8 +213,9 @@ struct WeightLane {
 // ------------------------------------------------ prompt-size GEMM (M > 16)
 //
 // out[m, col + n] = sum_g (sum_{k in g} aq[m,k] * w[n,k]) * as[m,g] * ws[n/128, g]
-// for M > 16: 128 x 128 output tiles per 256-lane workgroup (2 x 2 waves of
-// 64 x 64), one 128-column K group per step through a two-stage LDS ring.
+// for M > 16: 256 x 256 or 256 x 128 output tiles per workgroup of eight
+// waves, one 128-column K group per step through a ring of two or three LDS
+// stages.
 //
 // Every operand block -- 16 rows x one K group, 2 KB -- lands in LDS in
 // the tile layout of ecf8_llm.h straight from global memory
@@ -231,8 +232,27 @@ struct WeightLane {
 // stored.  Workgroups are ordered so each XCD (blockIdx.x mod 8) takes a
 // contiguous run of tiles, column block by column block: the weight block
 // a tile column reads stays in that XCD's L2 across its row blocks.
+//
+// Two waves share a SIMD.  They take turns, a barrier apart: four waves read
+// their operands from LDS while the other four multiply, so the reads hide
+// behind the MFMAs instead of all waves doing both in step.  LDS reads bound
+// it (an operand is read by each wave that uses it): without the MFMAs a 256
+// x 256 tile takes 0.82 of the time, without the loads to LDS 0.86.  Qwen3-8B
+// prompt of 2048 rows, us, all waves in step on 256 x 128 tiles before and
+// now: gate/up 262 -> 210, q/k/v 80 -> 69, o 47 -> 44, down 118 -> 110; M =
+// 4096: gate/up 533 -> 427 (1.93 PFLOP/s), down 256 -> 207.  (The weights'
+// operand straight from L2 into registers instead, a phase ahead: 1.1 to 1.3
+// times as long.)
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef int v4i __attribute__((ext_vector_type(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
+  const v2bf v = {(__bf16)lo, (__bf16)hi};
+  return __builtin_bit_cast(uint32_t, v);
+}
 
 __device__ __forceinline__ void lds_load16(const uint8_t *g, void *lds) {
   __builtin_amdgcn_global_load_lds(g, (__attribute__((address_space(3))) void *)lds, 16, 0, 0);
@@ -258,40 +278,94 @@ __device__ __forceinline__ void lds_barrier() {
   gemm_barrier();
 }
 
-// 16 bytes of LDS at byte offset `off` + the immediate O of a stage, read
-// by inline asm: the compiler cannot see that it reads LDS, so it does not
-// wait for the loads still filling the other stages (the caller waits for
-// lgkmcnt before using the result).
-template <int O>
-__device__ __forceinline__ uint4 lds_read16(uint32_t off) {
-  uint4 r;
-  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(off), "i"(O));
-  return r;
+// LDS of one wave only: the writes of all its lanes before the reads after.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-#ifndef ECF8_GEMM_BM
-#define ECF8_GEMM_BM 256
-#endif
-constexpr int kGemmBM = ECF8_GEMM_BM;        // tile rows: 2 x 64 per wave row pair
-constexpr int kGemmBN = 128;                 // tile columns
-constexpr int kGemmWaves = kGemmBM / 32;     // (BM / 64) x 2 waves of 64 x 64
-constexpr int kGemmABlocks = kGemmBM / 16, kGemmBBlocks = kGemmBN / 16;
-constexpr int kGemmStages = 3;
-// loads per wave and stage: A and B block halves, and one of scales
-constexpr int kGemmLoads = 2 * (kGemmABlocks + kGemmBBlocks) / kGemmWaves + 1;
-// one stage: A blocks, B blocks, A scales
-constexpr int kGemmStageBytes = (kGemmABlocks + kGemmBBlocks) * 2048 + kGemmBM * 4;
-static_assert(kGemmABlocks % kGemmWaves == 0 && kGemmBBlocks % kGemmWaves == 0,
-              "blocks deal evenly to the waves");
-static_assert(kGemmLoads < 64, "vmcnt immediate");
+// Waits for this wave's loads of group kg + 1; those of kg + 2 (with three
+// stages), issued later, may stay in flight.
+template <int kLoads, int kStages>
+__device__ __forceinline__ void gemm_wait_loads(int kg, int kgroups) {
+  if (kStages == 3 && kg + 2 < kgroups)
+    __builtin_amdgcn_s_waitcnt((kLoads & 15) | ((kLoads >> 4) << 14) | (0x7 << 4) | (0xF << 8));
+  else
+    __builtin_amdgcn_s_waitcnt((0x7 << 4) | (0xF << 8));  // vmcnt(0)
+}
 
-__global__ __launch_bounds__(kGemmWaves * 64) void fp8_gemm_kernel(
+// One load phase's operands from LDS: four A blocks at `a` (and, with kB,
+// four B blocks at `b`) and the A rows' scales at `sc`, read and waited for
+// in one asm block (no register is in flight past it).
+struct GemmOps {
+  u32x4 al[4], ah[4];
+  float sv[4];
+};
+__device__ __forceinline__ void gemm_read_a(uint32_t a, uint32_t sc, GemmOps &o) {
+  asm volatile(
+      "ds_read_b128 %0, %12\n"
+      "ds_read_b128 %1, %12 offset:1024\n"
+      "ds_read_b128 %2, %12 offset:2048\n"
+      "ds_read_b128 %3, %12 offset:3072\n"
+      "ds_read_b128 %4, %12 offset:4096\n"
+      "ds_read_b128 %5, %12 offset:5120\n"
+      "ds_read_b128 %6, %12 offset:6144\n"
+      "ds_read_b128 %7, %12 offset:7168\n"
+      "ds_read_b32 %8, %13\n"
+      "ds_read_b32 %9, %13 offset:64\n"
+      "ds_read_b32 %10, %13 offset:128\n"
+      "ds_read_b32 %11, %13 offset:192\n"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(o.al[0]), "=&v"(o.ah[0]), "=&v"(o.al[1]), "=&v"(o.ah[1]), "=&v"(o.al[2]),
+        "=&v"(o.ah[2]), "=&v"(o.al[3]), "=&v"(o.ah[3]), "=&v"(o.sv[0]), "=&v"(o.sv[1]),
+        "=&v"(o.sv[2]), "=&v"(o.sv[3])
+      : "v"(a), "v"(sc)
+      : "memory");
+}
+__device__ __forceinline__ void gemm_read_b(uint32_t b, u32x4 (&bl)[4], u32x4 (&bh)[4]) {
+  asm volatile(
+      "ds_read_b128 %0, %8\n"
+      "ds_read_b128 %1, %8 offset:1024\n"
+      "ds_read_b128 %2, %8 offset:2048\n"
+      "ds_read_b128 %3, %8 offset:3072\n"
+      "ds_read_b128 %4, %8 offset:4096\n"
+      "ds_read_b128 %5, %8 offset:5120\n"
+      "ds_read_b128 %6, %8 offset:6144\n"
+      "ds_read_b128 %7, %8 offset:7168\n"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(bl[0]), "=&v"(bh[0]), "=&v"(bl[1]), "=&v"(bh[1]), "=&v"(bl[2]), "=&v"(bh[2]),
+        "=&v"(bl[3]), "=&v"(bh[3])
+      : "v"(b)
+      : "memory");
+}
+
+__device__ __forceinline__ v8i join32(u32x4 lo, u32x4 hi) {
+  return __builtin_shufflevector(__builtin_bit_cast(v4i, lo), __builtin_bit_cast(v4i, hi), 0, 1, 2,
+                                 3, 4, 5, 6, 7);
+}
+
+// WM x WN = 8 waves of (64 kHalves) x 64 outputs each.
+template <int WM, int WN, int kHalves, int kStages>
+struct GemmShape {
+  static constexpr int kBM = 64 * kHalves * WM, kBN = 64 * WN;
+  static constexpr int kABlocks = kBM / 16, kBBlocks = kBN / 16;
+  static constexpr int kStageBytes = (kABlocks + kBBlocks) * 2048 + kBM * 4;
+  // loads per wave and stage: A and B block halves, and one of scales
+  static constexpr int kLoads = 2 * (kABlocks + kBBlocks) / 8 + 1;
+  static_assert(WM * WN == 8 && kABlocks % 8 == 0 && kBBlocks % 8 == 0, "blocks deal evenly");
+  static_assert(kStages * kStageBytes <= 163840 && kBM % 8 == 0 && kBM <= 512, "LDS");
+};
+
+template <int WM, int WN, int kHalves, int kStages>
+__global__ __launch_bounds__(512) void fp8_gemm_kernel(
     const uint8_t *__restrict__ aq, const float *__restrict__ as, int M, int K, LinearSegs segs,
     uint16_t *__restrict__ out, int ldo, int n_mb, int n_tiles) {
-  __shared__ __attribute__((aligned(16))) uint8_t s_ring[kGemmStages * kGemmStageBytes];
+  using Sh = GemmShape<WM, WN, kHalves, kStages>;
+  __shared__ __attribute__((aligned(16))) uint8_t s_ring[kStages * Sh::kStageBytes];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wm = wave >> 1, wn = wave & 1;
+  const int wm = wave % WM, wn = wave / WM;
   const int kgroups = K / kGroup;
 
   // tile order: XCD x = blockIdx.x % 8 takes tiles [x * per, (x + 1) * per)
@@ -299,152 +373,188 @@ __global__ __launch_bounds__(kGemmWaves * 64) void fp8_gemm_kernel(
   const int per = n_tiles / 8;
   if (tile < 8 * per) tile = (tile % 8) * per + tile / 8;
   const int mb = tile % n_mb, nb = tile / n_mb;
-  const int m0 = mb * kGemmBM;
+  const int m0 = mb * Sh::kBM;
 
-  int n0 = nb * kGemmBN;
-  const uint8_t *w = segs.w[0];
-  const float *ws = segs.ws[0];
-  int col = segs.col[0], seg_start = 0, wt = segs.tiled[0];
+  // each 128-column half of the tile lies in one segment; a wave loads
+  // blocks of, and multiplies, one half
+  auto segment = [&](int n, const uint8_t *&w, const float *&ws, int &col, int &wt) {
+    w = segs.w[0];
+    ws = segs.ws[0];
+    col = segs.col[0];
+    wt = segs.tiled[0];
+    int start = 0;
 #pragma unroll
-  for (int s = 1; s < ECF8_LINEAR_MAX_SEGS; ++s) {
-    if (s < segs.count && n0 >= segs.n_end[s - 1]) {
-      w = segs.w[s];
-      ws = segs.ws[s];
-      col = segs.col[s];
-      wt = segs.tiled[s];
-      seg_start = segs.n_end[s - 1];
+    for (int s = 1; s < ECF8_LINEAR_MAX_SEGS; ++s) {
+      if (s < segs.count && n >= segs.n_end[s - 1]) {
+        w = segs.w[s];
+        ws = segs.ws[s];
+        col = segs.col[s];
+        wt = segs.tiled[s];
+        start = segs.n_end[s - 1];
+      }
     }
-  }
-  n0 -= seg_start;
+    return n - start;
+  };
+  const int n_total = segs.n_end[segs.count - 1];
+  // loading: wave v fills B blocks v B/8 .. of the tile (columns past the
+  // last repeat its last 128)
+  constexpr int kNA = Sh::kABlocks / 8, kNB = Sh::kBBlocks / 8;
+  const uint8_t *lw;
+  const float *lws;
+  int lcol, lwt;
+  const int ln = min(nb * Sh::kBN + 16 * kNB * wave, n_total - 128 + (16 * kNB * wave) % 128);
+  const int ln0 = segment(ln, lw, lws, lcol, lwt);
+  // multiplying: the wave's 64 columns
+  const uint8_t *mw;
+  const float *mws;
+  int mcol, mwt;
+  const int mn = nb * Sh::kBN + 64 * wn;
+  const bool in = mn < n_total;
+  const int mn0 = segment(in ? mn : n_total - 64, mw, mws, mcol, mwt);
   typedef const __attribute__((address_space(4))) float ConstF;  // scalar loads
-  ConstF *const wsrow = (ConstF *)(ws + (size_t)(n0 / kGroup) * kgroups);
+  ConstF *const wsrow = (ConstF *)(mws + (size_t)(mn0 / kGroup) * kgroups);
   const int last_rb = (M + 15) / 16 - 1;  // the last 16-row block of aq
   const uint32_t ring = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)s_ring;
 
-  // loads of group kg into stage st: wave v fills A blocks v A/W.. and B
-  // blocks v B/W.. (A/W, B/W blocks per wave) and the scales of rows 32 v ..
-  // 32 v + 31 (lanes 0..31)
-  auto issue = [&](int st, int kg) {
-    uint8_t *const sa = s_ring + st * kGemmStageBytes;
-    uint8_t *const sb = sa + kGemmABlocks * 2048;
-    float *const ss = reinterpret_cast<float *>(sb + kGemmBBlocks * 2048);
-    constexpr int na = kGemmABlocks / kGemmWaves, nbk = kGemmBBlocks / kGemmWaves;
+  // group kg into its stage: A blocks, B blocks, A scales (lanes 0 .. of
+  // each wave)
+  auto issue = [&](int kg) {
+    uint8_t *const sa = s_ring + (kg % kStages) * Sh::kStageBytes;
+    uint8_t *const sb = sa + Sh::kABlocks * 2048;
+    float *const ss = reinterpret_cast<float *>(sb + Sh::kBBlocks * 2048);
 #pragma unroll
-    for (int h = 0; h < na; ++h) {
-      const int t = na * wave + h;
-      const int rb = min(m0 / 16 + t, last_rb);
-      const uint8_t *ab = aq + ((size_t)rb * kgroups + kg) * 2048;
+    for (int h = 0; h < kNA; ++h) {
+      const int t = kNA * wave + h;
+      const uint8_t *ab = aq + ((size_t)min(m0 / 16 + t, last_rb) * kgroups + kg) * 2048;
       lds_load16(ab + 16 * lane, sa + t * 2048);
       lds_load16(ab + 1024 + 16 * lane, sa + t * 2048 + 1024);
     }
 #pragma unroll
-    for (int h = 0; h < nbk; ++h) {
-      const int t = nbk * wave + h;
+    for (int h = 0; h < kNB; ++h) {
+      const int t = kNB * wave + h;
       const uint8_t *b0, *b1;
-      if (wt) {
-        const uint8_t *bb = w + ((size_t)(n0 / 16 + t) * kgroups + kg) * 2048;
+      if (lwt) {
+        const uint8_t *bb = lw + ((size_t)(ln0 / 16 + h) * kgroups + kg) * 2048;
         b0 = bb + 16 * lane;
         b1 = bb + 1024 + 16 * lane;
       } else {
-        b0 = w + (size_t)(n0 + 16 * t + (lane & 15)) * K + kg * kGroup + 16 * (lane >> 4);
+        b0 = lw + (size_t)(ln0 + 16 * h + (lane & 15)) * K + kg * kGroup + 16 * (lane >> 4);
         b1 = b0 + 64;
       }
       lds_load16(b0, sb + t * 2048);
       lds_load16(b1, sb + t * 2048 + 1024);
     }
-    if (lane < 32) {
-      const int row = min(m0 + 32 * wave + lane, M - 1);
-      lds_load4(as + (size_t)row * kgroups + kg, ss + 32 * wave);
+    constexpr int kRows = Sh::kBM / 8;  // rows of scales per wave
+    if (lane < kRows) {
+      const int row = min(m0 + kRows * wave + lane, M - 1);
+      lds_load4(as + (size_t)row * kgroups + kg, ss + kRows * wave);
     }
   };
 
-  v4f acc[4][4];
+  v4f acc[kHalves][4][4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int h = 0; h < kHalves; ++h)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[h][i][j] = v4f{0.f, 0.f, 0.f, 0.f};
 
   // the lane's LDS offsets in a stage: its A, B and scale reads
-  const uint32_t a_off = (uint32_t)(4 * wm) * 2048u + 16u * (uint32_t)lane;
-  const uint32_t b_off = (uint32_t)(kGemmABlocks + 4 * wn) * 2048u + 16u * (uint32_t)lane;
-  const uint32_t s_off =
-      (uint32_t)(kGemmABlocks + kGemmBBlocks) * 2048u + 4u * (64u * wm + 4u * (lane >> 4));
+  const uint32_t a_off = ring + (uint32_t)(4 * kHalves * wm) * 2048u + 16u * (uint32_t)lane;
+  const uint32_t b_off = ring + (uint32_t)(Sh::kABlocks + 4 * wn) * 2048u + 16u * (uint32_t)lane;
+  const uint32_t s_off = ring + (uint32_t)(Sh::kABlocks + Sh::kBBlocks) * 2048u +
+                         4u * (uint32_t)(64 * kHalves * wm + (lane & 15));
 
-  issue(0, 0);
-  if (kgroups > 1) issue(1, 1);
-  for (int kg = 0; kg < kgroups; ++kg) {
-    const int st = kg % kGemmStages;
-    // this stage's loads are done unless it is the last: the next one's
-    // kGemmLoads may stay in flight
-    if (kg + 1 < kgroups)
-      __builtin_amdgcn_s_waitcnt((kGemmLoads & 15) | ((kGemmLoads >> 4) << 14) | (0x7 << 4) |
-                                 (0xF << 8));
-    else
-      __builtin_amdgcn_s_waitcnt((0x7 << 4) | (0xF << 8));  // vmcnt(0)
-    // every wave's loads of stage st are in LDS, and every wave is done
-    // reading the stage refilled below (read in the previous step)
-    gemm_barrier();
-    const uint32_t base = ring + (uint32_t)st * kGemmStageBytes;
-    uint4 al[4], ah[4], bl[4], bh[4], sv[4];
-    al[0] = lds_read16<0>(base + a_off);
-    ah[0] = lds_read16<1024>(base + a_off);
-    al[1] = lds_read16<2048>(base + a_off);
-    ah[1] = lds_read16<3072>(base + a_off);
-    al[2] = lds_read16<4096>(base + a_off);
-    ah[2] = lds_read16<5120>(base + a_off);
-    al[3] = lds_read16<6144>(base + a_off);
-    ah[3] = lds_read16<7168>(base + a_off);
-    bl[0] = lds_read16<0>(base + b_off);
-    bh[0] = lds_read16<1024>(base + b_off);
-    bl[1] = lds_read16<2048>(base + b_off);
-    bh[1] = lds_read16<3072>(base + b_off);
-    bl[2] = lds_read16<4096>(base + b_off);
-    bh[2] = lds_read16<5120>(base + b_off);
-    bl[3] = lds_read16<6144>(base + b_off);
-    bh[3] = lds_read16<7168>(base + b_off);
-    sv[0] = lds_read16<0>(base + s_off);
-    sv[1] = lds_read16<64>(base + s_off);
-    sv[2] = lds_read16<128>(base + s_off);
-    sv[3] = lds_read16<192>(base + s_off);
-    const float sw = wsrow[kg];
-    __builtin_amdgcn_s_waitcnt((0x3F & 15) | (0x3 << 14) | (0x7 << 4) | (0x0 << 8));  // lgkmcnt(0)
-    // the stage read in the previous step is free: group kg + 2 goes there
-    if (kg + 2 < kgroups) issue((kg + 2) % kGemmStages, kg + 2);
-    v8i a[4], b[4];
-    v4f c[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      a[i] = v8i{(int)al[i].x, (int)al[i].y, (int)al[i].z, (int)al[i].w,
-                 (int)ah[i].x, (int)ah[i].y, (int)ah[i].z, (int)ah[i].w};
-      b[i] = v8i{(int)bl[i].x, (int)bl[i].y, (int)bl[i].z, (int)bl[i].w,
-                 (int)bh[i].x, (int)bh[i].y, (int)bh[i].z, (int)bh[i].w};
-      c[i] = v4f{__uint_as_float(sv[i].x) * sw, __uint_as_float(sv[i].y) * sw,
-                 __uint_as_float(sv[i].z) * sw, __uint_as_float(sv[i].w) * sw};
+  for (int s = 0; s < kStages - 1; ++s)
+    if (s < kgroups) issue(s);
+  gemm_wait_loads<Sh::kLoads, kStages>(-1, kgroups);
+  gemm_barrier();
+  if (wave >= 4) gemm_barrier();  // the second four waves run one phase behind
+  u32x4 bl[4], bh[4];
+  for (int kg = 0; kg < kgroups; ++kg) {
+    const uint32_t base = (uint32_t)(kg % kStages) * Sh::kStageBytes;
+    const float sw = wsrow[kg];
+#pragma unroll
+    for (int h = 0; h < kHalves; ++h) {
+      // load phase (the other four waves multiply)
+      GemmOps o;
+      if (h == 0) {
+        gemm_read_b(base + b_off, bl, bh);
+      }
+      gemm_read_a(base + a_off + 8192u * h, base + s_off + 256u * h, o);
+      // the stage read in the group before is free: both halves of the waves
+      // have passed their last load phase of it
+      if (h == 0 && kg + kStages - 1 < kgroups) issue(kg + kStages - 1);
+      // before the other four waves' first load phase of the next group, and
+      // (below) before this wave's: its own loads of that group are in LDS
+      if (h == kHalves - 1 && wave >= 4) gemm_wait_loads<Sh::kLoads, kStages>(kg, kgroups);
+      gemm_barrier();
+      // multiply phase (the other four waves load)
+      // product n, then the sums of product n - 2, which is done by then
+      // (the empty asm holds the compiler to this order: with all 16
+      // products first, 64 registers more are live)
+      v4f d[3];
+#pragma unroll
+      for (int n = 0; n < 18; ++n) {
+        if (n < 16) {
+          const v4f z = {0.f, 0.f, 0.f, 0.f};
+          // scale operands 0: the unscaled e4m3 x e4m3 form
+          d[n % 3] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+              join32(bl[n % 4], bh[n % 4]), join32(o.al[n / 4], o.ah[n / 4]), z, 0, 0, 0, 0, 0, 0);
+        }
+        if (n >= 2) {
+          const int i = (n - 2) / 4, j = (n - 2) % 4;
+          if (j == 0) o.sv[i] *= sw;
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            acc[h][i][j][q] = fmaf(d[(n - 2) % 3][q], o.sv[i], acc[h][i][j][q]);
+          asm volatile("" : "+v"(acc[h][i][j]));
+        }
+      }
+      if (h == kHalves - 1 && wave < 4) gemm_wait_loads<Sh::kLoads, kStages>(kg, kgroups);
+      gemm_barrier();
     }
+  }
+  if (wave < 4) gemm_barrier();
+  if (!in) return;
+  // Lane: columns 4 (l / 16) .. + 3 of each 16 x 16 tile, row l % 16.  Every
+  // wave is done with the ring (the last barrier): through its own part of
+  // it to whole lines, 64 rows of 128 bytes (+ 16: no bank conflicts) at a
+  // time.  K = 896, 2048 rows, N = 12288: 40.2 us, with the lanes' own 8-byte
+  // stores 47.5.
+  const bool whole =
+      (((uintptr_t)out | 2u * (uintptr_t)(uint32_t)ldo | 2u * (uintptr_t)(uint32_t)mcol) & 15) == 0;
+  constexpr int kRow = 144;
+  static_assert(8 * 64 * kRow <= kStages * Sh::kStageBytes, "output tiles fit the ring");
+  uint8_t *const st = s_ring + wave * (64 * kRow);
+#pragma unroll
+  for (int h = 0; h < kHalves; ++h) {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const v4f z = {0.f, 0.f, 0.f, 0.f};
-        // scale operands 0: the unscaled e4m3 x e4m3 form
-        const v4f d = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a[i], b[j], z, 0, 0, 0, 0,
-                                                                        0, 0);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) acc[i][j][q] = fmaf(d[q], c[i][q], acc[i][j][q]);
+        const v4f &c = acc[h][i][j];
+        *reinterpret_cast<u32x2 *>(st + (16 * i + (lane & 15)) * kRow + 32 * j + 8 * (lane >> 4)) =
+            u32x2{pack_bf16(c[0], c[1]), pack_bf16(c[2], c[3])};
       }
-  }
-
+    wave_sync();
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int m = m0 + 64 * wm + 16 * i + 4 * (lane >> 4) + q;
+    for (int t = 0; t < 8; ++t) {
+      const int row = 8 * t + (lane >> 3), m = m0 + 64 * kHalves * wm + 64 * h + row;
+      const u32x4 v = *reinterpret_cast<const u32x4 *>(st + row * kRow + 16 * (lane & 7));
       if (m < M) {
-        uint16_t *o = out + (size_t)m * ldo + col + n0 + 64 * wn + (lane & 15);
+        uint16_t *o = out + (size_t)m * ldo + mcol + mn0 + 8 * (lane & 7);
+        if (whole) {
+          *reinterpret_cast<u32x4 *>(o) = v;
+        } else {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) o[16 * j] = (uint16_t)f32_bf16(acc[i][j][q]);
+          for (int q = 0; q < 8; ++q) o[q] = (uint16_t)(v[q / 2] >> (16 * (q & 1)));
+        }
       }
     }
+    wave_sync();
+  }
 }
 
 // ------------------------------------------ middle form (16 < M, few tiles)
@@ -458,8 +568,6 @@ __global__ __launch_bounds__(kGemmWaves * 64) void fp8_gemm_kernel(
 // number of workgroups against re-reading the activations per column strip
 // (from L2).  HBM or L2 bounds it; MI355X, 64 rows: N = K = 4096 34.8 -> 8.9
 // us, N = 4096, K = 12288 94 -> 20 us.
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
 template <int P, int kCh>
 __global__ __launch_bounds__(512) void fp8_rows_kernel(const uint8_t *__restrict__ aq,
                                                        const float *__restrict__ as, int M, int K,
@@ -1984,11 +2092,19 @@ extern "C" int ecf8_fp8_linear(const void *aq, const float *as, int64_t M, int64
 #undef ECF8_ROWS
       return launched();
     }
-    const int n_mb = (int)((M + kGemmBM - 1) / kGemmBM);
-    const int64_t n_tiles = (n_total / kGemmBN) * n_mb;
-    if (n_tiles > INT32_MAX) return ECF8_ERR_UNSUPPORTED;
-    fp8_gemm_kernel<<<(unsigned)n_tiles, kGemmWaves * 64, 0, as_stream(stream)>>>(
-        a, as, (int)M, (int)K, s, o, (int)ldo, n_mb, (int)n_tiles);
+    // 256 x 256 tiles where they need fewer rounds of workgroups even at
+    // 1.75 times the time of a 256 x 128 tile.  MI355X, K = 4096, M = 2048,
+    // us, wide against slim: N = 24576 (3 rounds and 6) 227 and 257, N = 6144
+    // (1 and 2) 72 and 80, N = 4096 (1 and 1) 67 and 45.
+    const int n_mb = (int)((M + 255) / 256);
+    const int64_t wide = n_mb * ((n_total + 255) / 256), slim = n_mb * (n_total / 128);
+    if (slim > INT32_MAX) return ECF8_ERR_UNSUPPORTED;
+    if (7 * ((wide + cus - 1) / cus) < 4 * ((slim + cus - 1) / cus))
+      fp8_gemm_kernel<2, 4, 2, 2><<<(unsigned)wide, 512, 0, as_stream(stream)>>>(
+          a, as, (int)M, (int)K, s, o, (int)ldo, n_mb, (int)wide);
+    else
+      fp8_gemm_kernel<4, 2, 1, 3><<<(unsigned)slim, 512, 0, as_stream(stream)>>>(
+          a, as, (int)M, (int)K, s, o, (int)ldo, n_mb, (int)slim);
   }
   return launched();
 }

@@ -229,6 +229,40 @@ def test_fp8_linear_many_rows_either_form(cuda_device, M, shapes, Kd, layout):
     assert bool((out[:, N:] == 7.0).all()) and bool((out[M:] == 7.0).all())
 
 
+@pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("M,extra,Kd,ldo", [
+    (257, (), 128, 0), (300, (128,), 256, 0), (511, (128, 128), 896, 1), (512, (256, 128), 1152, 2),
+    (1024, (384,), 128, 4), (2048, (128,), 640, 0),
+])
+def test_fp8_linear_wide_tiles(cuda_device, M, extra, Kd, ldo, layout):
+    """256 x 256 tiles (more 256 x 128 tiles than CUs, up to as many wide
+    ones): segments that end in the middle of a tile, a half-empty last one,
+    1, 2 and more K groups, partial rows; row strides of 1, 2 and 4 columns
+    more take stores of 2 bytes instead of 16."""
+    from ecf8_amd.llm_kernels import LinearPlan
+
+    cus = torch.cuda.get_device_properties(cuda_device).multi_processor_count
+    rows = -(-M // 256)
+    shapes = (128 * (cus // rows + 1), *extra)
+    assert rows * sum(shapes) // 128 > cus >= rows * -(-sum(shapes) // 256)
+    gen = torch.Generator().manual_seed(M + Kd)
+    aq = _rand_fp8((M, Kd), gen, cuda_device)
+    a_s = (torch.rand(M, Kd // 128, generator=gen) * 1e-2 + 1e-4).to(cuda_device)
+    segs = [(_rand_fp8((n, Kd), gen, cuda_device),
+             (torch.rand(n // 128, Kd // 128, generator=gen) * 1e-3 + 1e-5).to(cuda_device))
+            for n in shapes]
+    N = sum(shapes)
+    out = torch.full((M + 1, N + ldo), 7.0, dtype=torch.bfloat16, device=cuda_device)
+    LinearPlan([(to_tiles(w), ws, 1) if layout else (w, ws) for w, ws in segs], out)(
+        to_tiles(aq), a_s, M)
+    a = (aq.double().view(M, Kd // 128, 128) * a_s.double()[:, :, None]).view(M, Kd)
+    ref = torch.cat([a @ (w.double().view(-1, 128, Kd // 128, 128)
+                          * ws.double()[:, None, :, None]).view(-1, Kd).t() for w, ws in segs], 1)
+    tol = 2 ** -7 * ref.abs() + 1e-4 * ref.abs().max()  # bf16 output, as above
+    assert bool(((out[:M, :N].double() - ref).abs() <= tol).all())
+    assert bool((out[:, N:] == 7.0).all()) and bool((out[M:] == 7.0).all())
+
+
 def test_fp8_linear_persistent_path_matches_fp64(cuda_device):
     """More 16-column tiles than one workgroup per CU at K = 4096 (the
     gate/up shape) takes the persistent kernel that keeps the activations
