@@ -69,30 +69,39 @@ __device__ __forceinline__ uint32_t f32_bf16(float f) {
   return u >> 16;
 }
 
-// fp32 -> e4m3fn, round to nearest even; |y| is clamped to 448 first, so
-// the result is always finite (callers pass values already scaled into
-// range).  Subnormals (|y| < 2^-6) have a step of 2^-9.
-__device__ __forceinline__ uint32_t f32_e4m3(float y) {
-  const uint32_t sign = (__float_as_uint(y) >> 24) & 0x80u;
-  const float a = fminf(fabsf(y), kFp8Max);
-  uint32_t code;
-  if (a < 0.015625f) {
-    code = (uint32_t)rintf(a * 512.f);  // 0..8; 8 is the smallest normal
-  } else {
-    const uint32_t b = __float_as_uint(a);
-    const uint32_t e = (b >> 23) - 120u;  // biased e4m3 exponent (bias 7)
-    const uint32_t m = b & 0x7fffffu;
-    uint32_t q = m >> 20;
-    const uint32_t rem = m & 0xfffffu;
-    q += (rem > 0x80000u) || (rem == 0x80000u && (q & 1u));
-    code = (e << 3) + q;  // a mantissa carry moves into the exponent
-  }
-  return sign | code;
+// Four fp32 -> four e4m3fn codes, round to nearest even, with the signs of
+// sg; |y| is clamped to 448 first (so is a NaN), the result is always finite
+// (callers pass values already scaled into range).  Subnormals (|y| < 2^-6)
+// have a step of 2^-9.  The hardware conversion, the same code for every
+// fp32 pattern as clamping and rounding the bits by hand.
+__device__ __forceinline__ uint32_t f32_e4m3x4(const float (&y)[4], const float (&sg)[4]) {
+  float c[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) c[i] = copysignf(fminf(fabsf(y[i]), kFp8Max), sg[i]);
+  const int lo = __builtin_amdgcn_cvt_pk_fp8_f32(c[0], c[1], 0, false);
+  return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(c[2], c[3], lo, true);
 }
 
+// Sum over the wave, in every lane: halves, then 16, 8, 4, 2, 1 lanes apart,
+// without LDS shuffles (after each step the values repeat with half the
+// period, so a row rotation brings the same partner as an exclusive-or).
 __device__ __forceinline__ float wave_sum(float v) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return __shfl(v, 0);  // every lane takes lane 0's association order
+  auto swap = [](uint32_t a, bool half) {
+    const auto u = half ? __builtin_amdgcn_permlane32_swap(a, a, false, false)
+                        : __builtin_amdgcn_permlane16_swap(a, a, false, false);
+    return __uint_as_float(u[0]) + __uint_as_float(u[1]);
+  };
+  v = swap(__float_as_uint(v), true);
+  v = swap(__float_as_uint(v), false);
+#define ECF8_DPP_ADD(ctrl)                                                                 \
+  v += __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), ctrl, \
+                                                             0xF, 0xF, true))
+  ECF8_DPP_ADD(0x128);  // row_ror:8
+  ECF8_DPP_ADD(0x124);  // row_ror:4
+  ECF8_DPP_ADD(0x4E);   // quad_perm 2, 3, 0, 1
+  ECF8_DPP_ADD(0xB1);   // quad_perm 1, 0, 3, 2
+#undef ECF8_DPP_ADD
+  return v;
 }
 
 __device__ __forceinline__ float wave_max(float v) {
@@ -129,11 +138,30 @@ __device__ __forceinline__ void quant16(const float (&v)[16], uint8_t *q_out, fl
   amax = fmaxf(amax, __shfl_xor(amax, 2));
   amax = fmaxf(amax, __shfl_xor(amax, 4));
   const float s = amax > 0.f ? amax / kFp8Max : 1.f;
+  // v / s, correctly rounded: with r = 1 / s correctly rounded and a quotient
+  // within an ulp (q after one correction), q + r (v - q s) is (Markstein
+  // 1990); s in this range keeps every quotient of 2^-11 or more (smaller
+  // ones round to 0) and its remainder normal.  A zero's sign is lost on the
+  // way and taken from v.
+  const bool plain = s >= 0x1p-60f && s <= 0x1p60f;
+  const float r = 1.f / s;
   uint32_t w[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    w[j] = f32_e4m3(v[4 * j] / s) | (f32_e4m3(v[4 * j + 1] / s) << 8) |
-           (f32_e4m3(v[4 * j + 2] / s) << 16) | (f32_e4m3(v[4 * j + 3] / s) << 24);
+    float q[4], sg[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float x = v[4 * j + i];
+      if (plain) {
+        q[i] = x * r;
+        q[i] = fmaf(fmaf(-q[i], s, x), r, q[i]);
+        q[i] = fmaf(fmaf(-q[i], s, x), r, q[i]);
+        sg[i] = x;
+      } else {
+        q[i] = sg[i] = x / s;
+      }
+    }
+    w[j] = f32_e4m3x4(q, sg);
   }
   *reinterpret_cast<uint4 *>(q_out) = make_uint4(w[0], w[1], w[2], w[3]);
   if (first_of_group) *s_out = s;
@@ -1057,52 +1085,64 @@ __device__ __forceinline__ uint32_t norm_rope(uint32_t x2, const RopeIn &in, flo
   const float rs = rsqrtf(ss / (float)kHeadDim + eps);
   x0 = x0 * rs * bf16_f32(in.w2 & 0xffffu);
   x1 = x1 * rs * bf16_f32(in.w2 >> 16);
-  const float y0 = __shfl_xor(x0, 32), y1 = __shfl_xor(x1, 32);  // dims d +- 64
+  // dims d +- 64 lie in the other half of the wave
+  const auto s0 = __builtin_amdgcn_permlane32_swap(__float_as_uint(x0), __float_as_uint(x0), false,
+                                                   false);
+  const auto s1 = __builtin_amdgcn_permlane32_swap(__float_as_uint(x1), __float_as_uint(x1), false,
+                                                   false);
+  const float y0 = __uint_as_float(lane < 32 ? s0[1] : s0[0]);
+  const float y1 = __uint_as_float(lane < 32 ? s1[1] : s1[0]);
   const float sg = lane < 32 ? -1.f : 1.f;
   x0 = x0 * in.c.x + sg * y0 * in.s.x;
   x1 = x1 * in.c.y + sg * y1 * in.s.y;
   return f32_bf16(x0) | (f32_bf16(x1) << 16);
 }
 
-__device__ __forceinline__ uint32_t norm_rope_pair(uint32_t x2, const uint16_t *__restrict__ nw,
-                                                   float eps, const float *__restrict__ cosv,
-                                                   const float *__restrict__ sinv, int p,
-                                                   int lane) {
-  return norm_rope(x2, rope_load(nw, cosv, sinv, p, lane), eps, lane);
-}
-
-// One wave per (token, head) of the fused qkv projection output
-// [B*T, (Hq + 2 Hkv) * 128]: q and k heads get RMSNorm over the head
-// (weights qn / kn) and the rotary embedding at position pos[0] + t
-// (rotate-half convention, cos/sin tables [Lmax, 64]); q goes to
-// q_out [B, Hq, T, 128], k and v to the caches [B, Hkv, Lmax, 128].
+// The heads of the fused qkv projection output [B*T, (Hq + 2 Hkv) * 128]: q
+// and k heads get RMSNorm over the head (weights qn / kn) and the rotary
+// embedding at position pos[0] + t (rotate-half convention, cos/sin tables
+// [Lmax, 64]); q goes to q_out [B, Hq, T, 128], k and v to the caches
+// [B, Hkv, Lmax, 128].  Workgroup (token, 16 heads), four heads per wave, all
+// loaded at once and sharing the token's rotary values.  HBM bounds it
+// (50 MB at 2048 tokens of 48 heads: @QK us; one head per wave 28.8).
+constexpr int kRopePer = 4;
 __global__ __launch_bounds__(256) void qk_norm_rope_kernel(
     const uint16_t *__restrict__ qkv, int T, int Hq, int Hkv, const uint16_t *__restrict__ qn,
     const uint16_t *__restrict__ kn, float eps, const float *__restrict__ cosv,
     const float *__restrict__ sinv, const int *__restrict__ pos, int Lmax,
-    uint16_t *__restrict__ q_out, uint16_t *__restrict__ kc, uint16_t *__restrict__ vc,
-    int n_items) {
+    uint16_t *__restrict__ q_out, uint16_t *__restrict__ kc, uint16_t *__restrict__ vc) {
   const int lane = threadIdx.x & 63;
-  const int item = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (item >= n_items) return;
   const int H = Hq + 2 * Hkv;
-  const int tok = item / H, hh = item % H;
-  const int b = tok / T, t = tok % T;
+  const int n_hb = (H + 4 * kRopePer - 1) / (4 * kRopePer);
+  const int tok = (int)blockIdx.x / n_hb, b = tok / T, t = tok % T;
+  const int h0 = ((int)blockIdx.x % n_hb * 4 +
+                  __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6)) * kRopePer;
+  if (h0 >= H) return;
   const int p = pos[0] + t;
   if (p < 0 || p >= Lmax) return;
-  const uint32_t x2 = *reinterpret_cast<const uint32_t *>(qkv + (size_t)tok * H * kHeadDim +
-                                                          hh * kHeadDim + 2 * lane);
-  const uint32_t outw =
-      hh >= Hq + Hkv ? x2 : norm_rope_pair(x2, hh < Hq ? qn : kn, eps, cosv, sinv, p, lane);
-  uint16_t *dst;
-  if (hh < Hq) {
-    dst = q_out + (((size_t)b * Hq + hh) * T + t) * kHeadDim;
-  } else if (hh < Hq + Hkv) {
-    dst = kc + (((size_t)b * Hkv + (hh - Hq)) * Lmax + p) * kHeadDim;
-  } else {
-    dst = vc + (((size_t)b * Hkv + (hh - Hq - Hkv)) * Lmax + p) * kHeadDim;
+  uint32_t x2[kRopePer];
+#pragma unroll
+  for (int i = 0; i < kRopePer; ++i)
+    x2[i] = *reinterpret_cast<const uint32_t *>(
+        qkv + ((size_t)tok * H + min(h0 + i, H - 1)) * kHeadDim + 2 * lane);
+  RopeIn in = rope_load(h0 < Hq ? qn : kn, cosv, sinv, p, lane);
+  const uint32_t wk = *reinterpret_cast<const uint32_t *>(kn + 2 * lane);
+#pragma unroll
+  for (int i = 0; i < kRopePer; ++i) {
+    const int hh = h0 + i;
+    if (hh >= H) break;
+    uint16_t *dst;
+    if (hh < Hq) {
+      dst = q_out + (((size_t)b * Hq + hh) * T + t) * kHeadDim;
+    } else if (hh < Hq + Hkv) {
+      in.w2 = wk;
+      dst = kc + (((size_t)b * Hkv + (hh - Hq)) * Lmax + p) * kHeadDim;
+    } else {
+      dst = vc + (((size_t)b * Hkv + (hh - Hq - Hkv)) * Lmax + p) * kHeadDim;
+    }
+    *reinterpret_cast<uint32_t *>(dst + 2 * lane) =
+        hh >= Hq + Hkv ? x2[i] : norm_rope(x2[i], in, eps, lane);
   }
-  *reinterpret_cast<uint32_t *>(dst + 2 * lane) = outw;
 }
 
 // ------------------------------------------------------ decode attention
@@ -1114,29 +1154,6 @@ struct AttnFused {
   float eps;
   const float *cosv, *sinv;
 };
-
-// Sum over the wave in the association of wave_sum (lane 0's: halves, then
-// 16, 8, 4, 2, 1 lanes apart), in every lane, without LDS shuffles: after
-// each step the values repeat with half the period, so a row rotation
-// brings the same partner as an exclusive-or.
-__device__ __forceinline__ float wave_sum_dpp(float v) {
-  auto swap = [](uint32_t a, bool half) {
-    const auto u = half ? __builtin_amdgcn_permlane32_swap(a, a, false, false)
-                        : __builtin_amdgcn_permlane16_swap(a, a, false, false);
-    return __uint_as_float(u[0]) + __uint_as_float(u[1]);
-  };
-  v = swap(__float_as_uint(v), true);
-  v = swap(__float_as_uint(v), false);
-#define ECF8_DPP_ADD(ctrl)                                                                 \
-  v += __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), ctrl, \
-                                                             0xF, 0xF, true))
-  ECF8_DPP_ADD(0x128);  // row_ror:8
-  ECF8_DPP_ADD(0x124);  // row_ror:4
-  ECF8_DPP_ADD(0x4E);   // quad_perm 2, 3, 0, 1
-  ECF8_DPP_ADD(0xB1);   // quad_perm 1, 0, 3, 2
-#undef ECF8_DPP_ADD
-  return v;
-}
 
 // Rows (16 lanes) 0..3 of x and y -> rows x0 + x1, y0 + y1, x2 + x3, y2 + y3.
 __device__ __forceinline__ float add_swap16(float x, float y) {
@@ -1325,7 +1342,7 @@ __global__ __launch_bounds__(64 * kAttnWaves) void attn_split_kernel(
     const float mh = fmaxf(fmaxf(rm[0], rm[1]), fmaxf(rm[2], rm[3]));
     const float e = valid ? expf(s[h] - mh) : 0.f;
     pw[half * kH + h][pg][16 * (lane & 3) + (lane >> 2)] = e;
-    const float sw = wave_sum_dpp(e);
+    const float sw = wave_sum(e);
     if (lane == 0) red[1][half * kH + h][pg] = sw;
   }
   lds_barrier();
@@ -1432,7 +1449,8 @@ __global__ __launch_bounds__(64) void attn_combine_kernel(const float *__restric
   if (ob) reinterpret_cast<uint32_t *>(ob)[bh * 64 + lane] = f32_bf16(a0) | (f32_bf16(a1) << 16);
   const float amax = wave_max_dpp(fmaxf(fabsf(a0), fabsf(a1)));
   const float sc = amax > 0.f ? amax / kFp8Max : 1.f;
-  const uint32_t q2 = f32_e4m3(a0 / sc) | (f32_e4m3(a1 / sc) << 8);
+  const float qs[4] = {a0 / sc, a1 / sc, 0.f, 0.f};
+  const uint32_t q2 = f32_e4m3x4(qs, qs);
   // row b = bh / Hq, group = head: bytes 2 lane, 2 lane + 1 of the group
   const int b = (int)(bh / (size_t)Hq), head = (int)(bh % (size_t)Hq);
   *reinterpret_cast<uint16_t *>(oq + tile_chunk_off(b, head, Hq, lane >> 3) + 2 * (lane & 7)) =
@@ -2164,11 +2182,13 @@ extern "C" int ecf8_qk_norm_rope(const void *qkv, int64_t B, int64_t T, int Hq, 
   if (!aligned(qkv, 4) || !aligned(q_norm, 4) || !aligned(k_norm, 4) || !aligned(q_out, 4) ||
       !aligned(k_cache, 4) || !aligned(v_cache, 4))
     return ECF8_ERR_MISALIGNED;
-  qk_norm_rope_kernel<<<(unsigned)((items + 3) / 4), 256, 0, as_stream(stream)>>>(
+  const int64_t per = 4 * kRopePer;  // heads per workgroup
+  const int64_t blocks = B * T * ((Hq + 2 * Hkv + per - 1) / per);
+  qk_norm_rope_kernel<<<(unsigned)blocks, 256, 0, as_stream(stream)>>>(
       static_cast<const uint16_t *>(qkv), (int)T, Hq, Hkv, static_cast<const uint16_t *>(q_norm),
       static_cast<const uint16_t *>(k_norm), eps, cos_t, sin_t, pos, (int)Lmax,
       static_cast<uint16_t *>(q_out), static_cast<uint16_t *>(k_cache),
-      static_cast<uint16_t *>(v_cache), (int)items);
+      static_cast<uint16_t *>(v_cache));
   return launched();
 }
 

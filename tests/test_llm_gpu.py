@@ -122,6 +122,46 @@ def test_act_quant_rows_of_any_group_multiple(cuda_device, Kd):
     assert bool((flat[16 * Kd:].cpu() == 0x11).all())
 
 
+@pytest.mark.parametrize("exponents", [(-126, 127), (-70, -50), (50, 70), (-20, 20)])
+def test_act_quant_bytes_over_the_exponent_range(cuda_device, exponents):
+    """Byte for byte the clamped cast of the fp32 quotient: groups whose
+    scale is inside, outside and at the ends of the range of the short
+    division, signed zeros, products that round at ties, infinities and NaN
+    (clamped to 448; the sign of inf / inf is not defined)."""
+    from ecf8_amd.llm_kernels import act_quant
+
+    lo, hi = exponents
+    gen = torch.Generator().manual_seed(hi)
+    M, Kd = 64, 2048
+    e = torch.randint(lo, hi + 1, (M, Kd // 128, 1), generator=gen).double()
+    x = (1 + torch.randint(0, 128, (M, Kd // 128, 128), generator=gen) / 128) * torch.exp2(
+        e - torch.randint(0, 20, (M, Kd // 128, 128), generator=gen))
+    x = x * (torch.randint(0, 2, x.shape, generator=gen) * 2 - 1)
+    x[0, :, ::3] = 0.0
+    x[1, :, ::3] = -0.0
+    x[2, ::2, 5] = float("inf")
+    x[3, ::2, 7] = float("nan")
+    # the largest of a group 448 x 2^n: every code and every tie is a value
+    ties = torch.cat([torch.arange(1, 32) / 1024, torch.arange(17, 64) / 32, torch.arange(1, 51) * 8])
+    x[4, :, 0], x[4, :, 1:1 + ties.numel() - 1] = 448 * torch.exp2(e[4, :, 0] - 8), (
+        ties[:-1] * torch.exp2(e[4] - 8))
+    x = x.view(M, Kd).to(torch.bfloat16)
+    q = torch.empty(pad16(M), Kd, dtype=FP8, device=cuda_device)
+    s = torch.empty(M, Kd // 128, device=cuda_device)
+    act_quant(x.to(cuda_device), M, q, s)
+    g = x.float().view(M, Kd // 128, 128)
+    amax = g.abs().nan_to_num(nan=0.0, posinf=float("inf")).amax(-1)
+    sr = torch.where(amax > 0, amax / 448.0, torch.ones_like(amax))
+    y = g / sr[:, :, None]
+    y = torch.where(y.isnan(), torch.full_like(y, 448.0).copysign(g), y.clamp(-448.0, 448.0))
+    ref = y.to(FP8).view(torch.uint8).view(M, Kd)
+    got = from_tiles(q, M, Kd).cpu().view(torch.uint8)
+    assert torch.equal(s.cpu(), sr)
+    free = (g.isinf() & sr.isinf()[:, :, None]).view(M, Kd)
+    assert torch.equal(got[~free], ref[~free])
+    assert bool(((got[free] & 0x7F) == 0x7E).all())
+
+
 # ------------------------------------------------------------ FP8 linear
 
 
