@@ -54,7 +54,7 @@ __global__ __launch_bounds__(kWaves * 64) void bf16_rows_kernel(
   const int p0 = (int)((int64_t)panels * blockIdx.x / gridDim.x);
   const int p1 = (int)((int64_t)panels * (blockIdx.x + 1) / gridDim.x);
 
-  // steps past K's end load the last one again; x is zero there
+  // steps past K's end load the last one again, unused
   u32x4 xf[kS], next[kS];
   auto load = [&](int pn, u32x4 (&v)[kS]) {
     const uint16_t *row = w + (size_t)(16 * pn + r) * K + 8 * g;
@@ -78,9 +78,11 @@ __global__ __launch_bounds__(kWaves * 64) void bf16_rows_kernel(
     if (panel + 1 < p1) load(panel + 1, next);
     v4f acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int u = 0; u < kS; ++u)
+    for (int u = 0; u < kS; ++u) {
+      if (wave * kS + u > last) break;  // uniform: zero times an infinite weight is not zero
       acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, xf[u]),
                                                     __builtin_bit_cast(v8bf, cur[u]), acc, 0, 0, 0);
+    }
     const int buf = panel & 1;
 #pragma unroll
     for (int i = 0; i < 4; ++i) s_red[buf][wave][i][lane] = acc[i];
@@ -124,7 +126,7 @@ __device__ __forceinline__ uint64_t wave_max64(uint64_t v) {
 // Best key of each of `chunks` runs of a row's logits (bf16; `vec`: rows are
 // 16-byte aligned, 8 per load): 64
 // workgroups a row and a small second kernel where the library's reduction
-// took 57 us for 16 rows of 151936 (@ARGFIG both).
+// took 57 us for 16 rows of 151936 (9 us both).
 __global__ __launch_bounds__(256) void argmax_chunk_kernel(const uint16_t *__restrict__ logits,
                                                            int64_t ld, int V, int chunks,
                                                            int vec, uint64_t *__restrict__ keys) {

@@ -33,6 +33,20 @@ def test_small_linear_matches_fp64(cuda_device, M, N, K, bias):
     assert bool(((got - want).abs() <= want.abs() * 2.0 ** -8 * 1.01 + norms * K * 2.0 ** -24).all())
 
 
+@pytest.mark.parametrize("K", [32, 96, 1056, 2048])
+def test_small_linear_keeps_infinities(cuda_device, K):
+    """An infinite weight or input in the last step of K: no step past K
+    turns it into a NaN."""
+    from ecf8_amd.head_kernels import small_linear
+
+    x, w = _rand((3, K), 5, cuda_device), _rand((32, K), 6, cuda_device)
+    x[:, -1] = 2.0
+    w[7, -1], w[9, -1] = float("inf"), float("-inf")
+    got = small_linear(x, w)
+    assert bool((got[:, 7] == float("inf")).all()) and bool((got[:, 9] == float("-inf")).all())
+    assert not bool(got.isnan().any())
+
+
 def test_small_linear_leaves_the_rest_to_the_library(cuda_device, monkeypatch):
     """Rows past 16, K or N off its steps, other dtypes, autocast: the
     library's result; autograd through the kernel: the library's gradients."""
