@@ -5,14 +5,22 @@ from __future__ import annotations
 
 import torch
 from torch.autograd import forward_ad
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 
+def _function_modes() -> bool:
+    return bool(torch._C._len_torch_function_stack()) and not all(
+        type(m) is DeviceContext for m in _get_current_function_mode_stack())
+
+
 def untracked() -> bool:
-    """No tracer, dispatch mode, dual level or autocast region is active."""
+    """No tracer, dispatch or function mode (but a default device), dual level
+    or autocast region is active."""
     return not (torch._C._len_torch_dispatch_stack() or forward_ad._current_level >= 0
-                or torch.is_autocast_enabled("cuda") or torch.jit.is_tracing()
+                or _function_modes() or torch.is_autocast_enabled("cuda") or torch.jit.is_tracing()
                 or torch.compiler.is_compiling())
 
 
@@ -28,8 +36,9 @@ def takes(tensors, dtype=torch.bfloat16, grad=False) -> bool:
 
 
 def bare(mod, cls) -> bool:
-    """``mod`` is exactly a ``cls`` without hooks, so its forward may be
-    computed without calling it."""
-    return (type(mod) is cls and not torch.nn.modules.module._has_any_global_hook()
+    """``mod`` is exactly a ``cls`` without hooks or a forward of its own, so
+    its forward may be computed without calling it."""
+    return (type(mod) is cls and "forward" not in mod.__dict__
+            and not torch.nn.modules.module._has_any_global_hook()
             and not (mod._forward_hooks or mod._forward_pre_hooks or mod._backward_hooks
                      or mod._backward_pre_hooks))

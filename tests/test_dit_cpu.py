@@ -55,3 +55,26 @@ def test_kernels_refuse_what_they_do_not_take():
 
     torch.vmap(f)(x)
     assert seen == [False]
+
+
+def test_own_forwards_and_function_modes_are_kept():
+    """A Linear whose forward was replaced on the instance runs that forward;
+    a function mode keeps calls in torch, a default device alone does not."""
+    from torch.overrides import TorchFunctionMode
+
+    from ecf8_amd import guards
+    from ecf8_amd.dit import _AdaNorm
+
+    class Watch(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    norm = _AdaNorm(8, 2)
+    norm.linear = torch.nn.Linear(8, 16).bfloat16()
+    assert guards.bare(norm.linear, torch.nn.Linear)
+    norm.linear.forward = lambda x: torch.full((x.shape[0], 16), 3.0)
+    assert all(bool((t == 3.0).all()) for t in norm(torch.randn(2, 8).bfloat16()))
+    with Watch():
+        assert not guards.untracked()
+    with torch.device("cpu"):
+        assert guards.untracked()
