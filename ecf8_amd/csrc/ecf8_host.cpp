@@ -10,7 +10,6 @@
 #include <algorithm>
 #include <memory>
 #include <new>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -119,7 +118,7 @@ void run_parallel(int n, F f) {
   int started = 0;
   try {
     for (; started < n - 1; ++started) th[started] = std::thread(f, started);
-  } catch (const std::system_error &) {
+  } catch (...) {  // no thread, or no memory for its state
   }
   for (int i = started; i < n; ++i) f(i);
   for (int i = 0; i < started; ++i) th[i].join();
