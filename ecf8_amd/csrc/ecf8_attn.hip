@@ -7,6 +7,8 @@
 #include <math.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "ecf8.h"
 #include "ecf8_attn.h"
 
@@ -95,8 +97,8 @@ struct Attn {
 // bf16, as the DiT's softmax does.
 //
 // Bound by the MFMA pipe and the exponentials (16 of each per 32 x 32 tile
-// per wave: ~512 and ~450 cycles).MI355X, causal
-// with three parts: 1 x 32 heads x 2048 queries 136 us with the packing
+// per wave: ~512 and ~450 cycles).  MI355X,
+// causal with three parts: 1 x 32 heads x 2048 queries 136 us with the packing
 // pass (fp32 library products, mask and softmax passes before: 1272 us),
 // 16 x 32 x 128 23 us (219).
 template <bool kCausal, bool kExact>
@@ -184,8 +186,9 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(Attn a) {
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int i = 0; i < 16; ++i) bm = fmaxf(bm, s[t][i]);
-    bm = fmaxf(bm, __shfl_xor(bm, 32));
-    const float mn = fmaxf(m, bm);
+    const auto hm = __builtin_amdgcn_permlane32_swap(__float_as_uint(bm), __float_as_uint(bm),
+                                                     false, false);
+    const float mn = fmaxf(m, fmaxf(__uint_as_float(hm[0]), __uint_as_float(hm[1])));
     if (__any(mn > m)) {  // uniform: some query's maximum moved
       const float f = __builtin_amdgcn_exp2f((m - mn) * a.scale);
       l *= f;
@@ -234,6 +237,213 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(Attn a) {
   const float inv = 1.f / l;
   const int batch = head / a.Hq;
   uint16_t *op = a.out + ((size_t)batch * a.T + qi) * a.out_stride +
+                 (size_t)(head % a.Hq) * kD + 4 * h;
+#pragma unroll
+  for (int d = 0; d < 4; ++d)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      *reinterpret_cast<u32x2 *>(op + 32 * d + 8 * i) =
+          u32x2{pack_bf16(o[d][4 * i] * inv, o[d][4 * i + 1] * inv),
+                pack_bf16(o[d][4 * i + 2] * inv, o[d][4 * i + 3] * inv)};
+}
+
+// ------------------------------------------- attention without a mask (DiT)
+
+constexpr int kPairQueries = 256;  // queries per workgroup: eight waves of 32
+
+// flash_kernel's computation (no mask, probabilities rounded to bf16) with
+// the two waves of a SIMD taking turns, a barrier apart: one runs its
+// products (the values' of the last block, then the scores' of this one;
+// operands are read from LDS eight products ahead) while the other runs its
+// softmax.
+// Keys and values of a block go through registers to a ring of three LDS
+// stages: block b + 1 is written in the phase in which the first four waves
+// run block b's softmax and the others its products, when its stage was last
+// read two phases before.
+//
+// Bound by the softmax phase (per wave and block 1024 cycles of MFMA, ~1100
+// of exponentials and other vector instructions, which share the SIMD's
+// issue).  MI355X, 24 heads x 4608 tokens: 261 us, 0.40 of the bf16 peak
+// while a CU has work (the grid's second round is 0.69 full); flash_kernel
+// with one exponent multiply and a rescale per block more 327 us.
+__global__ __launch_bounds__(512) void pair_attention_kernel(Attn a) {
+  __shared__ u32x4 s_k[3][kBlock * 16];
+  __shared__ u32x4 s_v[3][kBlock * 16];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const bool behind = wave >= 4;  // a phase behind the others
+  const int r = lane & 31, h = lane >> 5;
+  // a head's query tiles go to one XCD (see flash_kernel)
+  int id = blockIdx.x;
+  if (a.heads % 8 == 0) id = (id % 8) * (a.heads / 8 * a.tiles) + id / 8;
+  const int head = id / a.tiles;
+  const int q0 = (id % a.tiles) * kPairQueries + 32 * wave;
+  const int qi = min(q0 + r, a.T - 1);  // rows past T repeat the last, unstored
+  const bool used = q0 < a.T;           // uniform
+
+  v8bf qf[8];
+  {
+    const uint16_t *qp = a.q + ((size_t)head * a.T + qi) * kD + 8 * h;
+#pragma unroll
+    for (int kk = 0; kk < 8; ++kk) qf[kk] = *reinterpret_cast<const v8bf *>(qp + 16 * kk);
+  }
+  const u32x4 *kp = reinterpret_cast<const u32x4 *>(a.k + (size_t)head * a.Tp * kD);
+  const u32x4 *vp = reinterpret_cast<const u32x4 *>(a.v + (size_t)head * a.Tp * kD);
+  const int blocks = (a.T + kBlock - 1) / kBlock;
+
+  u32x4 kr[2], vr[2];
+  auto load = [&](int b) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      kr[i] = kp[(size_t)b * (kBlock * 16) + 512 * i + threadIdx.x];
+      vr[i] = vp[(size_t)b * (kBlock * 16) + 512 * i + threadIdx.x];
+    }
+  };
+  auto write = [&](int st) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      s_k[st][512 * i + threadIdx.x] = kr[i];
+      s_v[st][512 * i + threadIdx.x] = vr[i];
+    }
+  };
+  auto phase = [] {
+    __builtin_amdgcn_sched_barrier(0);
+    lds_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  v16f o[4], s[2];
+#pragma unroll
+  for (int d = 0; d < 4; ++d)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[d][i] = 0.f;
+  float m = -INFINITY, l = 0.f;  // of query r: both lanes hold the same m
+  u32x4 pf[4] = {};              // the probabilities of 16 keys each
+
+  auto values = [&](int st) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        const v8bf vf = *reinterpret_cast<const v8bf *>(&s_v[st][g * 256 + d * 64 + lane]);
+        o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, __builtin_bit_cast(v8bf, pf[g]), o[d],
+                                                       0, 0, 0);
+      }
+  };
+  auto scores = [&](int st) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[t][i] = 0.f;
+#pragma unroll
+    for (int kk = 0; kk < 8; ++kk)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const v8bf kf = *reinterpret_cast<const v8bf *>(&s_k[st][t * 512 + kk * 64 + lane]);
+        s[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[kk], s[t], 0, 0, 0);
+      }
+  };
+  // n products whose operands are read from LDS kAhead products before
+  auto order = [](auto n) {
+    constexpr int kN = decltype(n)::value, kAhead = 8;
+    __builtin_amdgcn_sched_group_barrier(0x100, kAhead, 0);  // LDS reads
+#pragma unroll
+    for (int i = 0; i < kN - kAhead; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);  // MFMA
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x8, kAhead, 0);
+  };
+
+  load(0);
+  write(0);
+  if (blocks > 1) load(1);
+  phase();
+  // block b + 1 to its stage, block b + 2 on its way
+  auto stage = [&](int b, int st) {
+    if (b + 1 < blocks) {
+      write(st);
+      if (b + 2 < blocks) load(b + 2);
+    }
+  };
+  if (behind) {
+    phase();
+    stage(0, 1);
+  }
+  if (used) {
+    scores(0);
+    order(std::integral_constant<int, 16>());
+  }
+  phase();
+  int st = 0;  // stage of block b
+  for (int b = 0;; ++b) {
+    const int st1 = st == 2 ? 0 : st + 1, st2 = st == 0 ? 2 : st - 1;  // of b + 1, b + 2
+    // softmax (the other four waves: products)
+    if (!behind) stage(b, st1);
+    __builtin_amdgcn_s_setprio(1);
+    if (used) {
+      const int key0 = b * kBlock;
+      if (key0 + kBlock > a.T) {  // uniform: keys past the last
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int i = 0; i < 16; ++i)
+            if (key0 + 32 * t + 8 * (i >> 2) + 4 * h + (i & 3) >= a.T) s[t][i] = -INFINITY;
+      }
+      float bm = s[0][0];
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) bm = fmaxf(bm, s[t][i]);
+      const auto hm = __builtin_amdgcn_permlane32_swap(__float_as_uint(bm), __float_as_uint(bm),
+                                                       false, false);
+      const float mn = fmaxf(m, fmaxf(__uint_as_float(hm[0]), __uint_as_float(hm[1])));
+      // uniform: some query's maximum moved by more than a factor 2^8 of its
+      // exponentials.  Below that m stays (nothing overflows, the quotient
+      // of the sums is the same); most blocks would rescale for a query.
+      if (__any(mn > m + 8.f)) {
+        const float f = __builtin_amdgcn_exp2f(m - mn);
+        l *= f;
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) o[d][i] *= f;
+        m = mn;
+      }
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          s[t][i] = __builtin_amdgcn_exp2f(s[t][i] - m);
+          l += s[t][i];
+        }
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          pf[g][j] = pack_bf16(s[g >> 1][8 * (g & 1) + 2 * j], s[g >> 1][8 * (g & 1) + 2 * j + 1]);
+    }
+    __builtin_amdgcn_s_setprio(0);
+    phase();
+    if (b + 1 == blocks) break;
+    // products (the other four waves: softmax)
+    if (behind) stage(b + 1, st2);
+    if (used) {
+      values(st);
+      scores(st1);
+      order(std::integral_constant<int, 32>());
+    }
+    phase();
+    st = st1;
+  }
+  if (!behind) phase();
+  if (!used) return;
+  values(st);
+  order(std::integral_constant<int, 16>());
+  l += __shfl_xor(l, 32);
+  if (q0 + r >= a.T) return;
+  const float inv = 1.f / l;
+  uint16_t *op = a.out + ((size_t)(head / a.Hq) * a.T + qi) * a.out_stride +
                  (size_t)(head % a.Hq) * kD + 4 * h;
 #pragma unroll
   for (int d = 0; d < 4; ++d)
@@ -576,16 +786,31 @@ extern "C" int ecf8_packed_attention(const void *q, const void *k_packed, const 
                                      void *stream) {
   if (!q || !k_packed || !v_packed || !out || B <= 0 || H <= 0 || T <= 0)
     return ECF8_ERR_INVALID_ARG;
-  const int64_t tiles = (T + kQueries - 1) / kQueries;
-  if (T > (1 << 24) || B > (1 << 24) || B * H * tiles > INT32_MAX || out_stride % 4)
+  if (T > (1 << 24) || B > (1 << 24) || B * H * ((T + kQueries - 1) / kQueries) > INT32_MAX ||
+      out_stride % 4)
     return ECF8_ERR_UNSUPPORTED;
   if (out_stride < (int64_t)H * kD) return ECF8_ERR_CAPACITY;
   if (!aligned(q, 16) || !aligned(k_packed, 16) || !aligned(v_packed, 16) || !aligned(out, 8))
     return ECF8_ERR_MISALIGNED;
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    return ECF8_ERR_HIP;
+  // While 128-query workgroups of four waves find a CU each, spreading the
+  // waves (one a SIMD) beats pairing them: MI355X, 24 heads, with the packing
+  // pass, us, four waves against eight: T = 1088 (216 workgroups) 43.3
+  // against 45.9, T = 2304 (432) 101.6 against 82.2, two batches of T = 1500
+  // (576) 117.5 against 113.6, T = 4608 354 against 288.
+  const bool spread = B * H * ((T + kQueries - 1) / kQueries) <= cus;
+  const int queries = spread ? kQueries : kPairQueries;
+  const int tiles = (int)((T + queries - 1) / queries);
   const Attn a{static_cast<const uint16_t *>(q), static_cast<const uint16_t *>(k_packed),
                static_cast<const uint16_t *>(v_packed), static_cast<uint16_t *>(out), out_stride,
-               (int)T, (int)padded(T), H, 1, (int)tiles, (int)(B * H), kLog2e};
-  flash_kernel<false, false><<<(unsigned)(B * H * tiles), 256, 0, as_stream(stream)>>>(a);
+               (int)T, (int)padded(T), H, 1, tiles, (int)(B * H), 1.f};
+  if (spread)
+    flash_kernel<false, false><<<(unsigned)(B * H * tiles), 256, 0, as_stream(stream)>>>(a);
+  else
+    pair_attention_kernel<<<(unsigned)(B * H * tiles), 512, 0, as_stream(stream)>>>(a);
   return launched();
 }
 

@@ -21,6 +21,7 @@ from .guards import untracked as _untracked
 from .llm_kernels import packed_kv
 
 HEAD_DIM = 128
+Q_SCALE = math.log2(math.e) / math.sqrt(HEAD_DIM)  # of scores that are powers of two
 
 
 class _Stream(ctypes.Structure):
@@ -87,7 +88,8 @@ def joint_attention(streams, heads, cos, sin, tail=None):
         return None
     B, T = streams[0][0].shape[0], sum(s[0].shape[1] for s in streams if s[0].dim() == 3)
     if (any(not _qkv_rows(s[0], heads) or s[0].shape[0] != B for s in streams)
-            or any(tuple(n.weight.shape) != (HEAD_DIM,) for n in norms)
+            or any(tuple(n.weight.shape) != (HEAD_DIM,) or not n.weight.is_contiguous()
+                   for n in norms)
             or any(tuple(t.shape) != (1, 1, T, HEAD_DIM // 2) or not t.is_contiguous()
                    or t.device != every[0].device for t in (cos, sin))):
         return None
@@ -95,7 +97,8 @@ def joint_attention(streams, heads, cos, sin, tail=None):
     if tail is not None:
         m = tail.shape[-1]
         if (tuple(tail.shape) != (B, T, m) or m % 8 or tail.stride(2) != 1
-                or tail.stride(1) % 8 or (B > 1 and tail.stride(0) != T * tail.stride(1))):
+                or tail.stride(1) % 8 or tail.stride(1) < m
+                or (B > 1 and tail.stride(0) != T * tail.stride(1))):
             return None
     dev = every[0].device
     arr = (_Stream * len(streams))(*[
@@ -104,8 +107,8 @@ def joint_attention(streams, heads, cos, sin, tail=None):
     q = torch.empty(B * T * C, dtype=torch.bfloat16, device=dev)
     k, v = packed_kv(B, heads, T, dev)
     out = torch.empty(B, T, C + m, dtype=torch.bfloat16, device=dev)
-    _launch(dev, "ecf8_dit_qkv", arr, len(streams), B, heads, 1e-6, 1.0 / math.sqrt(HEAD_DIM),
-            cos.data_ptr(), sin.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr())
+    _launch(dev, "ecf8_dit_qkv", arr, len(streams), B, heads, 1e-6, Q_SCALE, cos.data_ptr(),
+            sin.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr())
     _launch(dev, "ecf8_packed_attention", q.data_ptr(), k.data_ptr(), v.data_ptr(), B, heads, T,
             out.data_ptr(), C + m)
     if m:

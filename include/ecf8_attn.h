@@ -61,9 +61,10 @@ int ecf8_dit_qkv(const ecf8_dit_stream *streams, int n_streams, int64_t B, int H
                  void *v_packed, void *stream);
 
 /*
- * Attention of q bf16 [B, H, T, 128] (already scaled) over packed keys and
- * values of the same T tokens: fp32 scores and softmax, bf16
- * probabilities, fp32 sums; row t of batch b goes to out (bf16) +
+ * Attention of q bf16 [B, H, T, 128] (scaled by log2(e) / sqrt(128): a
+ * probability is a power of two of its score) over packed keys and values
+ * of the same T tokens: fp32 scores and softmax, bf16 probabilities, fp32
+ * sums; row t of batch b goes to out (bf16) +
  * (b * T + t) * out_stride, head h at column 128 h.
  */
 int ecf8_packed_attention(const void *q, const void *k_packed, const void *v_packed, int64_t B,

@@ -99,7 +99,10 @@ def _dit_reference(streams, heads, cos, sin, tail):
 
 @pytest.mark.parametrize("B,tokens,heads,tail", [
     (1, (1,), 1, 0), (1, (31, 32), 8, 0), (2, (5, 59), 2, 0), (1, (64,), 3, 8), (1, (65,), 8, 520),
-    (2, (127,), 2, 264), (1, (1, 127), 1, 0), (1, (128, 1), 16, 0), (3, (200,), 4, 1024)])
+    (2, (127,), 2, 264), (1, (1, 127), 1, 0), (1, (128, 1), 16, 0), (3, (200,), 4, 1024),
+    # over 256 workgroups of 128 queries: the kernel of 256 queries
+    (1, (1,), 264, 0), (1, (64,), 264, 8), (1, (65,), 257, 0), (1, (129,), 136, 0),
+    (2, (31, 225), 72, 0), (1, (257,), 96, 0), (1, (200, 313), 66, 0)])
 def test_dit_joint_attention_matches_fp64(cuda_device, B, tokens, heads, tail):
     """One stream (a strided slice of a wider projection, with a GELU tail)
     and two, at the edges of the 32-token, 64-key and 128-query tiles.
@@ -131,6 +134,20 @@ def test_dit_joint_attention_matches_fp64(cuda_device, B, tokens, heads, tail):
         if want[..., part].numel():
             err = (got[..., part].double() - want[..., part]).norm() / want[..., part].norm()
             assert float(err) <= 4 * 2.0 ** -9.8, float(err)
+
+
+def test_dit_joint_attention_leaves_odd_layouts(cuda_device):
+    """An expanded norm weight and a tail with overlapping rows run in torch."""
+    from ecf8_amd import dit_kernels as DK
+    from ecf8_amd.dit import _Norm
+
+    y = torch.randn(1, 4, 3 * 128, device=cuda_device).to(torch.bfloat16)
+    norms = [_Norm(128).to(cuda_device).requires_grad_(False) for _ in range(2)]
+    cos = torch.ones(1, 1, 4, 64, device=cuda_device)
+    tail = y.reshape(-1)[:16].expand(1, 4, 16)
+    assert DK.joint_attention([(y, *norms)], 1, cos, cos, tail=tail) is None
+    norms[0].weight = torch.nn.Parameter(norms[0].weight[:1].expand(128), requires_grad=False)
+    assert DK.joint_attention([(y, *norms)], 1, cos, cos) is None
 
 
 @pytest.mark.parametrize("B,T,C", [(1, 1, 8), (2, 3, 2048), (1, 5, 2056), (2, 2, 4096), (1, 3, 8192)])
