@@ -263,9 +263,9 @@ constexpr int kPairQueries = 256;  // queries per workgroup: eight waves of 32
 //
 // Bound by the softmax phase (per wave and block 1024 cycles of MFMA, ~1100
 // of exponentials and other vector instructions, which share the SIMD's
-// issue).  MI355X, 24 heads x 4608 tokens: 261 us, 0.40 of the bf16 peak
-// while a CU has work (the grid's second round is 0.69 full); flash_kernel
-// with one exponent multiply and a rescale per block more 327 us.
+// issue).  MI355X, 24 heads x 4608 tokens: 261 us (the MFMAs alone 127 us at
+// the clock it ran at; the grid's second round of workgroups is 0.69 full),
+// flash_kernel 327 us.
 __global__ __launch_bounds__(512) void pair_attention_kernel(Attn a) {
   __shared__ u32x4 s_k[3][kBlock * 16];
   __shared__ u32x4 s_v[3][kBlock * 16];
