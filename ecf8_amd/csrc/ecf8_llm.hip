@@ -589,21 +589,33 @@ __global__ __launch_bounds__(512) void fp8_gemm_kernel(
 //
 // The tile GEMM above has one workgroup per 256 x 128 outputs: a few dozen
 // at the row counts of a served batch or a short prompt, most CUs idle.
-// Here a workgroup of eight waves computes 16 kCh rows x 16 P columns and
-// splits K over its waves (wave w: the w-th run of groups); a wave reads its
-// operands straight into registers in MFMA order, one group ahead, and the
-// waves' sums meet in LDS and are added in wave order.  P trades the
-// number of workgroups against re-reading the activations per column strip
-// (from L2).  HBM or L2 bounds it; MI355X, 64 rows: N = K = 4096 34.8 -> 8.9
-// us, N = 4096, K = 12288 94 -> 20 us.
-template <int P, int kCh>
+// Here a workgroup of eight waves computes 16 kCh rows x 16 P columns, and
+// wave w multiplies the K groups w, w + 8, ... straight from its registers,
+// two of them ahead, so eight waves read a few dozen columns' weights at
+// once.  The sums are the tile GEMM's, bit for bit: every eight groups the
+// waves put their products into LDS, and each 16 x 16 tile of the strip has
+// one wave that adds them to its sums in group order, with that kernel's
+// scale and fma.  So a row's result does not depend on how many rows share
+// the call (above 16).
+//
+// P trades the number of workgroups against re-reading the activations per
+// column strip (from L2).  The latency of a round bounds it, ~3 us for 128 KB
+// of operands at P = 4 (L2) and the products' way through LDS.  MI355X, tile
+// layout, us, against the tile GEMM, and against waves that each add a run
+// of K (another order, that differs with the row count): 64 rows, N = K =
+// 4096 7.8 / 32.5 / 8.3, N = 4096, K = 12288 23.8 / 89.8 / 26.6; 256 rows
+// 13.2 / 33.1 / 12.9 and 41.4 / 111 / 33.2; 512 rows 25.2 / 33.5 / 23.9 and
+// 73 / 106 / 58.
+template <int P, int kCh, int kSub>
 __global__ __launch_bounds__(512) void fp8_rows_kernel(const uint8_t *__restrict__ aq,
                                                        const float *__restrict__ as, int M, int K,
                                                        LinearSegs segs, uint16_t *__restrict__ out,
                                                        int ldo) {
-  constexpr int kWaves = 8, kVals = 4 * kCh;
-  __shared__ float red[kWaves][kVals][64];
-  __shared__ __attribute__((aligned(16))) float s_sc[kWaves][2][64];
+  constexpr int kWaves = 8, kTurns = P / kSub, kTiles = kSub * kCh;  // tiles a turn
+  static_assert(P % kSub == 0 && kTiles <= kWaves, "a wave adds one tile a turn");
+  // products of a turn (kSub panels of eight groups), double-buffered
+  __shared__ v4f s_d[2][kWaves][kTiles][64];
+  __shared__ float s_sc[2][kWaves][64];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, g = lane >> 4;
@@ -635,16 +647,14 @@ __global__ __launch_bounds__(512) void fp8_rows_kernel(const uint8_t *__restrict
   for (int c = 0; c < kCh; ++c)
     ab[c] = aq + (size_t)min(m0 / 16 + c, last_rb) * kgroups * 2048 + 16 * lane;
   const float *asr = as + (size_t)min(m0 + min(lane, 16 * kCh - 1), M - 1) * kgroups;
-
-  const int run = (kgroups + kWaves - 1) / kWaves;
-  const int k0 = wave * run, k1 = min(k0 + run, kgroups);
+  const int rounds = (kgroups + kWaves - 1) / kWaves;
 
   struct Stage {
     u32x4 wv[P][2], av[kCh][2];
     float sa, sw;
   };
-  auto load = [&](int kg, Stage &s) {
-    const int k = min(kg, kgroups - 1);  // past the run: loaded, unused
+  auto load = [&](int rd, Stage &s) {
+    const int k = min(kWaves * rd + wave, kgroups - 1);  // past the last: loaded, unused
 #pragma unroll
     for (int p = 0; p < P; ++p) {
       const uint32_t at = (uint32_t)k * (uint32_t)wl.step + 16u * (uint32_t)p * (uint32_t)K;
@@ -659,60 +669,69 @@ __global__ __launch_bounds__(512) void fp8_rows_kernel(const uint8_t *__restrict
     s.sa = asr[k];
     s.sw = wsrow[k];
   };
-  v4f acc[P][kCh];
+  // wave's tile of turn t: panel t kSub + wave / kCh, rows 16 (wave % kCh)..;
+  // lane: columns 4 g .. + 3, row r
+  v4f acc[kTurns];
 #pragma unroll
-  for (int p = 0; p < P; ++p)
+  for (int t = 0; t < kTurns; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
+  auto step = [&](Stage &s, int rd) {
+    const int n = min(kWaves, kgroups - kWaves * rd);  // groups of this round
+    if (wave < n) s_sc[rd & 1][wave][lane] = s.sa * s.sw;
 #pragma unroll
-    for (int c = 0; c < kCh; ++c) acc[p][c] = v4f{0.f, 0.f, 0.f, 0.f};
-  auto step = [&](const Stage &s, int buf) {
-    // the rows' scales, lane = row, to the lanes that hold those rows' sums
-    // (the wave's own LDS: program order, no barrier)
-    s_sc[wave][buf][lane] = s.sa * s.sw;
-    __builtin_amdgcn_wave_barrier();
+    for (int t = 0; t < kTurns; ++t) {
+      const int buf = (rd * kTurns + t) & 1;
+      if (wave < n) {  // uniform
 #pragma unroll
-    for (int c = 0; c < kCh; ++c) {
-      const f32x4 sc = *reinterpret_cast<const f32x4 *>(&s_sc[wave][buf][16 * c + 4 * g]);
-      const v8i a = __builtin_shufflevector(__builtin_bit_cast(v4i, s.av[c][0]),
-                                            __builtin_bit_cast(v4i, s.av[c][1]), 0, 1, 2, 3, 4, 5,
-                                            6, 7);
+        for (int p = 0; p < kSub; ++p)
 #pragma unroll
-      for (int p = 0; p < P; ++p) {
-        const v8i b = __builtin_shufflevector(__builtin_bit_cast(v4i, s.wv[p][0]),
-                                              __builtin_bit_cast(v4i, s.wv[p][1]), 0, 1, 2, 3, 4,
-                                              5, 6, 7);
-        const v4f z = {0.f, 0.f, 0.f, 0.f};
-        const v4f d = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, z, 0, 0, 0, 0, 0, 0);
+          for (int c = 0; c < kCh; ++c) {
+            const v4f z = {0.f, 0.f, 0.f, 0.f};
+            s_d[buf][wave][p * kCh + c][lane] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                join32(s.wv[t * kSub + p][0], s.wv[t * kSub + p][1]),
+                join32(s.av[c][0], s.av[c][1]), z, 0, 0, 0, 0, 0, 0);
+          }
+      }
+      if (t == kTurns - 1 && rd + 2 < rounds) load(rd + 2, s);
+      // the products are in LDS; the other buffer (of the scales too) was
+      // last read before every wave's arrival here
+      lds_barrier();
+      if (wave < kTiles) {  // uniform
+        const float *sc = &s_sc[rd & 1][0][16 * (wave % kCh) + r];
+        auto add = [&](int v) {
+          const v4f d = s_d[buf][v][wave][lane];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) acc[p][c][i] = fmaf(d[i], sc[i], acc[p][c][i]);
+          for (int i = 0; i < 4; ++i) acc[t][i] = fmaf(d[i], sc[64 * v], acc[t][i]);
+        };
+        if (n == kWaves) {  // all reads in flight at once
+#pragma unroll
+          for (int v = 0; v < kWaves; ++v) add(v);
+        } else {
+          for (int v = 0; v < n; ++v) add(v);
+        }
       }
     }
-    __builtin_amdgcn_wave_barrier();
   };
-  if (k0 < k1) {
-    Stage s0, s1;
-    load(k0, s0);
-    for (int kg = k0; kg < k1; kg += 2) {
-      load(kg + 1, s1);
-      step(s0, 0);
-      load(kg + 2, s0);
-      if (kg + 1 < k1) step(s1, 1);  // uniform
-    }
+  Stage s0, s1;
+  load(0, s0);
+  if (rounds > 1) load(1, s1);
+  for (int rd = 0; rd < rounds; rd += 2) {
+    step(s0, rd);
+    if (rd + 1 < rounds) step(s1, rd + 1);  // uniform
   }
+  if (wave >= kTiles) return;
+  const int m = m0 + 16 * (wave % kCh) + r;
+  if (m >= M) return;
+  const bool whole =
+      (((uintptr_t)out | 2u * (uintptr_t)(uint32_t)ldo | 2u * (uintptr_t)(uint32_t)col) & 7) == 0;
 #pragma unroll
-  for (int p = 0; p < P; ++p) {
-    if (p) __syncthreads();  // red is rewritten
+  for (int t = 0; t < kTurns; ++t) {
+    uint16_t *o = out + (size_t)m * ldo + col + n0 + 16 * (t * kSub + wave / kCh) + 4 * g;
+    const u32x2 v = {pack_bf16(acc[t][0], acc[t][1]), pack_bf16(acc[t][2], acc[t][3])};
+    if (whole) {
+      *reinterpret_cast<u32x2 *>(o) = v;
+    } else {
 #pragma unroll
-    for (int c = 0; c < kCh; ++c)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) red[wave][4 * c + i][lane] = acc[p][c][i];
-    __syncthreads();
-    for (int t = threadIdx.x; t < 64 * kVals; t += 512) {
-      const int ci = t >> 6, l = t & 63;
-      float sum = 0.f;
-#pragma unroll
-      for (int v = 0; v < kWaves; ++v) sum += red[v][ci][l];
-      const int m = m0 + 16 * (ci >> 2) + 4 * (l >> 4) + (ci & 3);
-      if (m < M) out[(size_t)m * ldo + col + n0 + 16 * p + (l & 15)] = (uint16_t)f32_bf16(sum);
+      for (int q = 0; q < 4; ++q) o[q] = (uint16_t)(v[q / 2] >> (16 * (q & 1)));
     }
   }
 }
@@ -2076,36 +2095,39 @@ extern "C" int ecf8_fp8_linear(const void *aq, const float *as, int64_t M, int64
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
       return ECF8_ERR_HIP;
-    // The middle form while its 64 x 64 blocks are at most two per CU: the
-    // tile GEMM then has at most one workgroup on a quarter of the CUs.
-    // MI355X, us, middle form against tile GEMM (four weight copies rotated):
-    // N = K = 4096: M = 64 8.9 / 34.8, M = 256 13.4 / 35.6, M = 512 (512
-    // blocks) 24.3 / 36.2, M = 768 35.0 / 36.7, M = 1024 45.7 / 37.2; N =
-    // 24576: M = 64 (384 blocks) 35.5 / 39.0, M = 96 (768) 56.8 / 41.4.
+    // The middle form while its 64 x 64 blocks are at most two per CU.  Where
+    // M fills the 256-row tiles, the tile GEMM then has a workgroup on a
+    // quarter of the CUs at most; for few rows it can have one on each, and
+    // the line rests on the times alone.  MI355X, us, middle form against
+    // tile GEMM (weight copies rotated): N = K = 4096: M = 64 7.8 / 32.5, M =
+    // 256 13.2 / 33.1, M = 512 (512 blocks) 25.2 / 33.5, M = 768 36.6 / 33.8;
+    // N = 24576: M = 64 (384 blocks) 34.3 / 39.1, M = 128 (768) 51.7 / 40.1;
+    // N = 32768, M = 64 (512) 40.8 / 44.6; K = 512, M = 512, N = 4096 7.3 /
+    // 8.5 (one K group: 6.5 / 5.5).
     const int64_t blocks = (M + 63) / 64 * (n_total / 64);
     if (blocks <= 2 * (int64_t)cus) {
       // The narrowest strips that need no second round of workgroups; for a
       // single block of rows, where the weights come from HBM once, three
-      // workgroups per CU hide each other's loads (N = 24576, M = 64: two
-      // panels 35.5, four 38.7 us; N = 6144, M = 64: one 13.0, two 10.3,
-      // four 13.8).  32 rows a block where that covers M: M = 32, N = 4096
-      // 8.3 us.
+      // workgroups per CU in turn (N = 24576, M = 64: two panels 34.3, four
+      // 37.1 us; N = 28672: 43.8 and 38.0; N = 6144, M = 64: one 11.7, two
+      // 9.7, four 13.5).  32 rows a block where that covers M: M = 32, N =
+      // 4096 5.8 us.
       const bool narrow = M <= 32;
       const int64_t row_blocks = narrow ? 1 : (M + 63) / 64;
       const int64_t one = row_blocks * (n_total / 16);
       const int panels = one <= cus ? 1 : one / 2 <= (row_blocks == 1 ? 3 : 1) * cus ? 2 : 4;
       const dim3 grid((unsigned)(n_total / (16 * panels)), (unsigned)row_blocks);
-#define ECF8_ROWS(P, CH)                                                                    \
-  fp8_rows_kernel<P, CH><<<grid, 512, 0, as_stream(stream)>>>(a, as, (int)M, (int)K, s, o, \
-                                                              (int)ldo)
+#define ECF8_ROWS(P, CH, SUB)                                                                    \
+  fp8_rows_kernel<P, CH, SUB><<<grid, 512, 0, as_stream(stream)>>>(a, as, (int)M, (int)K, s, o, \
+                                                                   (int)ldo)
       if (narrow) {
-        if (panels == 1) ECF8_ROWS(1, 2);
-        else if (panels == 2) ECF8_ROWS(2, 2);
-        else ECF8_ROWS(4, 2);
+        if (panels == 1) ECF8_ROWS(1, 2, 1);
+        else if (panels == 2) ECF8_ROWS(2, 2, 2);
+        else ECF8_ROWS(4, 2, 4);
       } else {
-        if (panels == 1) ECF8_ROWS(1, 4);
-        else if (panels == 2) ECF8_ROWS(2, 4);
-        else ECF8_ROWS(4, 4);
+        if (panels == 1) ECF8_ROWS(1, 4, 1);
+        else if (panels == 2) ECF8_ROWS(2, 4, 2);
+        else ECF8_ROWS(4, 4, 2);
       }
 #undef ECF8_ROWS
       return launched();

@@ -270,6 +270,73 @@ def test_fp8_linear_many_rows_either_form(cuda_device, M, shapes, Kd, layout):
 
 
 @pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("shapes,Kd,pad", [
+    ((4096, 1024, 1024), 4096, 0), ((4096,), 4096, 0), ((1024,), 12288, 0),
+    ((128, 256, 128), 384, 2), ((512, 128), 2176, 1), ((8192,), 896, 4)])
+def test_fp8_linear_rows_do_not_depend_on_the_call(cuda_device, shapes, Kd, pad, layout):
+    """Above 16 rows every form adds the K groups in one order: the rows of a
+    short call have the bits that they have inside a long one (tile GEMM),
+    with any number of panels and row blocks, K groups that fill the waves'
+    rounds or not, and row strides that take narrow stores."""
+    from ecf8_amd.llm_kernels import LinearPlan
+
+    gen = torch.Generator(device=cuda_device).manual_seed(Kd + sum(shapes))
+
+    def fp8(n, k):
+        return torch.randn(n, k, generator=gen, device=cuda_device).to(FP8)
+
+    N = sum(shapes)
+    rows = 2048 if N > 1024 else 8448  # past two 64 x 64 blocks per CU
+    cus = torch.cuda.get_device_properties(cuda_device).multi_processor_count
+    assert rows // 64 * (N // 64) > 2 * cus
+    aq = fp8(rows, Kd)
+    a_s = torch.rand(rows, Kd // 128, generator=gen, device=cuda_device) + 0.1
+    segs = [(fp8(n, Kd), torch.rand(n // 128, Kd // 128, generator=gen, device=cuda_device) + 0.1)
+            for n in shapes]
+    out = torch.full((rows, N + pad), 7.0, dtype=torch.bfloat16, device=cuda_device)
+    plan = LinearPlan([(to_tiles(w), ws, 1) if layout else (w, ws) for w, ws in segs], out)
+    full = plan(to_tiles(aq), a_s, rows).clone()
+    for M in (17, 32, 33, 64, 65, 135, 256, 320, 321, 512, 1000):
+        out.fill_(7.0)
+        plan(to_tiles(aq[:M]), a_s[:M], M)
+        assert torch.equal(out[:M, :N].view(torch.int16), full[:M, :N].view(torch.int16)), M
+        assert bool((out[:, N:] == 7.0).all()) and bool((out[M:] == 7.0).all()), M
+
+
+@pytest.mark.parametrize("T", [17, 64, 135, 320])
+def test_prompt_layer_of_one_sequence_is_that_of_a_batch(cuda_device, T):
+    """A sequence's prompt pass has the same bits alone (17 to 320 rows) as
+    beside others (the linears of that call through the tile GEMM): what the
+    layer quantizes between its linears leaves no room for another order."""
+    from ecf8_amd.llm import Qwen3Config, Qwen3ForCausalLM, Qwen3Runner
+    from ecf8_amd.synth import quantize_fp8_blockwise
+
+    cfg = Qwen3Config(layers=1, intermediate=4096, vocab=128)
+    gen = torch.Generator(device=cuda_device).manual_seed(T)
+
+    def randn(*shape):
+        return torch.randn(*shape, generator=gen, device=cuda_device)
+
+    model = Qwen3ForCausalLM(cfg).to(cuda_device)
+    layer = model.model.layers[0]
+    for name, (o, i, sigma) in cfg.linear_shapes().items():
+        lin = layer.get_submodule(name)
+        w, s = quantize_fp8_blockwise(sigma * randn(o, i))
+        lin.weight, lin.weight_scale_inv = torch.nn.Parameter(w, requires_grad=False), s
+    B = -(-4096 // T)
+    x = randn(B * T, cfg.hidden)
+    got = []
+    for b in (1, B):
+        r = Qwen3Runner(model, b, T, T, cuda_device)
+        r.pos.zero_()
+        r.res.copy_(x[: b * T])
+        mlp = layer(r, 0, None, True)
+        got.append([t[:n].clone() for t, n in ((mlp, T), (r.res, T), (r.kc[0], 1), (r.vc[0], 1))])
+    for one, many in zip(*got):
+        assert torch.equal(one, many)
+
+
+@pytest.mark.parametrize("layout", [0, 1])
 @pytest.mark.parametrize("M,extra,Kd,ldo", [
     (257, (), 128, 0), (300, (128,), 256, 0), (511, (128, 128), 896, 1), (512, (256, 128), 1152, 2),
     (1024, (384,), 128, 4), (2048, (128,), 640, 0),
