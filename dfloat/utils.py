@@ -193,9 +193,10 @@ def split_fp8_counted(data: torch.Tensor):
         from ecf8_amd._lib import check, lib
 
         n = data.numel()
-        exps = torch.empty(n, dtype=torch.uint8)
-        packed = torch.empty(n // 2, dtype=torch.uint8)
-        counts = torch.empty(16, dtype=torch.int64)
+        # on the host whatever the caller's default device is
+        exps = torch.empty(n, dtype=torch.uint8, device="cpu")
+        packed = torch.empty(n // 2, dtype=torch.uint8, device="cpu")
+        counts = torch.empty(16, dtype=torch.int64, device="cpu")
         check(lib().ecf8_split_fp8(data.data_ptr(), n, exps.data_ptr(), packed.data_ptr(),
                                    counts.data_ptr(), host_threads()), "ecf8_split_fp8")
         return exps, packed, counts

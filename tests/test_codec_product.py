@@ -267,3 +267,18 @@ def test_split_counts_and_nibbles(n):
     assert torch.equal(counts, torch.bincount(want_e, minlength=16))
     again = split_fp8_counted(b.repeat_interleave(2)[::2].view(torch.float8_e4m3fn))  # strided
     assert torch.equal(again[0], want_e) and torch.equal(again[1], want_p)
+
+
+@pytest.mark.parametrize("n", [2, 400002])
+def test_host_compression_under_another_default_device(n):
+    """A host block compresses on the host, to the same tensors, where
+    factory calls go to another device (meta has no memory to write to)."""
+    from dfloat.compress import compress_flat
+
+    b = np.random.default_rng(n).integers(0, 256, n, dtype=np.uint8)
+    w = torch.from_numpy(b).view(torch.float8_e4m3fn)
+    want = compress_flat(w)
+    with torch.device("meta"):
+        got = compress_flat(w)
+    for key in ("luts", "encoded", "packed_other_4bits", "output_positions", "gaps"):
+        assert got[key].device.type == "cpu" and torch.equal(got[key], want[key]), key
