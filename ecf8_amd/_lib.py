@@ -103,7 +103,10 @@ _SIGNATURES = {
     "ecf8_greedy_work_bytes": ([_i64], _i64),
     "ecf8_greedy_emit": ([_vp, _i64, _i64, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _i32, _vp],
                          _i32),
+    "ecf8_greedy_emit_checked": ([_vp, _i64, _i64, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp,
+                                  _i32, _vp, _vp], _i32),
     "ecf8_embed_rows": ([_vp, _i64, _vp, _i64, _i64, _vp, _vp], _i32),
+    "ecf8_embed_rows_checked": ([_vp, _i64, _vp, _i64, _i64, _vp, _vp, _vp], _i32),
 }
 
 EXPORTED = tuple(_SIGNATURES)

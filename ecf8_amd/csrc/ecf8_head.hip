@@ -160,12 +160,14 @@ __global__ __launch_bounds__(256) void argmax_chunk_kernel(const uint16_t *__res
 }
 
 // Each row's token -> next[b] and tokens[b, step[0]]; then step += 1 and
-// pos += advance.  One workgroup, a wave per row in turn.
+// pos += advance.  One workgroup, a wave per row in turn.  A step outside
+// the rows writes no token and sets *refused (where there is one).
 __global__ __launch_bounds__(1024) void emit_kernel(const uint64_t *__restrict__ keys, int chunks,
                                                     int B, int64_t *__restrict__ tokens,
                                                     int64_t ldt, int64_t *__restrict__ next,
                                                     int64_t *__restrict__ step,
-                                                    int *__restrict__ pos, int advance) {
+                                                    int *__restrict__ pos, int advance,
+                                                    int *__restrict__ refused) {
   const int lane = threadIdx.x & 63;
   const int64_t at = step[0];
   for (int b = threadIdx.x >> 6; b < B; b += 16) {
@@ -185,18 +187,24 @@ __global__ __launch_bounds__(1024) void emit_kernel(const uint64_t *__restrict__
   if (threadIdx.x == 0) {
     step[0] = at + 1;
     if (advance) pos[0] += advance;
+    if (refused && (at < 0 || at >= ldt)) *refused = 1;
   }
 }
 
-// out[b, :] = float(table[token[b], :]); tokens outside the table write zeros
+// out[b, :] = float(table[token[b], :]); a token outside the table writes
+// zeros and sets *refused (where there is one)
 __global__ __launch_bounds__(256) void embed_kernel(const int64_t *__restrict__ token,
                                                     const uint16_t *__restrict__ table, int64_t V,
-                                                    int H, float *__restrict__ out) {
+                                                    int H, float *__restrict__ out,
+                                                    int *__restrict__ refused) {
   const int b = blockIdx.y, c = 8 * (blockIdx.x * 256 + threadIdx.x);
   if (c >= H) return;
   const int64_t t = token[b];
   u32x4 v = {0, 0, 0, 0};
-  if (t >= 0 && t < V) v = *reinterpret_cast<const u32x4 *>(table + (size_t)t * H + c);
+  if (t >= 0 && t < V)
+    v = *reinterpret_cast<const u32x4 *>(table + (size_t)t * H + c);
+  else if (refused)
+    *refused = 1;
   float4 *o = reinterpret_cast<float4 *>(out + (size_t)b * H + c);
   o[0] = make_float4(bf16_f32(v[0] & 0xffffu), bf16_f32(v[0] >> 16), bf16_f32(v[1] & 0xffffu),
                      bf16_f32(v[1] >> 16));
@@ -250,33 +258,49 @@ extern "C" int64_t ecf8_greedy_work_bytes(int64_t B) {
   return B <= 0 ? -1 : B * ECF8_GREEDY_CHUNKS * 8;
 }
 
-extern "C" int ecf8_greedy_emit(const void *logits, int64_t ld, int64_t B, int64_t V, void *work,
-                                int64_t work_bytes, int64_t *tokens, int64_t ld_tokens,
-                                int64_t *next_token, int64_t *step, int *pos, int advance,
-                                void *stream) {
+extern "C" int ecf8_greedy_emit_checked(const void *logits, int64_t ld, int64_t B, int64_t V,
+                                        void *work, int64_t work_bytes, int64_t *tokens,
+                                        int64_t ld_tokens, int64_t *next_token, int64_t *step,
+                                        int *pos, int advance, int *refused, void *stream) {
   if (!logits || !work || !tokens || !next_token || !step || (advance && !pos) || B <= 0 ||
       V <= 0 || ld < V || ld_tokens <= 0)
     return ECF8_ERR_INVALID_ARG;
   if (B > 65535 || V > (1 << 30)) return ECF8_ERR_UNSUPPORTED;
   if (work_bytes < ecf8_greedy_work_bytes(B)) return ECF8_ERR_CAPACITY;
   if (!aligned(logits, 2) || !aligned(work, 8) || !aligned(tokens, 8) ||
-      !aligned(next_token, 8) || !aligned(step, 8))
+      !aligned(next_token, 8) || !aligned(step, 8) || !aligned(refused, 4))
     return ECF8_ERR_MISALIGNED;
   auto *keys = static_cast<uint64_t *>(work);
   argmax_chunk_kernel<<<dim3(ECF8_GREEDY_CHUNKS, (unsigned)B), 256, 0, as_stream(stream)>>>(
       static_cast<const uint16_t *>(logits), ld, (int)V, ECF8_GREEDY_CHUNKS,
       ld % 8 == 0 && aligned(logits, 16), keys);
   emit_kernel<<<1, 1024, 0, as_stream(stream)>>>(keys, ECF8_GREEDY_CHUNKS, (int)B, tokens,
-                                                 ld_tokens, next_token, step, pos, advance);
+                                                 ld_tokens, next_token, step, pos, advance,
+                                                 refused);
+  return launched();
+}
+
+extern "C" int ecf8_greedy_emit(const void *logits, int64_t ld, int64_t B, int64_t V, void *work,
+                                int64_t work_bytes, int64_t *tokens, int64_t ld_tokens,
+                                int64_t *next_token, int64_t *step, int *pos, int advance,
+                                void *stream) {
+  return ecf8_greedy_emit_checked(logits, ld, B, V, work, work_bytes, tokens, ld_tokens,
+                                  next_token, step, pos, advance, nullptr, stream);
+}
+
+extern "C" int ecf8_embed_rows_checked(const int64_t *token, int64_t B, const void *table,
+                                       int64_t V, int64_t H, float *out, int *refused,
+                                       void *stream) {
+  if (!token || !table || !out || B <= 0 || V <= 0 || H <= 0) return ECF8_ERR_INVALID_ARG;
+  if (H % 8 || H > (1 << 24) || B > 65535) return ECF8_ERR_UNSUPPORTED;
+  if (!aligned(token, 8) || !aligned(table, 16) || !aligned(out, 16) || !aligned(refused, 4))
+    return ECF8_ERR_MISALIGNED;
+  embed_kernel<<<dim3((unsigned)((H + 2047) / 2048), (unsigned)B), 256, 0, as_stream(stream)>>>(
+      token, static_cast<const uint16_t *>(table), V, (int)H, out, refused);
   return launched();
 }
 
 extern "C" int ecf8_embed_rows(const int64_t *token, int64_t B, const void *table, int64_t V,
                                int64_t H, float *out, void *stream) {
-  if (!token || !table || !out || B <= 0 || V <= 0 || H <= 0) return ECF8_ERR_INVALID_ARG;
-  if (H % 8 || H > (1 << 24) || B > 65535) return ECF8_ERR_UNSUPPORTED;
-  if (!aligned(token, 8) || !aligned(table, 16) || !aligned(out, 16)) return ECF8_ERR_MISALIGNED;
-  embed_kernel<<<dim3((unsigned)((H + 2047) / 2048), (unsigned)B), 256, 0, as_stream(stream)>>>(
-      token, static_cast<const uint16_t *>(table), V, (int)H, out);
-  return launched();
+  return ecf8_embed_rows_checked(token, B, table, V, H, out, nullptr, stream);
 }

@@ -62,9 +62,24 @@ def greedy_work(B: int, device) -> torch.Tensor:
     return torch.empty(n // 8, dtype=torch.int64, device=device)
 
 
-def greedy_emit(logits, work, tokens, next_token, step, pos=None, advance: int = 0):
+def refusal_flag() -> torch.Tensor:
+    """A flag in pinned host memory for ``refused=`` below: zero until a
+    kernel refuses a call's values, which the host may look up at any time."""
+    return torch.zeros(1, dtype=torch.int32, device="cpu", pin_memory=torch.cuda.is_available())
+
+
+def _flag_ptr(refused):
+    if refused is None:
+        return None
+    if refused.dtype != torch.int32 or not (refused.is_cuda or refused.is_pinned()):
+        raise ECF8Error("refused must be int32 in pinned host or device memory")
+    return refused.data_ptr()
+
+
+def greedy_emit(logits, work, tokens, next_token, step, pos=None, advance: int = 0, refused=None):
     """argmax of each row of ``logits`` (bf16 [B, V]) -> next_token[b] and
-    tokens[b, step[0]]; then step += 1 and pos += advance."""
+    tokens[b, step[0]]; then step += 1 and pos += advance.  A step outside
+    the token buffer writes no token and sets ``refused``."""
     dev = logits.device
     _need(logits, torch.bfloat16, "logits", dev)
     for t, n in ((tokens, "tokens"), (next_token, "next_token"), (step, "step"), (work, "work")):
@@ -75,16 +90,16 @@ def greedy_emit(logits, work, tokens, next_token, step, pos=None, advance: int =
     if tokens.dim() != 2 or tokens.shape[0] < B or next_token.numel() < B or step.numel() < 1:
         raise ECF8Error("tokens, next_token or step too small")
     with torch.cuda.device(dev):
-        check(lib().ecf8_greedy_emit(logits.data_ptr(), logits.stride(0), B, V, work.data_ptr(),
-                                     work.numel() * 8, tokens.data_ptr(), tokens.shape[1],
-                                     next_token.data_ptr(), step.data_ptr(),
-                                     pos.data_ptr() if advance else None, advance,
-                                     torch.cuda.current_stream(dev).cuda_stream),
-              "ecf8_greedy_emit")
+        check(lib().ecf8_greedy_emit_checked(
+            logits.data_ptr(), logits.stride(0), B, V, work.data_ptr(), work.numel() * 8,
+            tokens.data_ptr(), tokens.shape[1], next_token.data_ptr(), step.data_ptr(),
+            pos.data_ptr() if advance else None, advance, _flag_ptr(refused),
+            torch.cuda.current_stream(dev).cuda_stream), "ecf8_greedy_emit")
 
 
-def embed_rows(token, table, out):
-    """out fp32 [>= B, H] = float(table[token]) for int64 tokens [B]."""
+def embed_rows(token, table, out, refused=None):
+    """out fp32 [>= B, H] = float(table[token]) for int64 tokens [B]; a token
+    outside the table writes zeros and sets ``refused``."""
     dev = out.device
     _need(token, torch.int64, "token", dev)
     _need(table, torch.bfloat16, "table", dev)
@@ -93,5 +108,6 @@ def embed_rows(token, table, out):
     if out.dim() != 2 or out.shape[1] != H or out.shape[0] < B:
         raise ECF8Error("out does not fit the embedded rows")
     with torch.cuda.device(dev):
-        check(lib().ecf8_embed_rows(token.data_ptr(), B, table.data_ptr(), V, H, out.data_ptr(),
-                                    torch.cuda.current_stream(dev).cuda_stream), "ecf8_embed_rows")
+        check(lib().ecf8_embed_rows_checked(
+            token.data_ptr(), B, table.data_ptr(), V, H, out.data_ptr(), _flag_ptr(refused),
+            torch.cuda.current_stream(dev).cuda_stream), "ecf8_embed_rows")

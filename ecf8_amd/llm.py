@@ -166,8 +166,16 @@ class _GreedyRunner:
     """Generation mechanics shared by the dense and the MoE runners: a
     subclass provides ``layer()`` and the buffers named here (``res``, ``h``,
     ``q``, ``kc``/``vc``, ``attn``, ``pos``, ``step``, ``tokens``,
-    ``next_tok``); prefill runs eagerly, a decode step can be captured as one
-    HIP graph."""
+    ``next_tok``, ``refused``); prefill runs eagerly, a decode step can be
+    captured as one HIP graph.  A step's kernels cannot raise: a token outside
+    the vocabulary or a step past the token buffer sets ``refused``, and the
+    next call raises."""
+
+    def _raise_refused(self):
+        if self._refused_host[0]:
+            self.refused.zero_()
+            raise ECF8Error("a decode step was given a token outside the vocabulary, or ran past "
+                            "the token buffer")
 
     def _plan(self, layer, index, which, weights, out):
         """Linear argument blocks are cached per (layer, which, weight
@@ -243,6 +251,7 @@ class _GreedyRunner:
         B, T = self.B, self.T
         if tuple(prompt.shape) != (B, T):
             raise ECF8Error(f"prompt must be [{B}, {T}]")
+        self._raise_refused()
         self.pos.zero_()
         self.step.zero_()
         emb = F.embedding(prompt.to(self.dev).reshape(-1), self.model.model.embed_tokens.weight)
@@ -265,12 +274,14 @@ class _GreedyRunner:
         if not hasattr(self, "_greedy_work"):
             self._greedy_work = HK.greedy_work(self.B, self.dev)
         HK.greedy_emit(logits, self._greedy_work, self.tokens, self.next_tok, self.step, self.pos,
-                       advance)
+                       advance, self.refused)
 
     def _decode_body(self):
         table = self.model.model.embed_tokens.weight
-        if table.dtype == torch.bfloat16 and self.B <= 65535:
-            HK.embed_rows(self.next_tok, table, self.res)
+        # every token that the head can emit lies in the table
+        if (table.dtype == torch.bfloat16 and self.B <= 65535
+                and table.shape[0] >= self.model.lm_head.weight.shape[0]):
+            HK.embed_rows(self.next_tok, table, self.res, self.refused)
         else:
             self.res[: self.B].copy_(F.embedding(self.next_tok, table))
         logits = self._forward(False)
@@ -279,6 +290,7 @@ class _GreedyRunner:
 
     def decode_step(self) -> torch.Tensor:
         """One greedy step, eagerly (hooks and launches from Python)."""
+        self._raise_refused()
         return self._decode_body()
 
     def capture(self):
@@ -286,6 +298,7 @@ class _GreedyRunner:
         first (it initializes every lazily built state, e.g. each hooked
         layer's decode table), then restores the counters."""
         torch.cuda.synchronize(self.dev)
+        self._raise_refused()
         pos, step = self.pos.clone(), self.step.clone()
         s = torch.cuda.Stream(self.dev)
         s.wait_stream(torch.cuda.current_stream(self.dev))
@@ -308,6 +321,7 @@ class _GreedyRunner:
             raise ECF8Error("new_tokens does not fit the cache")
         self.prefill(prompt)
         for _ in range(new_tokens - 1):
+            self._raise_refused()
             if self.graph is not None:
                 self.graph.replay()  # refreshes self.logits in place
             else:
@@ -352,6 +366,8 @@ class Qwen3Runner(_GreedyRunner):
         self.work = K.attention_work(B, Hq, max_len, dev)
         self.next_tok = torch.zeros(B, dtype=torch.int64, device=dev)
         self.tokens = torch.zeros(B, max_len, dtype=torch.int64, device=dev)
+        self.refused = HK.refusal_flag()
+        self._refused_host = self.refused.numpy()
         self.graph = None
         self.logits = None  # logits of the last decode step
         self._plans = {}

@@ -33,6 +33,7 @@ from . import decode as _dev
 from . import llm_kernels as K
 from . import tiled
 from ._lib import ECF8Error
+from .head_kernels import refusal_flag
 from .llm import FP8Linear, RMSNorm, _GreedyRunner, _rotary_tables, weight_layout
 from .synth import QWEN3_MOE_ATTN, QWEN3_MOE_EXPERT
 
@@ -282,6 +283,8 @@ class Qwen3MoeRunner(_GreedyRunner):
                         for layer in layers]
         self.next_tok = torch.zeros(B, dtype=torch.int64, device=dev)
         self.tokens = torch.zeros(B, max_len, dtype=torch.int64, device=dev)
+        self.refused = refusal_flag()
+        self._refused_host = self.refused.numpy()
         self.graph = None
         self.logits = None
         self._plans = {}

@@ -37,10 +37,21 @@ int ecf8_greedy_emit(const void *logits, int64_t ld, int64_t B, int64_t V, void 
                      int64_t work_bytes, int64_t *tokens, int64_t ld_tokens, int64_t *next_token,
                      int64_t *step, int *pos, int advance, void *stream);
 
+/* ecf8_greedy_emit; a step outside the token buffer also sets refused[0]
+ * (memory that the device can write, e.g. pinned host memory). */
+int ecf8_greedy_emit_checked(const void *logits, int64_t ld, int64_t B, int64_t V, void *work,
+                             int64_t work_bytes, int64_t *tokens, int64_t ld_tokens,
+                             int64_t *next_token, int64_t *step, int *pos, int advance,
+                             int *refused, void *stream);
+
 /* out fp32 [B, H] = rows token[b] of table bf16 [V, H] (zeros for a token
  * outside the table); H a multiple of 8. */
 int ecf8_embed_rows(const int64_t *token, int64_t B, const void *table, int64_t V, int64_t H,
                     float *out, void *stream);
+
+/* ecf8_embed_rows; a token outside the table also sets refused[0]. */
+int ecf8_embed_rows_checked(const int64_t *token, int64_t B, const void *table, int64_t V,
+                            int64_t H, float *out, int *refused, void *stream);
 
 #ifdef __cplusplus
 }

@@ -109,3 +109,45 @@ def test_embed_rows_matches_embedding(cuda_device, B, H):
     out = torch.full((B + 1, H), 5.0, device=cuda_device)
     embed_rows(tok, table, out)
     assert torch.equal(out[:B], F.embedding(tok, table).float()) and bool((out[B] == 5.0).all())
+
+
+@pytest.mark.parametrize("graph", [False, True])
+@pytest.mark.parametrize("what", ["token", "negative", "step"])
+def test_decode_step_refuses_bad_state_at_the_next_call(cuda_device, what, graph):
+    """A token outside the vocabulary or a step past the token buffer stays
+    inside the kernels' bounds checks and makes the runner's next call raise;
+    after that the runner works on."""
+    from ecf8_amd._lib import ECF8Error
+    from ecf8_amd.llm import Qwen3Config, Qwen3ForCausalLM, Qwen3Runner
+    from ecf8_amd.synth import quantize_fp8_blockwise
+
+    cfg = Qwen3Config(layers=1, intermediate=4096, vocab=128)
+    model = Qwen3ForCausalLM(cfg).to(cuda_device)
+    for name, (o, i, sigma) in cfg.linear_shapes().items():
+        lin = model.model.layers[0].get_submodule(name)
+        w, s = quantize_fp8_blockwise(sigma * torch.randn(o, i, device=cuda_device))
+        lin.weight, lin.weight_scale_inv = torch.nn.Parameter(w, requires_grad=False), s
+    with torch.no_grad():
+        r = Qwen3Runner(model, 2, 4, 16, cuda_device)
+        prompt = torch.randint(0, 128, (2, 4))
+        r.prefill(prompt)
+        if graph:
+            r.capture()
+        step = r.graph.replay if graph else r.decode_step
+        want = r.generate(prompt, 3).clone()
+        if what == "step":
+            r.step.fill_(r.tokens.shape[1])
+        else:
+            r.next_tok[1] = 128 if what == "token" else -1
+        tokens = r.tokens.clone()
+        step()
+        torch.cuda.synchronize()
+        if what == "step":
+            assert torch.equal(r.tokens, tokens)
+        with pytest.raises(ECF8Error, match="vocabulary"):
+            r.decode_step()
+        for call in (r.capture, lambda: r.prefill(prompt), lambda: r.generate(prompt, 3)):
+            r.refused.fill_(1)  # raising cleared it
+            with pytest.raises(ECF8Error, match="vocabulary"):
+                call()
+        assert torch.equal(r.generate(prompt, 3), want)
