@@ -1863,45 +1863,108 @@ __global__ __launch_bounds__(WAVES * 64) void moe_linear16_kernel(MoeLinear a) {
   }
 }
 
-// The same grouped linear for many rows per expert (a prompt): workgroup
-// (strip, slot) of eight waves computes a 128-column strip of expert
-// active[slot], wave w its columns [16 w, +16), for 16 kChunks rows at a
-// time, so an expert's weights are read once per 64 (or 32) rows instead of
-// once per 16.  The rows' activations go to LDS in MFMA lane order (gathered 16-byte parts),
-// shared by the eight waves and double-buffered; a wave's weight panel goes
-// straight to its registers, one stage of PARTS groups ahead.
+// Block u of the rows that the active experts have past their first kRows, in
+// turn, kRows rows (or the rest of an expert's) each: its expert and its
+// number in it; false past the last.  Each wave finds it by itself, 256
+// experts at a time, four per lane.
+template <int kRows>
+__device__ __forceinline__ bool moe_row_block(const MoeLinear &a, int n_active, int u, int &e,
+                                              int &block) {
+  const int lane = threadIdx.x & 63;
+  for (int page = 0; page < n_active; page += 256) {
+    int ex[4], n[4], sum = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int slot = page + 4 * lane + i;
+      ex[i] = slot < n_active ? a.active[slot] : -1;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int rows = ex[i] < 0 ? 0 : a.offsets[ex[i] + 1] - a.offsets[ex[i]];
+      n[i] = max(rows - 1, 0) / kRows;
+      sum += n[i];
+    }
+    int end = sum;  // inclusive scan over the lanes
+#define ECF8_DPP_SCAN(ctrl, rows) \
+  end += __builtin_amdgcn_update_dpp(0, end, ctrl, rows, 0xF, false)
+    ECF8_DPP_SCAN(0x111, 0xF);  // row_shr:1
+    ECF8_DPP_SCAN(0x112, 0xF);  // row_shr:2
+    ECF8_DPP_SCAN(0x114, 0xF);  // row_shr:4
+    ECF8_DPP_SCAN(0x118, 0xF);  // row_shr:8
+    ECF8_DPP_SCAN(0x142, 0xA);  // row_bcast:15 to rows 1 and 3
+    ECF8_DPP_SCAN(0x143, 0xC);  // row_bcast:31 to rows 2 and 3
+#undef ECF8_DPP_SCAN
+    const uint64_t past = __ballot(u < end);
+    if (past) {
+      int at = u - (end - sum), found = -1;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (found < 0 && at < n[i]) found = ex[i];
+        if (found < 0) at -= n[i];
+      }
+      const int src = __builtin_ctzll(past);
+      e = __builtin_amdgcn_readlane(found, src);
+      block = __builtin_amdgcn_readlane(at, src) + 1;
+      return true;
+    }
+    u -= __builtin_amdgcn_readlane(end, 63);
+  }
+  return false;
+}
+
+// The same grouped linear for many rows per expert (a prompt): a workgroup of
+// eight waves computes a 128-column strip of a block of 16 kChunks rows, wave
+// w its columns [16 w, +16), so an expert's weights are read once per 64 (or
+// 32) rows instead of once per 16.  The rows' activations go to LDS in MFMA
+// lane order (gathered 16-byte parts), shared by the eight waves and
+// double-buffered; a wave's weight panel goes straight to its registers, one
+// stage of PARTS groups ahead.  Workgroups (strip, slot < n_experts) take the
+// active experts' first rows, those after them the blocks past these, one
+// each (moe_row_block), so that the experts that most tokens pick do not hold
+// up a few workgroups.
 //
 // The sums are moe_linear16_kernel's, bit for bit: group kg adds to partial
 // sum kg mod PARTS (that kernel's wave), the partial sums are added in
-// order.  HBM bounds it (weights read once, 403 MB for gate/up and 201 MB for
-// down of 128 experts); MI355X, 512 tokens, tile-layout weights: gate/up 347
-// -> 113 us, down 107 -> 70 us.
+// order.  The latency of a block's loads bounds it, one after the other:
+// routing, scales and rows, then two to four stages of weights (2.9 to 3.6
+// TB/s of weights where a copy reads and writes at 6.2).  MI355X, 128 experts,
+// tile-layout weights, us, gate/up and down, 16-row form against this one:
+// 512 tokens routed evenly 339 / 104 against 113 / 68; all on eight experts
+// 172 / 92 against 62 / 47 (142 / 92 when an expert's workgroups walked all
+// its rows); every token on one expert among others 318 / 104 against 113 /
+// 60 (147 / 105).
 template <int PARTS, int kChunks>
-__global__ __launch_bounds__(512, 8 / kChunks) void moe_rows_kernel(MoeLinear a) {
+__global__ __launch_bounds__(512, 8 / kChunks) void moe_rows_kernel(MoeLinear a, int n_experts) {
   constexpr int kRows = 16 * kChunks, kMaxGroups = 16;
   constexpr int kCopies = 2 * kChunks < 8 ? 8 / (2 * kChunks) : 1;  // waves per 1 KB part
   __shared__ u32x4 s_a[2][PARTS][kChunks][2][64];
   __shared__ __attribute__((aligned(16))) float s_s[kMaxGroups][kRows];
-  const int slot = blockIdx.y;
-  if (slot >= a.n_active[0]) return;  // uniform
-  const int e = a.active[slot];
-  const int r0 = a.offsets[e], rows = a.offsets[e + 1] - r0;
-  const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int r = lane & 15, g = lane >> 4;
   const int seg = (int)(blockIdx.x * 128) / a.seg_n;  // seg_n is a multiple of 128
   const int n0 = (int)(blockIdx.x * 128) - seg * a.seg_n + 16 * wave;
-  const uint8_t *w = reinterpret_cast<const uint8_t *>(a.w[(size_t)e * a.n_segs + seg]);
   const int K = a.K, kgroups = K / kGroup;
-  const float *wsrow =
-      reinterpret_cast<const float *>(a.ws[(size_t)e * a.n_segs + seg]) +
-      (size_t)(n0 / kGroup) * kgroups;
-  const WeightLane wl(w, a.wtiled != 0, n0, r, g, K);
-  const Rsrc wr = wl.rsrc(K);
   const int stages = (kgroups + PARTS - 1) / PARTS;
+  const int n_active = a.n_active[0];
 
-  for (int rc = 0; rc < rows; rc += kRows) {
-    const int mrows = min(kRows, rows - rc);
+  int u = (int)blockIdx.y - n_experts, e, block = 0;
+  if (u < 0) {  // uniform
+    if ((int)blockIdx.y >= n_active) return;
+    e = a.active[blockIdx.y];
+  } else if (!moe_row_block<kRows>(a, n_active, u, e, block)) {
+    return;
+  }
+  do {
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));  // nothing per lane is kept from block to block
+    const int r = lane & 15, g = lane >> 4;
+    const int r0 = a.offsets[e], rc = kRows * block;
+    const int mrows = min(kRows, a.offsets[e + 1] - r0 - rc);
+    const uint8_t *w = reinterpret_cast<const uint8_t *>(a.w[(size_t)e * a.n_segs + seg]);
+    const float *wsrow =
+        reinterpret_cast<const float *>(a.ws[(size_t)e * a.n_segs + seg]) +
+        (size_t)(n0 / kGroup) * kgroups;
+    const WeightLane wl(w, a.wtiled != 0, n0, r, g, K);
+    const Rsrc wr = wl.rsrc(K);
     const int nch = (mrows + 15) >> 4;  // 16-row chunks in use (uniform)
     // scales, [group][row]; rows past the last take its values, unused
     for (int i = threadIdx.x; i < kRows * kgroups; i += 512) {
@@ -1998,8 +2061,10 @@ __global__ __launch_bounds__(512, 8 / kChunks) void moe_rows_kernel(MoeLinear a)
         if (m < mrows)
           a.out[(size_t)(r0 + rc + m) * a.ldo + seg * a.seg_n + n0 + r] = (uint16_t)f32_bf16(sum);
       }
+    if (u < 0) return;
+    u += (int)gridDim.y - n_experts;
     lds_barrier();  // s_s and s_a are refilled for the next rows
-  }
+  } while (moe_row_block<kRows>(a, n_active, u, e, block));
 }
 
 // y[m, :] = sum_k pair_w[q] * down[q, :] over q = pair_pos[m * top_k + k],
@@ -2359,17 +2424,23 @@ extern "C" int ecf8_moe_linear_pairs(const void *aq, const float *as, const int 
   // registers.  MI355X, 128 experts, row-major weights, us for gate/up K =
   // 2048 and down K = 768, 16-row form against this one: 32 tokens (2 rows)
   // 88.2 / 40.8 against 99.4 / 42.9, 48 tokens 103.9 / 46.2 against 102.3 /
-  // 45.7, 64 tokens 112.9 / 48.2 against 103.3 / 46.8, 128 tokens 145.7 /
-  // 53.7 against 105.7 / 48.6, 1024 tokens 798 / 255 against 253 / 151.
+  // 45.7, 64 tokens 114.5 / 49.0 against 103.9 / 49.6, 128 tokens 144.7 /
+  // 53.3 against 106.8 / 51.4, 1024 tokens 787 / 249 against 229 / 144.  64
+  // tokens on eight experts (64 rows each): 26.3 / 16.6 against 23.3 / 16.6,
+  // tile-layout weights 19.0 / 13.1 against 20.1 / 13.5.
   // 32 rows for down keep two workgroups per CU, its loads' latency being
   // most of its two stages (64 rows: 86.0 against 92.4 us at 512 tokens, but
   // 67.5 against 48.6 at 128); the four-part form spills at 128 VGPRs.
   if (pairs >= 4 * (int64_t)n_experts && groups <= ECF8_MOE_FOUR_WAVE_GROUPS) {
-    const dim3 strips((unsigned)(n_segs * seg_n / 128), (unsigned)n_experts);
+    // each expert's first rows, then at most pairs / 64 (32) blocks past them
+    // (a few stand for more, in turns)
+    const int64_t past = pairs / (groups == 6 ? 32 : 64), most = 65536 - n_experts;
+    const dim3 strips((unsigned)(n_segs * seg_n / 128),
+                      (unsigned)(n_experts + (past < 1 ? 1 : past > most ? most : past)));
     if (groups == 6)
-      moe_rows_kernel<3, 2><<<strips, 512, 0, as_stream(stream)>>>(a);
+      moe_rows_kernel<3, 2><<<strips, 512, 0, as_stream(stream)>>>(a, n_experts);
     else
-      moe_rows_kernel<4, 4><<<strips, 512, 0, as_stream(stream)>>>(a);
+      moe_rows_kernel<4, 4><<<strips, 512, 0, as_stream(stream)>>>(a, n_experts);
     return launched();
   }
   const dim3 grid((unsigned)(n_segs * seg_n / 16), (unsigned)n_experts);

@@ -197,8 +197,9 @@ int ecf8_moe_linear(const void *aq, const float *as, const int *row_of, const in
 
 /* ecf8_moe_linear, told the number of (token, expert) pairs in `offsets`:
  * with four rows per expert or more on average it reads an expert's weights
- * once per 64 (or 32) rows instead of once per 16, with the same sums.  pairs only
- * chooses the kernel (0: not known). */
+ * once per 64 (or 32) rows instead of once per 16, with the same sums.  pairs
+ * chooses the kernel and sizes its grid (0: not known); the results do not
+ * depend on it. */
 int ecf8_moe_linear_pairs(const void *aq, const float *as, const int *row_of, const int *offsets,
                           const int *active, const int *n_active, int n_experts,
                           const void *const *weights, const float *const *weight_scales,

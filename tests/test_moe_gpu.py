@@ -143,6 +143,46 @@ def _pair_linear_ref(a_rows, a_s_rows, w, ws):
     return (part * scale).sum(-1)
 
 
+@pytest.mark.parametrize("K", [768, 1024])
+@pytest.mark.parametrize("counts,pairs", [
+    ([2000], 2000), ([0, 513, 0, 1, 448], 962), ([700] + [1] * 127, 827),
+    ([0] * 299 + [1500], 1500), ([200 if e % 37 == 0 else e % 3 for e in range(520)], 2080)])
+def test_grouped_linear_many_rows_of_few_experts(cuda_device, K, counts, pairs):
+    """Rows past an expert's first block are spread over workgroups: one or
+    few experts with most of the rows, more experts than one wave looks
+    through at a time, fewer pairs stated than there are (workgroups take
+    several blocks in turn), and an active list that leaves an expert out:
+    the 16-row form's bits, and nothing elsewhere."""
+    from ecf8_amd._lib import lib
+    from ecf8_amd.llm_kernels import MoeLinearPlan, to_tiles
+
+    E, M, seg_n = len(counts), sum(counts), 128
+    gen = torch.Generator().manual_seed(E + K)
+    weights = [(_rand_fp8((seg_n, K), gen, cuda_device),
+                (torch.rand(1, K // 128, generator=gen) * 0.01).to(cuda_device))
+               for _ in range(5)]
+    out = torch.empty(M, seg_n, dtype=torch.bfloat16, device=cuda_device)
+    plan = MoeLinearPlan([[weights[e % 5]] for e in range(E)], out)
+    aq = to_tiles(_rand_fp8((M, K), gen, cuda_device))
+    a_s = torch.rand(M, K // 128, generator=gen).to(cuda_device)
+    i32 = dict(dtype=torch.int32, device=cuda_device)
+    offsets = torch.tensor([sum(counts[:e]) for e in range(E + 1)], **i32)
+    every = [e for e in range(E) if counts[e]]
+    for listed in (every, every[1:] if len(every) > 1 else every, every[::-1]):
+        active = torch.tensor(listed + [0] * (E - len(listed)), **i32)
+        n_active = torch.tensor([len(listed)], **i32)
+        got = []
+        for stated in (0, pairs, 4 * E):
+            out.fill_(7.0)
+            assert lib().ecf8_moe_linear_pairs(
+                aq.data_ptr(), a_s.data_ptr(), None, offsets.data_ptr(), active.data_ptr(),
+                n_active.data_ptr(), E, plan.w_table.data_ptr(), plan.s_table.data_ptr(), 1, seg_n,
+                K, 0, stated, out.data_ptr(), seg_n, torch.cuda.current_stream().cuda_stream) == 0
+            got.append(out.clone())
+        for g in got[1:]:
+            assert torch.equal(g.view(torch.int16), got[0].view(torch.int16))
+
+
 @pytest.mark.parametrize("K,n_segs,seg_n", [(768, 1, 256), (768, 2, 128), (2048, 2, 128),
                                              (640, 1, 128), (128, 3, 128), (1024, 1, 384)])
 @pytest.mark.parametrize("layout", [0, 1])
