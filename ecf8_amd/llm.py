@@ -227,11 +227,10 @@ class _GreedyRunner:
         """Causal attention of the prompt, positions 0..T-1, in fp32 on the
         bf16 queries and caches."""
         cfg = self.cfg
-        need = (self.B, cfg.kv_heads, T)
-        if getattr(self, "_kv_work", (None,))[0] != need:
-            self._kv_work = (need, K.packed_kv(*need, self.dev))
-        K.prompt_attention(self.q, self.kc[index], self.vc[index], T, self._kv_work[1], self.attn,
-                           cfg.heads)
+        # given back after each layer (to the next one's call): the decode
+        # steps that follow have no use for it
+        work = K.packed_kv(self.B, cfg.kv_heads, T, self.dev)
+        K.prompt_attention(self.q, self.kc[index], self.vc[index], T, work, self.attn, cfg.heads)
 
     def _forward(self, prefill: bool):
         """All layers + final norm + lm_head; returns bf16 logits [B, vocab]

@@ -228,3 +228,22 @@ def test_dit_blocks_agree_with_the_torch_path(cuda_device, monkeypatch, kind, B)
     leaf = args[0].clone().requires_grad_()
     run(leaf, *args[1:])[0].float().sum().backward()
     assert "ecf8_packed_attention" not in calls and bool(torch.isfinite(leaf.grad).all())
+
+
+def test_prompt_attention_leaves_no_workspace(cuda_device):
+    """A prompt's packed keys and values go back to the allocator: nothing
+    of their size stays with the runner."""
+    from types import SimpleNamespace
+
+    from ecf8_amd.llm import _GreedyRunner
+
+    B, T, Hkv, Hq = 2, 512, 8, 32
+    r = _GreedyRunner()
+    r.B, r.dev, r.cfg = B, cuda_device, SimpleNamespace(heads=Hq, kv_heads=Hkv)
+    r.q = torch.randn(B * Hq * T * 128, device=cuda_device).to(torch.bfloat16)
+    r.kc = [torch.randn(B, Hkv, T, 128, device=cuda_device).to(torch.bfloat16)]
+    r.vc = [torch.randn(B, Hkv, T, 128, device=cuda_device).to(torch.bfloat16)]
+    r.attn = torch.empty(B * T, Hq * 128, dtype=torch.bfloat16, device=cuda_device)
+    before = torch.cuda.memory_allocated(cuda_device)
+    r._prefill_attention(0, T)
+    assert torch.cuda.memory_allocated(cuda_device) == before
