@@ -1166,6 +1166,9 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(
 
 // ------------------------------------------------------ decode attention
 
+// Eight bytes at any dword: a v cache may start at any.
+typedef uint32_t u32x2a4 __attribute__((ext_vector_type(2), aligned(4)));
+
 // What the fused form of the split kernel needs besides the caches.
 struct AttnFused {
   const uint16_t *qkv;  // [B, (Hq + 2 Hkv) * 128], one new token per sequence
@@ -1279,7 +1282,7 @@ __global__ __launch_bounds__(64 * kAttnWaves) void attn_split_kernel(
   u32x2 vv[16];
 #pragma unroll
   for (int st = 0; st < 16; ++st)
-    vv[st] = *reinterpret_cast<const u32x2 *>(
+    vv[st] = *reinterpret_cast<const u32x2a4 *>(
         vc + (row0 + min(64 * pg + 4 * st + rr, n - 1)) * kHeadDim + 64 * half + 4 * dg);
 
   if constexpr (kFused) {

@@ -553,6 +553,34 @@ def test_decode_attention_matches_fp32(cuda_device, pos0, G):
 
 
 @pytest.mark.parametrize("G", [4, 8])
+def test_decode_attention_takes_a_v_cache_at_any_dword(cuda_device, G):
+    """The values' cache may start at any multiple of 4 bytes: the same bits
+    as from a 16-byte aligned one."""
+    from ecf8_amd.llm_kernels import attention_work, decode_attention
+
+    B, Hkv, Lmax = 2, 2, 300
+    Hq, dev = G * Hkv, cuda_device
+    gen = torch.Generator(device=dev).manual_seed(G)
+
+    def rand(*shape):
+        return torch.randn(shape, generator=gen, device=dev).to(torch.bfloat16)
+
+    q, kc, vc = rand(B, Hq, 128), rand(B, Hkv, Lmax, 128), rand(B, Hkv, Lmax, 128)
+    pos = torch.tensor([Lmax - 1], dtype=torch.int32, device=dev)
+    work = attention_work(B, Hq, Lmax, dev)
+    oq = torch.empty(pad16(B), Hq * 128, dtype=FP8, device=dev)
+    os_, got = torch.empty(B, Hq, device=dev), []
+    for at in (0, 2, 4, 6):
+        v = torch.empty(vc.numel() + 8, dtype=torch.bfloat16, device=dev)[at:at + vc.numel()]
+        assert v.data_ptr() % 16 == 2 * at
+        v = v.view(vc.shape).copy_(vc)
+        ob = torch.empty(B, Hq * 128, dtype=torch.bfloat16, device=dev)
+        decode_attention(q, kc, v, pos, work, oq, os_, Hq, out_bf16=ob)
+        got.append(ob)
+    assert all(torch.equal(o, got[0]) for o in got)
+
+
+@pytest.mark.parametrize("G", [4, 8])
 @pytest.mark.parametrize("p", [0, 1, 30, 31, 32, 33, 63, 64, 223, 254, 255, 256, 287, 288, 700])
 def test_fused_decode_attention_at_the_edges_of_its_splits(cuda_device, p, G):
     """Positions at the edges of a wave's 64 and a workgroup's 256; the
