@@ -136,6 +136,63 @@ def test_dit_joint_attention_matches_fp64(cuda_device, B, tokens, heads, tail):
             assert float(err) <= 4 * 2.0 ** -9.8, float(err)
 
 
+@pytest.mark.parametrize("heads", [2, 96])  # one and two waves a SIMD
+@pytest.mark.parametrize("along,rises", [
+    ((.1, .1, .45, .45, .45, .45), {2: 8}), ((.1, .1, .1, .1, .1, .5), {5: 8}),
+    ((.1, .1, .29, .29, .29, .29), {2: 5}), ((.05, .2, .35, .55, .75, .95), {1: 3, 2: 3, 3: 5, 5: 5}),
+    ((.1, .5, .1, .1, .9, .1), {1: 8, 4: 8})])
+def test_dit_joint_attention_rescales_where_maxima_rise(cuda_device, heads, along, rises):
+    """Row maxima (base-2 units) that rise by more than the 8 at which sums
+    are rescaled, in a middle block of 64 keys and in the partial last one,
+    by less than that, and step by step; for half of the queries of a wave
+    only (the others point the other way).  The values of the first two
+    blocks are 1000 times as large, so that what the rescale leaves of them
+    counts.  Against fp64 on the same bf16-rounded q and k, relative L2: the
+    probabilities and the output are rounded to bf16, 2^-9.8 rms each."""
+    from ecf8_amd import dit_kernels as DK
+    from ecf8_amd.dit import _Norm
+
+    T, C = 5 * 64 + 17, heads * 128
+    gen = torch.Generator(device=cuda_device).manual_seed(int(100 * sum(along)) + heads)
+
+    def rand(*shape):
+        return torch.randn(shape, generator=gen, device=cuda_device)
+
+    u = rand(heads, 128)
+    u = u / u.norm(dim=-1, keepdim=True) * math.sqrt(128)
+    sign = torch.where(torch.arange(T, device=cuda_device) % 3 == 1, -1.0, 1.0)[:, None, None]
+    a = torch.tensor(along, device=cuda_device).repeat_interleave(64)[:T, None, None]
+    q = sign * u + 0.02 * rand(T, heads, 128)
+    across = rand(T, heads, 128)
+    across = across - (across * u).sum(-1, keepdim=True) / 128 * u
+    across = across / across.norm(dim=-1, keepdim=True) * math.sqrt(128)
+    k = a * u + (1 - a * a).sqrt() * across
+    v = rand(T, heads, 128)
+    v[:128] *= 1000
+    y = torch.stack([q, k, v], 1).to(torch.bfloat16).reshape(1, T, 3 * C)
+    norms = [_Norm(128).to(cuda_device).requires_grad_(False) for _ in range(2)]
+    for m in norms:
+        m.weight.data.fill_(1.5)
+    cos = torch.ones(1, 1, T, 64, device=cuda_device)
+    got = DK.joint_attention([(y, *norms)], heads, cos, torch.zeros_like(cos))
+
+    q, k, v = y[0].double().unflatten(1, (3, heads, 128)).permute(1, 2, 0, 3)
+
+    def norm(x, scale):
+        x = x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + 1e-6) * 1.5
+        return (x * scale).float().to(torch.bfloat16).double()
+
+    s = norm(q, DK.Q_SCALE) @ norm(k, 1.0).transpose(-1, -2).contiguous()
+    tops = torch.stack([b.amax(-1) for b in s.split(64, -1)], -1)[:, sign[:, 0, 0] > 0]
+    for b, least in rises.items():
+        rise = tops[..., b] - tops[..., :b].amax(-1)
+        assert float(rise.min()) > least and (least >= 8 or float(rise.max()) < 8)
+    want = (torch.softmax(s * math.log(2), -1) @ v).transpose(0, 1).reshape(T, C)
+    for rows in (sign[:, 0, 0] > 0, sign[:, 0, 0] < 0):
+        err = (got[0][rows].double() - want[rows]).norm() / want[rows].norm()
+        assert float(err) <= 3 * 2.0 ** -9.8, float(err)
+
+
 def test_dit_joint_attention_leaves_odd_layouts(cuda_device):
     """An expanded norm weight and a tail with overlapping rows run in torch."""
     from ecf8_amd import dit_kernels as DK
