@@ -32,6 +32,16 @@ __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, v);
 }
 
+// Eight bf16 with their infinities and NaNs replaced by zeros.
+__device__ __forceinline__ u32x4 finite_or_zero(u32x4 v) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    if ((v[j] & 0x7f80u) == 0x7f80u) v[j] &= 0xffff0000u;
+    if ((v[j] & 0x7f800000u) == 0x7f800000u) v[j] &= 0xffffu;
+  }
+  return v;
+}
+
 // Workgroup barrier that waits for LDS only (a __syncthreads would also
 // wait for the prefetched global loads).
 __device__ __forceinline__ void lds_barrier() {
@@ -93,7 +103,8 @@ struct Attn {
 //
 // kExact (the prompt): a probability enters the second product as the sum
 // of three bf16 parts, which hold its 24 mantissa bits, so that product is
-// that of the fp32 probabilities.  Otherwise probabilities are rounded to
+// that of the fp32 probabilities (an infinite value times a probability
+// above zero is infinite, as there).  Otherwise probabilities are rounded to
 // bf16, as the DiT's softmax does.
 //
 // Bound by the MFMA pipe and the exponentials (16 of each per 32 x 32 tile
@@ -147,20 +158,10 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(Attn a) {
     for (int i = 0; i < 16; ++i) o[d][i] = 0.f;
   float m = -INFINITY, l = 0.f;  // of query r: both lanes hold the same m
 
-  load(0, kr, vr);
-  for (int b = 0; b < blocks; ++b) {
-    const int buf = b & 1;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      s_k[buf][256 * i + threadIdx.x] = kr[i];
-      s_v[buf][256 * i + threadIdx.x] = vr[i];
-    }
-    // this block is in LDS; the other buffer was last read in block b - 1,
-    // before every wave's arrival here
-    lds_barrier();
-    if (b + 1 < blocks) load(b + 1, kr, vr);
+  // one block's keys and values, in LDS or packed in memory
+  auto step = [&](int b, const u32x4 *k, const u32x4 *v, auto careful) {
     const int key0 = b * kBlock;
-    if (q0 >= a.T || (kCausal && key0 > q0 + 31)) continue;  // uniform per wave
+    if (q0 >= a.T || (kCausal && key0 > q0 + 31)) return;  // uniform per wave
 
     v16f s[2];
 #pragma unroll
@@ -169,7 +170,7 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(Attn a) {
       for (int i = 0; i < 16; ++i) s[t][i] = 0.f;
 #pragma unroll
       for (int kk = 0; kk < 8; ++kk) {
-        const v8bf kf = *reinterpret_cast<const v8bf *>(&s_k[buf][t * 512 + kk * 64 + lane]);
+        const v8bf kf = *reinterpret_cast<const v8bf *>(&k[t * 512 + kk * 64 + lane]);
         s[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[kk], s[t], 0, 0, 0);
       }
     }
@@ -190,7 +191,8 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(Attn a) {
                                                      false, false);
     const float mn = fmaxf(m, fmaxf(__uint_as_float(hm[0]), __uint_as_float(hm[1])));
     if (__any(mn > m)) {  // uniform: some query's maximum moved
-      const float f = __builtin_amdgcn_exp2f((m - mn) * a.scale);
+      float f = __builtin_amdgcn_exp2f((m - mn) * a.scale);
+      if (careful && m == mn) f = 1.f;  // both may be -inf
       l *= f;
 #pragma unroll
       for (int d = 0; d < 4; ++d)
@@ -198,11 +200,12 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(Attn a) {
         for (int i = 0; i < 16; ++i) o[d][i] *= f;
       m = mn;
     }
+    const float top = careful && m == -INFINITY ? 0.f : m;
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        s[t][i] = __builtin_amdgcn_exp2f((s[t][i] - m) * a.scale);
+        s[t][i] = __builtin_amdgcn_exp2f((s[t][i] - top) * a.scale);
         l += s[t][i];
       }
 #pragma unroll
@@ -224,12 +227,48 @@ __global__ __launch_bounds__(256, 2) void flash_kernel(Attn a) {
       }
 #pragma unroll
       for (int d = 0; d < 4; ++d) {
-        const v8bf vf = *reinterpret_cast<const v8bf *>(&s_v[buf][g * 256 + d * 64 + lane]);
+        const u32x4 vf = v[g * 256 + d * 64 + lane];
+        const u32x4 vs = careful ? finite_or_zero(vf) : vf;
 #pragma unroll
         for (int q = kParts - 1; q >= 0; --q)  // small parts first
-          o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, __builtin_bit_cast(v8bf, pf[q]), o[d],
-                                                         0, 0, 0);
+          o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              __builtin_bit_cast(v8bf, q ? vs : vf), __builtin_bit_cast(v8bf, pf[q]), o[d], 0, 0,
+              0);
       }
+    }
+  };
+
+  load(0, kr, vr);
+  for (int b = 0; b < blocks; ++b) {
+    const int buf = b & 1;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      s_k[buf][256 * i + threadIdx.x] = kr[i];
+      s_v[buf][256 * i + threadIdx.x] = vr[i];
+    }
+    // this block is in LDS; the other buffer was last read in block b - 1,
+    // before every wave's arrival here
+    lds_barrier();
+    if (b + 1 < blocks) load(b + 1, kr, vr);
+    step(b, s_k[buf], s_v[buf], std::false_type());
+  }
+  if constexpr (kExact) {
+    // The smaller parts of a probability, zero or below zero, make NaN of an
+    // infinite value, and a block whose scores are all -inf makes NaN of the
+    // sums.  Then once more, each wave by itself.
+    bool nan = l != l;
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) nan |= o[d][i] != o[d][i];
+    if (__any(nan)) {  // uniform
+#pragma unroll
+      for (int d = 0; d < 4; ++d)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[d][i] = 0.f;
+      m = -INFINITY, l = 0.f;
+      for (int b = 0; b < blocks; ++b)
+        step(b, kp + (size_t)b * (kBlock * 16), vp + (size_t)b * (kBlock * 16), std::true_type());
     }
   }
   l += __shfl_xor(l, 32);

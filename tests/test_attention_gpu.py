@@ -53,6 +53,47 @@ def test_prompt_attention_matches_fp64(cuda_device, B, T, Hq, Hkv, Lmax):
     assert bool((out[B * T:] == 3.0).all())
 
 
+@pytest.mark.parametrize("T,Hq,Hkv", [(70, 4, 1), (130, 4, 2), (300, 8, 2)])
+def test_prompt_attention_of_infinite_values_and_scores(cuda_device, T, Hq, Hkv):
+    """As in fp32: an infinite value makes its dim infinite for the queries
+    that attend to it (NaN where both infinities meet), a NaN NaN, and leaves
+    the other dims alone; keys whose scores are -inf drop out, also a whole
+    block of 64 of them."""
+    from ecf8_amd.llm_kernels import packed_kv, prompt_attention
+
+    gen = torch.Generator(device=cuda_device).manual_seed(T)
+
+    def rand(*shape):
+        return torch.randn(shape, generator=gen, device=cuda_device).to(torch.bfloat16)
+
+    q, kc, vc = rand(1, Hq, T, 128), rand(1, Hkv, T, 128), rand(1, Hkv, T, 128)
+    work = packed_kv(1, Hkv, T, cuda_device)
+    out = torch.empty(T, Hq * 128, dtype=torch.bfloat16, device=cuda_device)
+
+    def check(rows, v, skip=()):
+        prompt_attention(q, kc, v, T, work, out, Hq)
+        got = out.double().view(T, Hq, 128).transpose(0, 1)[None, :, rows]
+        want = _causal64(q, kc, v.nan_to_num(0, 0, 0))[:, :, rows]
+        dims = [d for d in range(128) if d not in skip]
+        bound = want.abs() * 2.0 ** -8 * 1.01 + float(v.nan_to_num(0, 0, 0).abs().max()) * 2.0 ** -16
+        assert bool(((got - want).abs() <= bound)[..., dims].all())
+        return got
+
+    v = vc.clone()
+    inf = math.inf
+    v[..., 5, 3], v[..., 66, 40], v[..., 7, 100], v[..., 9, 77] = inf, -inf, inf, math.nan
+    v[..., 68, 100] = -inf
+    got = check(slice(68, T), v, (3, 40, 77, 100))
+    assert bool((got[..., 3] == inf).all()) and bool((got[..., 40] == -inf).all())
+    assert bool(got[..., 77].isnan().all()) and bool(got[..., 100].isnan().all())
+    q[..., 0] = q[..., 0].abs() + 0.1
+    kc[..., :64, 0] = -inf
+    check(slice(64, T), vc)
+    kc[..., 64:, :] = rand(1, Hkv, T - 64, 128)
+    kc[..., 10, 0] = 0.5  # one key of the block remains
+    check(slice(10, T), vc)
+
+
 def test_prompt_attention_refuses_what_does_not_fit(cuda_device):
     from ecf8_amd._lib import ECF8Error
     from ecf8_amd.llm_kernels import packed_kv, prompt_attention
