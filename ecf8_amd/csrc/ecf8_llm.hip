@@ -1122,8 +1122,9 @@ __device__ __forceinline__ uint32_t norm_rope(uint32_t x2, const RopeIn &in, flo
 // embedding at position pos[0] + t (rotate-half convention, cos/sin tables
 // [Lmax, 64]); q goes to q_out [B, Hq, T, 128], k and v to the caches
 // [B, Hkv, Lmax, 128].  Workgroup (token, 16 heads), four heads per wave, all
-// loaded at once and sharing the token's rotary values.  HBM bounds it
-// (50 MB at 2048 tokens of 48 heads: 15.8 us; one head per wave 29.5).
+// loaded at once and sharing the token's rotary values.  Loads in
+// flight bound it: 50 MB at 2048 tokens of 48 heads in 15.8 us, 3.2 TB/s
+// where a copy moves 6.2 (one head per wave 29.5 us).
 constexpr int kRopePer = 4;
 __global__ __launch_bounds__(256) void qk_norm_rope_kernel(
     const uint16_t *__restrict__ qkv, int T, int Hq, int Hkv, const uint16_t *__restrict__ qn,
