@@ -161,7 +161,7 @@ def encode_exponents_for_cuda(exponents_4bits, codec, bytes_per_thread: int = 8,
         exps = np.ascontiguousarray(exponents_4bits, dtype=np.uint8)
     bits, vals, eof_bits, eof_val = _code_arrays(codec)
     L = lib()
-    n, threads = exps.size, host_threads()
+    n, threads = exps.size, host_threads(exps.size)
     nb, ng, no = ctypes.c_int64(), ctypes.c_int64(), ctypes.c_int64()
     vp = lambda a: a.ctypes.data_as(ctypes.c_void_p)  # noqa: E731
     check(L.ecf8_encoded_sizes_threads(vp(exps), n, vp(bits), bytes_per_thread, threads_per_block,
@@ -178,9 +178,17 @@ def encode_exponents_for_cuda(exponents_4bits, codec, bytes_per_thread: int = 8,
             torch.from_numpy(op))
 
 
-def host_threads() -> int:
-    """Threads of the host codec: torch's own count, at most 16."""
-    return max(1, min(torch.get_num_threads(), 16))
+def host_threads(n: int) -> int:
+    """Threads of the host codec for n weights: one below 2.6 million, above
+    that torch's own count, at most 16 and 262,144 weights or more each.
+
+    Torch's threads wait for work in a loop for some milliseconds after an
+    operation of theirs, and a new thread beside them waits for its turn on a
+    core.  On 16 cores, a block compressed and then copied by torch, over and
+    over: 1 M weights 4.1 ms on one thread, 3.0 to 7.8 on two to 16 (1.2 in a
+    process without such operations); 2 M 7.8 and 5.8 to 8.8; 4 M 15.4 and
+    7.9; 16 M 63 and 12.8."""
+    return max(1, min(torch.get_num_threads(), 16, n >> 18)) if n >= 5 << 19 else 1
 
 
 def split_fp8_counted(data: torch.Tensor):
@@ -198,7 +206,7 @@ def split_fp8_counted(data: torch.Tensor):
         packed = torch.empty(n // 2, dtype=torch.uint8, device="cpu")
         counts = torch.empty(16, dtype=torch.int64, device="cpu")
         check(lib().ecf8_split_fp8(data.data_ptr(), n, exps.data_ptr(), packed.data_ptr(),
-                                   counts.data_ptr(), host_threads()), "ecf8_split_fp8")
+                                   counts.data_ptr(), host_threads(n)), "ecf8_split_fp8")
         return exps, packed, counts
     exps, packed = get_exponents_and_other_4bits_fp8_e4m3(data)
     return exps, packed, torch.bincount(exps.reshape(-1), minlength=16)

@@ -282,3 +282,31 @@ def test_host_compression_under_another_default_device(n):
         got = compress_flat(w)
     for key in ("luts", "encoded", "packed_other_4bits", "output_positions", "gaps"):
         assert got[key].device.type == "cpu" and torch.equal(got[key], want[key]), key
+
+
+@pytest.mark.parametrize("threads", [1, 2, 3, 16, 200])
+def test_split_on_any_number_of_threads(threads):
+    """Parts that divide the block evenly and not: the one-thread outputs."""
+    from ecf8_amd._lib import lib
+
+    for n in (2, 262142, 262146, 400002):
+        w = torch.from_numpy(np.random.default_rng(n).integers(0, 256, n, dtype=np.uint8))
+        got = []
+        for t in (1, threads):
+            out = (torch.full((n,), 99, dtype=torch.uint8), torch.zeros(n // 2, dtype=torch.uint8),
+                   torch.full((16,), -1, dtype=torch.int64))
+            assert lib().ecf8_split_fp8(w.data_ptr(), n, *(o.data_ptr() for o in out), t) == 0
+            got.append(out)
+        assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
+def test_small_blocks_compress_on_one_thread(monkeypatch):
+    """Few weights on one thread, whatever torch has; many on torch's count,
+    at most 16."""
+    from dfloat import utils
+
+    monkeypatch.setattr(torch, "get_num_threads", lambda: 64)
+    got = [utils.host_threads(n) for n in (0, 2, 1 << 20, (5 << 19) - 1, 5 << 19, 1 << 24)]
+    assert got == [1, 1, 1, 1, 10, 16]
+    monkeypatch.setattr(torch, "get_num_threads", lambda: 3)
+    assert utils.host_threads(1 << 24) == 3
