@@ -86,8 +86,8 @@ def cpu_baseline(block, n_elements, alg_bytes, repeats=3):
 
 def cpu_encode(flat, seed: int = 0):
     """CPU encode timings (the reference's CPU path is its encoder,
-    dfloat/utils.py:373-499): the product's C++ encoder (ecf8_encode_exponents,
-    one thread) over the whole layer, and the oracle's per-symbol Python
+    dfloat/utils.py:373-499): the product's C++ encoder
+    (ecf8_encode_exponents_threads) over the whole layer, and the oracle's per-symbol Python
     restatement of the reference loop over the 4096x4096 tensor the
     reference's CPU case names (seeded N(0, 0.02), 128x128 block scales),
     whose output the C decoder then checks against the original bytes."""
@@ -95,6 +95,7 @@ def cpu_encode(flat, seed: int = 0):
     import torch
 
     from dfloat.compress import compress_flat
+    from dfloat.utils import host_threads
     from ecf8_amd.synth import synthetic_fp8
     from oracle import codec as oc
     from oracle import native
@@ -112,10 +113,9 @@ def cpu_encode(flat, seed: int = 0):
                                             "output_positions", "gaps")))
     return {
         "product_cpp": {"value": round(n / full / 1e6, 2), "unit": "M elements/s",
-                        "cores": torch.get_num_threads(),
-                        "sample": f"whole layer ({n} elements): split and counts (torch, "
-                                  f"{torch.get_num_threads()} threads), codebook, LUTs, bitstream "
-                                  f"(C++ encoder, 1 thread), {full:.2f} s"},
+                        "cores": host_threads(n),
+                        "sample": f"whole layer ({n} elements): split, counts and bitstream (C++, "
+                                  f"{host_threads(n)} threads), codebook, LUTs, {full:.2f} s"},
         "reference_loop_python": {"value": round(part.size / py / 1e6, 4), "unit": "M elements/s",
                                   "cores": 1, "kind": "port",
                                   "sample": f"4096x4096 seeded N(0, 0.02) tensor ({part.size} "
