@@ -62,6 +62,9 @@ typedef struct ecf8_linear_seg {
  * for each of n_segs (1..3) segments, e.g. q/k/v or gate/up in one launch.
  * aq: e4m3fn [M, K] in the tile layout (16-byte aligned, ceil(M/16) * 16
  * rows), as: fp32 [M, K/128].  K and every seg.n must be multiples of 128.
+ * Above 16 rows the groups are added in order whatever M is: a row's bits do
+ * not depend on how many rows share the call.  (Up to 16 rows, waves add
+ * parts of K.)
  */
 int ecf8_fp8_linear(const void *aq, const float *as, int64_t M, int64_t K,
                     const ecf8_linear_seg *segs, int n_segs, void *out, int64_t ldo,
