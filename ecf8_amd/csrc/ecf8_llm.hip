@@ -603,18 +603,21 @@ __global__ __launch_bounds__(512) void fp8_gemm_kernel(
 // of operands at P = 4 (L2) and the products' way through LDS.  MI355X, tile
 // layout, us, against the tile GEMM, and against waves that each add a run
 // of K (another order, that differs with the row count): 64 rows, N = K =
-// 4096 7.8 / 32.5 / 8.3, N = 4096, K = 12288 23.8 / 89.8 / 26.6; 256 rows
-// 13.2 / 33.1 / 12.9 and 41.4 / 111 / 33.2; 512 rows 25.2 / 33.5 / 23.9 and
-// 73 / 106 / 58.
-template <int P, int kCh, int kSub>
+// 4096 7.6 / 32.5 / 8.4, N = 4096, K = 12288 23.6 / 89.8 / 26.7; 256 rows
+// 12.4 / 33.1 / 12.8 and 38.6 / 111 / 33.0; 512 rows 23.6 / 33.5 / 23.8 and
+// 67 / 106 / 58.  16 tiles fill one LDS buffer, with two barriers a round and
+// two tiles a wave; eight at a time in two buffers took 1.05 to 1.09 times as
+// long.
+template <int P, int kCh>
 __global__ __launch_bounds__(512) void fp8_rows_kernel(const uint8_t *__restrict__ aq,
                                                        const float *__restrict__ as, int M, int K,
                                                        LinearSegs segs, uint16_t *__restrict__ out,
                                                        int ldo) {
-  constexpr int kWaves = 8, kTurns = P / kSub, kTiles = kSub * kCh;  // tiles a turn
-  static_assert(P % kSub == 0 && kTiles <= kWaves, "a wave adds one tile a turn");
-  // products of a turn (kSub panels of eight groups), double-buffered
-  __shared__ v4f s_d[2][kWaves][kTiles][64];
+  constexpr int kWaves = 8, kTiles = P * kCh;  // 16 x 16 tiles
+  constexpr int kPer = (kTiles + kWaves - 1) / kWaves, kBufs = kPer > 1 ? 1 : 2;
+  static_assert(kTiles <= kWaves || kTiles % kWaves == 0, "tiles deal evenly");
+  // products of a round of eight groups
+  __shared__ v4f s_d[kBufs][kWaves][kTiles][64];
   __shared__ float s_sc[2][kWaves][64];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -669,47 +672,48 @@ __global__ __launch_bounds__(512) void fp8_rows_kernel(const uint8_t *__restrict
     s.sa = asr[k];
     s.sw = wsrow[k];
   };
-  // wave's tile of turn t: panel t kSub + wave / kCh, rows 16 (wave % kCh)..;
+  // wave's tiles: wave + 8 h, tile i being panel i / kCh, rows 16 (i % kCh)..;
   // lane: columns 4 g .. + 3, row r
-  v4f acc[kTurns];
+  v4f acc[kPer];
 #pragma unroll
-  for (int t = 0; t < kTurns; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
+  for (int h = 0; h < kPer; ++h) acc[h] = v4f{0.f, 0.f, 0.f, 0.f};
   auto step = [&](Stage &s, int rd) {
     const int n = min(kWaves, kgroups - kWaves * rd);  // groups of this round
-    if (wave < n) s_sc[rd & 1][wave][lane] = s.sa * s.sw;
+    const int buf = rd & (kBufs - 1);
+    if (wave < n) {  // uniform
+      s_sc[rd & 1][wave][lane] = s.sa * s.sw;
 #pragma unroll
-    for (int t = 0; t < kTurns; ++t) {
-      const int buf = (rd * kTurns + t) & 1;
-      if (wave < n) {  // uniform
+      for (int p = 0; p < P; ++p)
 #pragma unroll
-        for (int p = 0; p < kSub; ++p)
-#pragma unroll
-          for (int c = 0; c < kCh; ++c) {
-            const v4f z = {0.f, 0.f, 0.f, 0.f};
-            s_d[buf][wave][p * kCh + c][lane] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
-                join32(s.wv[t * kSub + p][0], s.wv[t * kSub + p][1]),
-                join32(s.av[c][0], s.av[c][1]), z, 0, 0, 0, 0, 0, 0);
-          }
-      }
-      if (t == kTurns - 1 && rd + 2 < rounds) load(rd + 2, s);
-      // the products are in LDS; the other buffer (of the scales too) was
-      // last read before every wave's arrival here
-      lds_barrier();
-      if (wave < kTiles) {  // uniform
-        const float *sc = &s_sc[rd & 1][0][16 * (wave % kCh) + r];
-        auto add = [&](int v) {
-          const v4f d = s_d[buf][v][wave][lane];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) acc[t][i] = fmaf(d[i], sc[64 * v], acc[t][i]);
-        };
-        if (n == kWaves) {  // all reads in flight at once
-#pragma unroll
-          for (int v = 0; v < kWaves; ++v) add(v);
-        } else {
-          for (int v = 0; v < n; ++v) add(v);
+        for (int c = 0; c < kCh; ++c) {
+          const v4f z = {0.f, 0.f, 0.f, 0.f};
+          s_d[buf][wave][p * kCh + c][lane] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+              join32(s.wv[p][0], s.wv[p][1]), join32(s.av[c][0], s.av[c][1]), z, 0, 0, 0, 0, 0, 0);
         }
+    }
+    if (rd + 2 < rounds) load(rd + 2, s);
+    // the products are in LDS; with two buffers the other one (and that of
+    // the scales) was last read before every wave's arrival here
+    lds_barrier();
+    if (wave < kTiles) {  // uniform
+      const float *sc = &s_sc[rd & 1][0][16 * (wave % kCh) + r];
+      auto add = [&](int v) {
+        const float f = sc[64 * v];
+#pragma unroll
+        for (int h = 0; h < kPer; ++h) {
+          const v4f d = s_d[buf][v][wave + kWaves * h][lane];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[h][i] = fmaf(d[i], f, acc[h][i]);
+        }
+      };
+      if (n == kWaves) {  // all reads in flight at once
+#pragma unroll
+        for (int v = 0; v < kWaves; ++v) add(v);
+      } else {
+        for (int v = 0; v < n; ++v) add(v);
       }
     }
+    if (kBufs == 1) lds_barrier();
   };
   Stage s0, s1;
   load(0, s0);
@@ -719,14 +723,14 @@ __global__ __launch_bounds__(512) void fp8_rows_kernel(const uint8_t *__restrict
     if (rd + 1 < rounds) step(s1, rd + 1);  // uniform
   }
   if (wave >= kTiles) return;
-  const int m = m0 + 16 * (wave % kCh) + r;
+  const int m = m0 + 16 * (wave % kCh) + r;  // 8 is a multiple of kCh
   if (m >= M) return;
   const bool whole =
       (((uintptr_t)out | 2u * (uintptr_t)(uint32_t)ldo | 2u * (uintptr_t)(uint32_t)col) & 7) == 0;
 #pragma unroll
-  for (int t = 0; t < kTurns; ++t) {
-    uint16_t *o = out + (size_t)m * ldo + col + n0 + 16 * (t * kSub + wave / kCh) + 4 * g;
-    const u32x2 v = {pack_bf16(acc[t][0], acc[t][1]), pack_bf16(acc[t][2], acc[t][3])};
+  for (int h = 0; h < kPer; ++h) {
+    uint16_t *o = out + (size_t)m * ldo + col + n0 + 16 * ((wave + kWaves * h) / kCh) + 4 * g;
+    const u32x2 v = {pack_bf16(acc[h][0], acc[h][1]), pack_bf16(acc[h][2], acc[h][3])};
     if (whole) {
       *reinterpret_cast<u32x2 *>(o) = v;
     } else {
@@ -2168,35 +2172,35 @@ extern "C" int ecf8_fp8_linear(const void *aq, const float *as, int64_t M, int64
     // M fills the 256-row tiles, the tile GEMM then has a workgroup on a
     // quarter of the CUs at most; for few rows it can have one on each, and
     // the line rests on the times alone.  MI355X, us, middle form against
-    // tile GEMM (weight copies rotated): N = K = 4096: M = 64 7.8 / 32.5, M =
-    // 256 13.2 / 33.1, M = 512 (512 blocks) 25.2 / 33.5, M = 768 36.6 / 33.8;
-    // N = 24576: M = 64 (384 blocks) 34.3 / 39.1, M = 128 (768) 51.7 / 40.1;
-    // N = 32768, M = 64 (512) 40.8 / 44.6; K = 512, M = 512, N = 4096 7.3 /
-    // 8.5 (one K group: 6.5 / 5.5).
+    // tile GEMM (weight copies rotated): N = K = 4096: M = 64 7.6 / 32.5, M =
+    // 256 12.4 / 33.1, M = 512 (512 blocks) 23.6 / 33.5, M = 768 about 35 /
+    // 33.8; N = 24576: M = 64 (384 blocks) 34.5 / 39.1, M = 128 (768) about
+    // 50 / 40.1; N = 32768, M = 64 (512) 38.8 / 44.6; K = 512, M = 512, N =
+    // 4096 6.9 / 8.5 (one K group: 6.1 / 5.5).
     const int64_t blocks = (M + 63) / 64 * (n_total / 64);
     if (blocks <= 2 * (int64_t)cus) {
       // The narrowest strips that need no second round of workgroups; for a
       // single block of rows, where the weights come from HBM once, three
       // workgroups per CU in turn (N = 24576, M = 64: two panels 34.3, four
-      // 37.1 us; N = 28672: 43.8 and 38.0; N = 6144, M = 64: one 11.7, two
-      // 9.7, four 13.5).  32 rows a block where that covers M: M = 32, N =
-      // 4096 5.8 us.
+      // 36 us; N = 28672: 43.8 and 36.6; N = 6144, M = 64: one 11.7, two 9.7,
+      // four 12.9).  32 rows a block where that covers M: M = 32, N = 4096
+      // 5.8 us.
       const bool narrow = M <= 32;
       const int64_t row_blocks = narrow ? 1 : (M + 63) / 64;
       const int64_t one = row_blocks * (n_total / 16);
       const int panels = one <= cus ? 1 : one / 2 <= (row_blocks == 1 ? 3 : 1) * cus ? 2 : 4;
       const dim3 grid((unsigned)(n_total / (16 * panels)), (unsigned)row_blocks);
-#define ECF8_ROWS(P, CH, SUB)                                                                    \
-  fp8_rows_kernel<P, CH, SUB><<<grid, 512, 0, as_stream(stream)>>>(a, as, (int)M, (int)K, s, o, \
-                                                                   (int)ldo)
+#define ECF8_ROWS(P, CH)                                                                    \
+  fp8_rows_kernel<P, CH><<<grid, 512, 0, as_stream(stream)>>>(a, as, (int)M, (int)K, s, o, \
+                                                              (int)ldo)
       if (narrow) {
-        if (panels == 1) ECF8_ROWS(1, 2, 1);
-        else if (panels == 2) ECF8_ROWS(2, 2, 2);
-        else ECF8_ROWS(4, 2, 4);
+        if (panels == 1) ECF8_ROWS(1, 2);
+        else if (panels == 2) ECF8_ROWS(2, 2);
+        else ECF8_ROWS(4, 2);
       } else {
-        if (panels == 1) ECF8_ROWS(1, 4, 1);
-        else if (panels == 2) ECF8_ROWS(2, 4, 2);
-        else ECF8_ROWS(4, 4, 2);
+        if (panels == 1) ECF8_ROWS(1, 4);
+        else if (panels == 2) ECF8_ROWS(2, 4);
+        else ECF8_ROWS(4, 4);
       }
 #undef ECF8_ROWS
       return launched();
